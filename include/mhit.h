@@ -233,15 +233,16 @@ int mhit_set_tuning(mhit_ctx *ctx, const mhit_tuning *in);
  * drops in raster order of their first cell (x fastest, then y, then z);
  * volume[q] in cells, deq[q] = dx (6 volume/pi)^(1/3).  *n_drops is the total
  * count; the first max_drops entries are filled.  Needs phiflag = 1.  The
- * context's first call allocates a labelling workspace (4 N^3 bytes of labels
- * plus 12 bytes per possible drop, N^3/8 + 1 of them, at most 2^24) that the
- * context keeps until mhit_destroy; later calls allocate nothing. */
+ * context's first call allocates a labelling workspace (4 N^3 bytes of labels,
+ * one bit per cell and 12 bytes per possible drop, N^3/8 + 1 of them, at most
+ * 2^24) that the context keeps until mhit_destroy; later calls allocate
+ * nothing. */
 int mhit_drop_count(mhit_ctx *ctx, int max_drops, int *n_drops, double *volume, double *deq);
 
 /* mhit_drop_count without any device allocation: no counterpart in the
  * reference.  For callers that cannot allocate (code under HIP graph capture,
  * serving loops, harnesses that forbid hipMalloc).  The labelling workspace is
- * a static device array of MHIT_NOALLOC_MAX_N^3-cell size (11.6 MB), one per
+ * a static device array of MHIT_NOALLOC_MAX_N^3-cell size (11.8 MB), one per
  * GPU, held until the process ends; boxes with N > MHIT_NOALLOC_MAX_N get
  * MHIT_ERR_BAD_N.  Same arguments and results as mhit_drop_count.  Every call
  * on one GPU uses that GPU's array: calls that overlap on one GPU (from

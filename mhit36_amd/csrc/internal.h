@@ -193,10 +193,10 @@ void launch_debug_math(int op, size_t count, const double *x, double *y, const d
 // smallest linear index of their set; list the roots; count cells per root
 // (roots sorted ascending).
 // The workspace: labels (n^3), the sorted root list and its volumes (cap
-// each), per-chunk counts and offsets, the root count.
+// each), the bitmask of the cells, per-chunk counts, the root count.
 struct CclWork {
-    unsigned *lab, *roots, *counts, *offs, *nroots;
-    unsigned long long *vol;
+    unsigned *lab, *roots, *counts, *nroots;
+    unsigned long long *vol, *mask;
     unsigned cap;
 };
 // Most drops a box of n3 cells can hold: components need an empty cell between
@@ -205,24 +205,25 @@ constexpr size_t ccl_cap(size_t n3)
 {
     return n3 / 8 + 1 < ((size_t)1 << 24) ? n3 / 8 + 1 : ((size_t)1 << 24);
 }
-// The root list is built over CCL_CHUNKS contiguous chunks of cells.
+// The bitmask: rows of ceil(n/64) words.
+constexpr size_t ccl_words(int n) { return (size_t)((n + 63) / 64) * n * n; }
+// The root list is built over at most CCL_CHUNKS contiguous chunks of mask words.
 constexpr int CCL_CHUNKS = 4096;
 constexpr size_t ccl_up(size_t b) { return (b + 255) / 256 * 256; }
 constexpr size_t ccl_workspace_bytes(int n)
 {
     return ccl_up((size_t)n * n * n * 4) + ccl_up(ccl_cap((size_t)n * n * n) * 4) +
-           ccl_up(ccl_cap((size_t)n * n * n) * 8) + 2 * ccl_up(CCL_CHUNKS * 4) + 256;
+           ccl_up(ccl_cap((size_t)n * n * n) * 8) + ccl_up(ccl_words(n) * 8) + ccl_up(CCL_CHUNKS * 4) + 256;
 }
 CclWork ccl_carve(void *base, int n);
 // The allocation-free drop count works in a static device array sized for
-// boxes up to NOALLOC_MAX_N^3 cells (11.6 MB per GPU).
+// boxes up to NOALLOC_MAX_N^3 cells (11.8 MB per GPU).
 constexpr int NOALLOC_MAX_N = 128;
 constexpr size_t NOALLOC_SCRATCH_BYTES = ccl_workspace_bytes(NOALLOC_MAX_N);
 constexpr int NOALLOC_MAX_DEVICES = 64;
 // Device address of that array on `device` (looked up once per device with
 // hipGetSymbolAddress, that device made current for the lookup); null on error.
 void *noalloc_scratch(int device);
-void launch_ccl_label(const Fields &f, const Consts &c, unsigned *lab, hipStream_t s);
 // Label, list the roots in raster order, count each drop's cells.  Afterwards
 // *w.nroots holds the drop count; w.vol[0..count) the volumes when count <= cap.
 void launch_ccl_count(const Fields &f, const Consts &c, const CclWork &w, hipStream_t s);

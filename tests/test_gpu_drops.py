@@ -76,3 +76,26 @@ def test_workspace_reused_across_calls():
             cnt, vol, deq = s.drop_count()
             rc, rvol, rdeq = orc.drop_count(s.get_field(5))
             assert cnt == rc and np.array_equal(vol, rvol) and np.array_equal(deq, rdeq)
+
+
+@pytest.mark.parametrize("n", [4, 16, 54, 64, 72, 96, 128, 162])
+def test_mask_word_edges(n):
+    """Rows of one mask word, exact and ragged words, and several words: runs
+    that cross word ends and the periodic seam, full rows, full and empty boxes."""
+    rng = np.random.default_rng(n)
+    fields = [np.zeros((n, n, n)), np.ones((n, n, n)), rng.uniform(0, 1, (n, n, n)) ** 0.3,
+              rng.uniform(0, 1, (n, n, n)) ** 5]
+    rows = np.zeros((n, n, n))
+    rows[:, ::3, ::3] = 1.0                           # full rows, two apart where n allows
+    rows[n // 2, 1::3, ::6] = 1.0                     # some joined by a straight and diagonal cells
+    fields.append(rows)
+    edge = np.zeros((n, n, n))
+    for x in {0, 1, n - 2, n - 1, min(62, n - 1), min(63, n - 1), min(64, n - 1)}:
+        edge[x, rng.integers(0, n, 6), rng.integers(0, n, 6)] = 1.0
+    fields.append(edge)
+    with Solver(nx=n, dt=1e-3, mu=0.01, phiflag=1, inphi=1) as s:
+        for phi in fields:
+            s.set_field(5, phi)
+            cnt, vol, deq = s.drop_count(max_drops=n ** 3)
+            rc, rvol, rdeq = orc.drop_count(phi)
+            assert cnt == rc and np.array_equal(vol, rvol) and np.array_equal(deq, rdeq)
