@@ -90,6 +90,7 @@ struct Fields {
     double *mtab;                // log/expm1 table (devmath.h layout)
     Scalars *sc;
     double *diag;                // 3 diagnostic sums (kinetic, strain, phase)
+    Scalars *mirror = nullptr;   // host-mapped copy of *sc as the last step left it
     EnsSlot *slot = nullptr;     // host-mapped progress record (ensemble boxes only)
     int ld;                      // spectrum leading dimension (>= n/2+1)
 };

@@ -1837,7 +1837,7 @@ __global__ void __launch_bounds__(64) k_reduce_planes(const double *__restrict__
 
 // Means (main.f90:906-913), signed umax (937-941), CFL (942-945), halt flag.
 __device__ __forceinline__ void k_finalize_body(uint3 blk, const double *__restrict__ psum, const double *__restrict__ pmax,
-                                                 Scalars *__restrict__ sc, Consts c, EnsSlot *slot)
+                                                 Scalars *__restrict__ sc, Consts c, Scalars *mirror, EnsSlot *slot)
 {
     if (sc->halted) return;
     const int n = c.n, lane = threadIdx.x;
@@ -1870,9 +1870,21 @@ __device__ __forceinline__ void k_finalize_body(uint3 blk, const double *__restr
         sc->cou = cou;
         const int steps = sc->steps + 1;
         sc->steps = steps;
-        int halt = 0;
-        if (nan) { sc->halted = 1; sc->status = 6; halt = 1; }
-        else if (cou > 7.0) { sc->halted = 1; sc->status = 5; halt = 1; }
+        const int status = nan ? 6 : cou > 7.0 ? 5 : 0, halt = status != 0;
+        if (halt) {
+            sc->halted = 1;
+            sc->status = status;
+        }
+        // the host's copy, its step count last: what mhit_step waits for
+        mirror->umean = gu;
+        mirror->vmean = gv;
+        mirror->wmean = gw;
+        mirror->gumax = gumax;
+        mirror->cou = cou;
+        mirror->halted = halt;
+        mirror->status = status;
+        __threadfence_system();
+        *(volatile int *)&mirror->steps = steps;
         if (slot) {
             slot->clk[steps % CLK_RING] = wall_clock64();
             if (halt) slot->halted = 1;
@@ -1883,9 +1895,9 @@ __device__ __forceinline__ void k_finalize_body(uint3 blk, const double *__restr
 }
 
 __global__ void __launch_bounds__(64) k_finalize(const double *__restrict__ psum, const double *__restrict__ pmax,
-                                                 Scalars *__restrict__ sc, Consts c, EnsSlot *slot)
+                                                 Scalars *__restrict__ sc, Consts c, Scalars *mirror, EnsSlot *slot)
 {
-    k_finalize_body(make_uint3(blockIdx.x, blockIdx.y, blockIdx.z), psum, pmax, sc, c, slot);
+    k_finalize_body(make_uint3(blockIdx.x, blockIdx.y, blockIdx.z), psum, pmax, sc, c, mirror, slot);
 }
 
 // ---------------------------------------------------------------------------
@@ -2035,7 +2047,7 @@ __global__ void __launch_bounds__(64) kg_reduce_planes(const GangBox *__restrict
 __global__ void __launch_bounds__(64) kg_finalize(const GangBox *__restrict__ g)
 {
     const GangBox &B = g[blockIdx.x];
-    k_finalize_body(make_uint3(0, 0, 0), B.f.psum, B.f.pmax, B.f.sc, B.c, B.f.slot);
+    k_finalize_body(make_uint3(0, 0, 0), B.f.psum, B.f.pmax, B.f.sc, B.c, B.f.mirror, B.f.slot);
 }
 
 
@@ -2917,7 +2929,7 @@ void launch_reduce(const Fields &f, const Consts &c, hipStream_t s, LaunchInfo *
 
 void launch_finalize(const Fields &f, const Consts &c, hipStream_t s, LaunchInfo *li)
 {
-    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(64), 0, s, f.psum, f.pmax, f.sc, c, f.slot);
+    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(64), 0, s, f.psum, f.pmax, f.sc, c, f.mirror, f.slot);
     li->name = "finalize"; li->bytes = 6.0 * 8.0 * c.n;
 }
 

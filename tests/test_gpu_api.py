@@ -242,3 +242,34 @@ def test_checkpoint_resume_is_bitwise(tmp_path, precision):
     with Solver(**other) as d:
         with pytest.raises(Exception):
             d.load_state(tmp_path / "box.state")
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("n", [4, 48, 108, 128, 192])
+def test_field_copies_in_pieces(n, precision):
+    """Fields in and out through the staged copy: one piece, a ragged last
+    piece, several threads; two boxes copying at once from two threads; the
+    pending mean of a velocity component subtracted in every piece."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    def one(seed):
+        rng = np.random.default_rng(seed)
+        kw = dict(nx=n, dt=1e-4, mu=0.01, phiflag=1, inphi=1, inflow=1, precision=precision)
+        with Solver(**kw) as s:
+            for f in (1, 2, 3, 4, 5):
+                a = np.asfortranarray(rng.standard_normal((n, n, n)))
+                s.set_field(f, a)
+                want = a.astype(np.float32).astype(np.float64) if precision and f != 4 else a
+                assert np.array_equal(s.get_field(f), want), f
+            u = np.asfortranarray(rng.uniform(0.1, 0.2, (n, n, n)))
+            for f in (1, 2, 3):
+                s.set_field(f, u)
+            s.set_field(5, np.zeros((n, n, n)))
+            d = s.step(1)                              # leaves pending means
+            got = s.get_field(1)
+            assert d.umean != 0.0 and abs(got.mean()) < 1e-6
+            return float(got.max()), d.gumax
+
+    with ThreadPoolExecutor(2) as ex:
+        a, b = ex.map(one, (1, 2))
+    assert one(1) == a and one(2) == b
