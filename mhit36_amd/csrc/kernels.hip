@@ -2602,23 +2602,48 @@ void launch_debug_math(int op, size_t count, const double *x, double *y, const d
 
 static inline double F(const Consts &c) { return 8.0 * (double)c.n * c.n * c.n; }
 
-// Planes per block for the z-marching kernels: the largest of 32..2 dividing
-// n that still gives >= `target` blocks (over `boxes` boxes launched
-// together), else the largest of 8..2 dividing n.  One box asks for 2048
-// blocks; a gang for 1024, since thin slabs cost halo planes (a block
-// recomputes kz + 4 psi planes for kz output planes).
-static int march_kz(int n, int tx, int ty, int boxes = 1, int target = 2048)
+// Planes per block for the z-marching kernels: of the powers of two dividing n,
+// the one of least cost rounds (kz + extra), the rounds of resident blocks
+// times the planes each works through; up to two rounds count whole, beyond
+// that blocks end at different times and the rounds blur.  A thicker slab has
+// to gain 2%.  `boxes` boxes launched together count as so many times the blocks.
+static int march_kz(int n, int tiles, int slots, int extra, int most, int boxes = 1)
 {
-    for (int kz = 32; kz > 1; kz >>= 1)
-        if (n % kz == 0 && boxes * (n / kz) * ((n + tx - 1) / tx) * ((n + ty - 1) / ty) >= target) return kz;
-    for (int kz = 8; kz > 1; kz >>= 1)
-        if (n % kz == 0) return kz;
-    return 1;
+    int best = 1;
+    double least = 0.0;
+    for (int kz = 2; kz <= most && n % kz == 0; kz *= 2) {
+        const double r = (double)boxes * tiles * (n / kz) / slots;
+        const double cost = (r <= 1.0 ? 1.0 : r <= 2.0 ? 2.0 : r) * (kz + extra);
+        if (best == 1 || cost < 0.98 * least) {
+            best = kz;
+            least = cost;
+        }
+    }
+    return best;
+}
+// The constants are fitted to sweeps of kz at 16^3 to 512^3 (16, 32, 48, 64,
+// 96, 108, 128, 192, 256, 384, 512; times in us, this rule / the best kz / a
+// target of 2048 blocks, the rule before):
+//   phase field FP64   64^3: 13.1 / 13.1 / 22.3  128^3: 32.5 / 32.5 / 54.9  256^3: 184 / 184 / 195
+//   phase field FP32   64^3: 9.2 / 9.2 / 14.0    128^3: 17.8 / 17.8 / 22.8  256^3: 86.4 / 86.4 / 86.4
+//   momentum FP64      64^3: 14.4 / 14.4 / 25.3  128^3: 52.6 / 52.6 / 56.3  256^3: 386 / 380 / 386
+//   momentum FP32      64^3: 13.1 / 13.1 / 25.9  128^3: 31.9 / 31.9 / 35.4  256^3: 192 / 192 / 201
+// A phase-field block recomputes 4 planes of psi in its prologue; two FP64
+// blocks are resident per CU, of FP32's four the last adds little.  A momentum
+// block's prologue reads planes that its neighbour has just read.
+static int kz_acdi(int n, int mixed, int boxes = 1)
+{
+    return march_kz(n, ((n + ATX - 1) / ATX) * ((n + ATY - 1) / ATY), mixed ? 768 : 512, 4, 64, boxes);
+}
+static int kz_momentum(int n, int mixed, int boxes = 1)
+{
+    const int tx = mixed ? 2 * PTX : MTX, ty = mixed ? PTY : MTY;
+    return march_kz(n, ((n + tx - 1) / tx) * ((n + ty - 1) / ty), mixed ? 768 : 1024, mixed ? 3 : 1, 32, boxes);
 }
 
 void launch_acdi(const Fields &f, const Consts &c, const Tuning &tu, hipStream_t s, LaunchInfo *li)
 {
-    const int n = c.n, kz = tu.v[KNOB_KZ_ACDI] ? tu.v[KNOB_KZ_ACDI] : march_kz(n, ATX, ATY);
+    const int n = c.n, kz = tu.v[KNOB_KZ_ACDI] ? tu.v[KNOB_KZ_ACDI] : kz_acdi(n, c.mixed);
     dim3 grid((n + ATX - 1) / ATX, (n + ATY - 1) / ATY, n / kz);
     if (c.mixed)
         hipLaunchKernelGGL(k_acdi<float>, grid, dim3(ATHREADS), 0, s, (const float *)f.u, (const float *)f.v,
@@ -2632,7 +2657,7 @@ void launch_acdi(const Fields &f, const Consts &c, const Tuning &tu, hipStream_t
 void launch_momentum(const Fields &f, const Consts &c, const Tuning &tu, double alpha, double beta, hipStream_t s,
                      LaunchInfo *li)
 {
-    const int n = c.n, kz = tu.v[KNOB_KZ_MOM] ? tu.v[KNOB_KZ_MOM] : march_kz(n, MTX, MTY);
+    const int n = c.n, kz = tu.v[KNOB_KZ_MOM] ? tu.v[KNOB_KZ_MOM] : kz_momentum(n, c.mixed);
     dim3 grid((n + MTX - 1) / MTX, (n + MTY - 1) / MTY, n / kz);
     if (c.mixed) {
         using T = float;
@@ -2764,8 +2789,8 @@ int knob_default(int knob, const Consts &c, const FftPlan &pl)
 {
     const bool regs = plan_regs(pl);
     switch (knob) {
-    case KNOB_KZ_ACDI: return march_kz(c.n, ATX, ATY);
-    case KNOB_KZ_MOM: return march_kz(c.n, MTX, MTY);
+    case KNOB_KZ_ACDI: return kz_acdi(c.n, c.mixed);
+    case KNOB_KZ_MOM: return kz_momentum(c.n, c.mixed);
     case KNOB_XPAIRS:
     case KNOB_XIPAIRS: return regs ? rpairs(pl) : pairs_per_block(pl);
     default: return regs ? rtile(pl) : col_tile(pl);
@@ -2945,7 +2970,7 @@ void gang_layout(const GangBox *d, int nbox, const GangSize *sizes, GangLaunch *
     gl->phiflag = d[0].c.phiflag;
     for (int b = 0; b < nbox; b++) {
         const int n = d[b].c.n;
-        const int ka = march_kz(n, ATX, ATY, nbox, 1024), km = march_kz(n, MTX, MTY, nbox, 1024);
+        const int ka = kz_acdi(n, gl->mixed, nbox), km = kz_momentum(n, gl->mixed, nbox);
         gl->grid[GP_ACDI].kz[b] = ka;
         gl->grid[GP_MOM].kz[b] = km;
         const int blocks[GP_COUNT] = {
