@@ -1202,8 +1202,8 @@ __device__ __forceinline__ void stage_regs(double2 (&v)[8], int tj, int LM, int 
     constexpr int Q = 8 / R;
 #pragma unroll
     for (int q = 0; q < Q; q++) {
-        const int jj = tj + q * LM;
-        const int k = jj % Ns;
+        const unsigned jj = (unsigned)(tj + q * LM);
+        const int k = (int)(jj % (unsigned)Ns);
         double2 x[R];
 #pragma unroll
         for (int r = 0; r < R; r++) x[r] = v[q + r * Q];
@@ -1229,8 +1229,8 @@ __device__ __forceinline__ void store_stage(const double2 (&v)[8], double2 *lds,
     constexpr int Q = 8 / R;
 #pragma unroll
     for (int q = 0; q < Q; q++) {
-        const int jj = tj + q * LM;
-        const int base = (jj / Ns) * Ns * R + jj % Ns;
+        const unsigned jj = (unsigned)(tj + q * LM), k = jj % (unsigned)Ns;
+        const int base = (int)((jj - k) * R + k);
 #pragma unroll
         for (int r = 0; r < R; r++) lds[rlds<XL>(line, base + r * Ns, lstride, pstride)] = v[q + r * Q];
     }
@@ -1262,101 +1262,166 @@ __device__ void fft_regs(double2 (&v)[8], int tj, int line, double2 *lds, int ls
     }
 }
 
-// The stage plan of a power-of-two length n = 2^L, L >= 4, at compile time:
-// the radices, sub-lengths Ns and twiddle offsets that the host plan builder
-// gives for that n (radix-8 stages, then two 4s when L mod 3 = 1, one 4 when
-// L mod 3 = 2).  With L known the stage loop unrolls and every index of the
-// exchanges (jj / Ns, jj % Ns, the line strides) is a shift or a mask; the
-// generic fft_regs computes them from the runtime plan with integer divides.
-__host__ __device__ constexpr int cplan_nst(int L)
+// The stage plan of a length N at compile time: the radices of the host plan
+// builder (plan_radices), with the sub-lengths Ns and twiddle offsets that the
+// host derives from them.  With N known the stage loop unrolls and every index
+// of the exchanges (jj / Ns, jj % Ns, the line strides) becomes shifts, masks
+// or a multiplication; fft_regs computes them from the runtime plan with
+// integer divides.
+struct CPlan {
+    int nst, R[MAXSTAGES], Ns[MAXSTAGES], off[MAXSTAGES];
+};
+__host__ __device__ constexpr CPlan cplan(int n)
 {
-    return L % 3 == 0 ? L / 3 : L / 3 + 1;
+    CPlan p = {};
+    p.nst = plan_radices(n, p.R);
+    int ns = 1, off = 0;
+    for (int s = 0; s < p.nst; s++) {
+        p.Ns[s] = ns;
+        p.off[s] = off;
+        off += ns * (p.R[s] - 1);
+        ns *= p.R[s];
+    }
+    return p;
 }
-__host__ __device__ constexpr int cplan_R(int L, int s)
+constexpr bool is_pow2(int n) { return (n & (n - 1)) == 0; }
+// Threads per line.  A power of two, or any plan with a radix-8 stage: n/8, one
+// radix-8 butterfly each (a radix-3 stage then takes 2 2/3 per thread, the
+// third for two threads of three).  Radices 4, 3 and 2 only: n/3, or n/6 with
+// two butterflies each from 144 on (FFT passes of a step at 108^3 FP64 63 against
+// 66 us, at 144^3 106 against 99 us).
+__host__ __device__ constexpr int line_threads(int n)
 {
-    return L % 3 == 0 ? 8 : L % 3 == 2 ? (s < L / 3 ? 8 : 4) : (s < L / 3 - 1 ? 8 : 4);
-}
-__host__ __device__ constexpr int cplan_Ns(int L, int s)
-{
-    int ns = 1;
-    for (int t = 0; t < s; t++) ns *= cplan_R(L, t);
-    return ns;
-}
-__host__ __device__ constexpr int cplan_twoff(int L, int s)
-{
-    int o = 0;
-    for (int t = 0; t < s; t++) o += cplan_Ns(L, t) * (cplan_R(L, t) - 1);
-    return o;
+    if (is_pow2(n)) return n / 8;
+    const CPlan p = cplan(n);
+    return p.R[0] == 8 ? n / 8 : n < 144 ? n / 3 : n / 6;
 }
 
-// The compile-time plan is the host's plan (plan_radices) for every compiled
-// length; Ns and the twiddle offsets follow from the radices the same way in
-// both.
-constexpr bool cplan_is_host_plan(int L)
-{
-    int rad[MAXSTAGES] = {};
-    const int ns = plan_radices(1 << L, rad);
-    if (ns != cplan_nst(L)) return false;
-    for (int st = 0; st < ns; st++)
-        if (rad[st] != cplan_R(L, st)) return false;
-    return true;
-}
-static_assert(cplan_is_host_plan(4) && cplan_is_host_plan(5) && cplan_is_host_plan(6) && cplan_is_host_plan(7) &&
-                  cplan_is_host_plan(8) && cplan_is_host_plan(9) && cplan_is_host_plan(10) &&
-                  cplan_is_host_plan(11),
-              "compile-time FFT plan differs from the host plan");
-
-template <int SG, bool XL, int L, int S = 0>
+template <int SG, bool XL, int N, int S = 0>
 __device__ __forceinline__ void fft_regs_c(double2 (&v)[8], int tj, int line, double2 *lds, int lstride,
                                            int pstride, const double2 *__restrict__ tw)
 {
-    static_assert(L >= 4, "the compile-time plan covers n >= 16");
-    constexpr int LM = (1 << L) / 8, R = cplan_R(L, S), Ns = cplan_Ns(L, S);
+    constexpr CPlan P = cplan(N);
+    constexpr int LM = N / 8, R = P.R[S], Ns = P.Ns[S];
+    static_assert(is_pow2(N) && N >= 16, "8 elements per thread");
     if constexpr (S > 0) {
 #pragma unroll
         for (int m = 0; m < 8; m++) v[m] = lds[rlds<XL>(line, tj + m * LM, lstride, pstride)];
         __syncthreads();
     }
-    stage_regs<R, SG>(v, tj, LM, Ns, tw + cplan_twoff(L, S), S == 0);
-    if constexpr (S + 1 < cplan_nst(L)) {
+    stage_regs<R, SG>(v, tj, LM, Ns, tw + P.off[S], S == 0);
+    if constexpr (S + 1 < P.nst) {
         store_stage<R, XL>(v, lds, line, tj, LM, Ns, lstride, pstride);
         __syncthreads();
-        fft_regs_c<SG, XL, L, S + 1>(v, tj, line, lds, lstride, pstride, tw);
+        fft_regs_c<SG, XL, N, S + 1>(v, tj, line, lds, lstride, pstride, tw);
     }
 }
 
-// All stages of one line: the compile-time plan for n = 2^L, L > 0, else the
-// runtime plan pl.
-template <int SG, bool XL, int L>
+// The same for a length with a factor 3, whose stages do not share one set of
+// positions per thread: thread tj of the line's T takes butterflies tj, tj + T,
+// ... of each stage.  The first stage reads position p through ld(p), the last
+// writes through st(p, value); LDS carries the exchanges between stages and may
+// also be what ld reads (FROM_LDS: a barrier before the first write to it).
+// Against the LDS form above, whose threads hold one butterfly of the smallest
+// radix: no staging of input and output, indices known at compile time, and
+// threads that all work in the radix-8 stages (of n/3 per line, 3/8 did).  The
+// FFT passes of a mixed-precision step, us: 96^3 64 -> 54, 192^3 242 -> 164,
+// 384^3 2025 -> 1160, 432^3 4272 -> 1880 (bound by memory from 192^3 on: 3.9-5.3
+// TB/s in the y passes).  Holding the least common multiple of the radices
+// per thread (24 points, no exchange between forward and inverse in the z pass)
+// left too few wavefronts: 192^3 186, 384^3 1258 us.
+template <int SG, bool XL, int N, bool FROM_LDS, int S = 0, typename LD, typename ST>
+__device__ __forceinline__ void fft_threes(int tj, int line, double2 *lds, int lstride, int pstride,
+                                           const double2 *__restrict__ tw, LD &&ld, ST &&st)
+{
+    constexpr CPlan P = cplan(N);
+    constexpr int T = line_threads(N), R = P.R[S], Ns = P.Ns[S], L = N / R, Q = (L + T - 1) / T;
+    constexpr bool last = S + 1 == P.nst;
+    double2 x[Q][R];
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+        const int j = tj + q * T;
+        if (L % T == 0 || j < L)
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                if constexpr (S == 0) x[q][r] = ld(j + r * L);
+                else x[q][r] = lds[rlds<XL>(line, j + r * L, lstride, pstride)];
+            }
+    }
+    if (S > 0 || FROM_LDS) __syncthreads();
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+        const int j = tj + q * T;
+        if (L % T == 0 || j < L) {
+            const unsigned k = (unsigned)j % (unsigned)Ns;
+            if constexpr (S > 0)
+#pragma unroll
+                for (int r = 1; r < R; r++) {
+                    const double2 wv = tw[P.off[S] + (int)k * (R - 1) + r - 1];
+                    const double wi = SG < 0 ? -wv.y : wv.y;
+                    const double xr = x[q][r].x, xi = x[q][r].y;
+                    x[q][r] = make_double2(xr * wv.x - xi * wi, xr * wi + xi * wv.x);
+                }
+            dft<R, SG>(x[q]);
+            const int base = (int)(((unsigned)j - k) * R + k);
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                if constexpr (last) st(base + r * Ns, x[q][r]);
+                else lds[rlds<XL>(line, base + r * Ns, lstride, pstride)] = x[q][r];
+            }
+        }
+    }
+    if constexpr (!last) {
+        __syncthreads();
+        fft_threes<SG, XL, N, false, S + 1>(tj, line, lds, lstride, pstride, tw, ld, st);
+    }
+}
+
+// All stages of one line of a power of two: the compile-time plan for N > 0,
+// else the runtime plan pl.
+template <int SG, bool XL, int N>
 __device__ __forceinline__ void fft_lines(double2 (&v)[8], int tj, int line, double2 *lds, int lstride,
                                           int pstride, const FftPlan &pl, const double2 *__restrict__ tw)
 {
-    if constexpr (L > 0) fft_regs_c<SG, XL, L>(v, tj, line, lds, lstride, pstride, tw);
+    if constexpr (N > 0) fft_regs_c<SG, XL, N>(v, tj, line, lds, lstride, pstride, tw);
     else fft_regs<SG, XL>(v, tj, line, lds, lstride, pstride, pl, tw);
 }
 
 __host__ __device__ constexpr int rline_stride(int n) { return n + n / 8 + 1; }
 
 // Default launch shapes of the register kernels: columns per block of the y/z
-// passes and x-line pairs per block (threads = shape * n/8 <= 1024, pairs
+// passes and x-line pairs per block (threads = shape * line_threads <= 1024, pairs
 // dividing n*n/2).  A column tile keeps whole 128-byte lines (8 columns) up to
 // 2*LDS_CAP of LDS, one block per CU: at 1024 rows that beats two blocks of
 // 4-column tiles, whose 64-byte row pieces half-use each line (z pass 5.9 ->
-// 5.4 ms at 1024^3).  Line pairs stay within LDS_CAP.
+// 5.4 ms at 1024^3).  Line pairs stay within LDS_CAP; with a factor 3 within
+// 28 KB, five blocks per CU (forward x pass of 384^3 FP64 with 8, 4, 2 pairs:
+// 404, 372, 415 us; 432^3 with 4, 2, 1: 704, 614, 670 us).
 static constexpr int rtile_n(int n)
 {
     int t = 8;
-    while (t > 1 && t * (n / 8) > FFT_MAX_THREADS) t >>= 1;
+    while (t > 1 && t * line_threads(n) > FFT_MAX_THREADS) t >>= 1;
     while (t > 1 && (size_t)t * n * sizeof(double2) > 2 * LDS_CAP) t >>= 1;
     return t;
 }
 static constexpr int rpairs_n(int n)
 {
     int p = 8;
-    while (p > 1 && p * (n / 8) > FFT_MAX_THREADS) p >>= 1;
-    while (p > 1 && (size_t)p * rline_stride(n) * sizeof(double2) > LDS_CAP) p >>= 1;
+    while (p > 1 && p * line_threads(n) > FFT_MAX_THREADS) p >>= 1;
+    const size_t cap = is_pow2(n) ? LDS_CAP : 28 * 1024;
+    while (p > 1 && (size_t)p * rline_stride(n) * sizeof(double2) > cap) p >>= 1;
     while (p > 1 && (n * n / 2) % p != 0) p >>= 1;
     return p;
+}
+// Most threads a block of the kernel for N is launched with (N = 0: any power
+// of two): x passes up to 16 pairs, column passes their default tile.
+static constexpr int x_threads(int n)
+{
+    return n == 0 || is_pow2(n) ? FFT_MAX_THREADS : std::min(FFT_MAX_THREADS, (16 * line_threads(n) + 63) / 64 * 64);
+}
+static constexpr int col_threads(int n)
+{
+    return n == 0 || is_pow2(n) ? FFT_MAX_THREADS : (rtile_n(n) * line_threads(n) + 63) / 64 * 64;
 }
 
 // 16-byte streaming store of one complex value (written once, not re-read by this kernel).
@@ -1385,7 +1450,7 @@ __device__ __forceinline__ int mirror_lane(int tj, int LM)
     return (int)(threadIdx.x & 63) - tj + ((LM - tj) & (LM - 1));
 }
 
-template <typename T, int L = 0>
+template <typename T, int N = 0>
 __device__ __forceinline__ void k_xfwd_r_body(uint3 blk,
     const T *__restrict__ us, const T *__restrict__ vs, const T *__restrict__ ws,
     double2 *__restrict__ spec, const double2 *__restrict__ tw, const Scalars *__restrict__ sc,
@@ -1393,17 +1458,14 @@ __device__ __forceinline__ void k_xfwd_r_body(uint3 blk,
 {
     if (halted(sc)) return;
     extern __shared__ double2 lds[];
-    const int n = L ? (1 << L) : c.n, half = n / 2, nh = n / 2 + 1, LM = n / 8;
+    const int n = N ? N : c.n, half = n / 2, nh = n / 2 + 1, LM = N ? line_threads(N) : n / 8;
     const int lstride = rline_stride(n);
     const int t = threadIdx.x, pl_ = t / LM, tj = t - pl_ * LM;
     const int pair = blk.x * ppb + pl_;
     const int k = pair / half, j = 2 * (pair - k * half);
     const int kp = k + 1 == n ? 0 : k + 1;
     const double cdiv = c.rho * c.dxi / c.dt;
-    double2 v[8];
-#pragma unroll
-    for (int m = 0; m < 8; m++) {
-        const int i = tj + m * LM;
+    auto rhs = [&](int i) {                     // Poisson right-hand side at points (i, j, k) and (i, j+1, k)
         const int ip = i + 1 == n ? 0 : i + 1;
         double rr[2];
 #pragma unroll
@@ -1417,33 +1479,43 @@ __device__ __forceinline__ void k_xfwd_r_body(uint3 blk,
             if (c.fp32_rhs) r = (double)(float)r;
             rr[h] = r;
         }
-        v[m] = make_double2(rr[0], rr[1]);
-    }
-    fft_lines<-1, true, L>(v, tj, pl_, lds, lstride, 1, pl, tw);
-    if (LM <= 64) {
-        // split z into the two real lines' half spectra (q = 0 .. n/2); z[n-q]
-        // from the mirror lane instead of a round trip through LDS
-        const int src = mirror_lane(tj, LM);
-        double2 *r1 = spec + spec_row(k, j, n, ld), *r2 = spec + spec_row(k, j + 1, n, ld);
+        return make_double2(rr[0], rr[1]);
+    };
+    double2 v[8];
+    if constexpr (N > 0 && !is_pow2(N)) {
+        fft_threes<-1, true, N, false>(tj, pl_, lds, lstride, 1, tw, rhs, [&](int p, double2 z) {
+            lds[rlds<true>(pl_, p, lstride, 1)] = z;
+        });
+        __syncthreads();
+    } else {
 #pragma unroll
-        for (int m = 0; m < 4; m++) {
-            const int q = tj + m * LM;
-            double2 zm = lane_get2(v[7 - m], src);
-            if (tj == 0) zm = v[(8 - m) & 7];
-            const double a = v[m].x, b = v[m].y, cc = zm.x, d = zm.y;
-            nt_store2(&r1[q], (a + cc) * 0.5, (b - d) * 0.5);
-            nt_store2(&r2[q], (b + d) * 0.5, (cc - a) * 0.5);
-        }
-        if (tj == 0) {                        // q = n/2, its own mirror
-            const double a = v[4].x, b = v[4].y, cc = v[4].x, d = v[4].y;
-            nt_store2(&r1[half], (a + cc) * 0.5, (b - d) * 0.5);
-            nt_store2(&r2[half], (b + d) * 0.5, (cc - a) * 0.5);
-        }
-        return;
-    }
+        for (int m = 0; m < 8; m++) v[m] = rhs(tj + m * LM);
+        fft_lines<-1, true, N>(v, tj, pl_, lds, lstride, 1, pl, tw);
+        if (LM <= 64) {
+            // split z into the two real lines' half spectra (q = 0 .. n/2); z[n-q]
+            // from the mirror lane instead of a round trip through LDS
+            const int src = mirror_lane(tj, LM);
+            double2 *r1 = spec + spec_row(k, j, n, ld), *r2 = spec + spec_row(k, j + 1, n, ld);
 #pragma unroll
-    for (int m = 0; m < 8; m++) lds[rlds<true>(pl_, tj + m * LM, lstride, 1)] = v[m];
-    __syncthreads();
+            for (int m = 0; m < 4; m++) {
+                const int q = tj + m * LM;
+                double2 zm = lane_get2(v[7 - m], src);
+                if (tj == 0) zm = v[(8 - m) & 7];
+                const double a = v[m].x, b = v[m].y, cc = zm.x, d = zm.y;
+                nt_store2(&r1[q], (a + cc) * 0.5, (b - d) * 0.5);
+                nt_store2(&r2[q], (b + d) * 0.5, (cc - a) * 0.5);
+            }
+            if (tj == 0) {                        // q = n/2, its own mirror
+                const double a = v[4].x, b = v[4].y, cc = v[4].x, d = v[4].y;
+                nt_store2(&r1[half], (a + cc) * 0.5, (b - d) * 0.5);
+                nt_store2(&r2[half], (b + d) * 0.5, (cc - a) * 0.5);
+            }
+            return;
+        }
+#pragma unroll
+        for (int m = 0; m < 8; m++) lds[rlds<true>(pl_, tj + m * LM, lstride, 1)] = v[m];
+        __syncthreads();
+    }
     for (int e = t; e < ppb * nh; e += blockDim.x) {
         int pq = e / nh, q = e - pq * nh;
         int pr = blk.x * ppb + pq;
@@ -1456,18 +1528,20 @@ __device__ __forceinline__ void k_xfwd_r_body(uint3 blk,
     }
 }
 
-template <typename T, int L>
-__global__ void __launch_bounds__(FFT_MAX_THREADS) k_xfwd_r(
+// With a factor 3, at most 4 waves per SIMD: left to itself the compiler holds
+// some lengths to 46 VGPRs and waits for each load (48^3 FP64: 13.3 -> 7.2 us).
+template <typename T, int N>
+__global__ void __launch_bounds__(x_threads(N)) __attribute__((amdgpu_waves_per_eu(1, N && !is_pow2(N) ? 4 : 8))) k_xfwd_r(
     const T *__restrict__ us, const T *__restrict__ vs, const T *__restrict__ ws,
     double2 *__restrict__ spec, const double2 *__restrict__ tw, const Scalars *__restrict__ sc,
     Consts c, FftPlan pl, int ppb, int ld)
 {
-    k_xfwd_r_body<T, L>(make_uint3(blockIdx.x, blockIdx.y, blockIdx.z), us, vs, ws, spec, tw, sc, c, pl, ppb, ld);
+    k_xfwd_r_body<T, N>(make_uint3(blockIdx.x, blockIdx.y, blockIdx.z), us, vs, ws, spec, tw, sc, c, pl, ppb, ld);
 }
 
 
-// L > 0: n = 2^L and TK columns per block, both compile-time
-template <int SG, int L = 0, int TK = 0>
+// N > 0: n = N and TK columns per block, both compile-time
+template <int SG, int N = 0, int TK = 0>
 __device__ __forceinline__ void k_ypass_r_body(uint3 blk, double2 *__restrict__ spec,
                                                              const double2 *__restrict__ tw,
                                                              const Scalars *__restrict__ sc, FftPlan pl, int ld,
@@ -1475,32 +1549,39 @@ __device__ __forceinline__ void k_ypass_r_body(uint3 blk, double2 *__restrict__ 
 {
     if (halted(sc)) return;
     extern __shared__ double2 lds[];
-    const int n = L ? (1 << L) : pl.n, nh = n / 2 + 1, LM = n / 8, tkx = TK ? TK : tkx_;
+    const int n = N ? N : pl.n, nh = n / 2 + 1, LM = n / 8, tkx = TK ? TK : tkx_;
     const int q0 = blk.x * tkx, k = blk.y;
     const int t = threadIdx.x, line = t % tkx, tj = t / tkx;
     const bool ok = q0 + line < nh;
     double2 *base = spec + spec_row(k, 0, n, ld) + q0 + line;
+    if constexpr (N > 0 && !is_pow2(N)) {
+        fft_threes<SG, false, N, false>(
+            tj, line, lds, 1, tkx, tw,
+            [&](int p) { return ok ? base[(size_t)p * ld] : make_double2(0.0, 0.0); },
+            [&](int p, double2 z) { if (ok) nt_store2(&base[(size_t)p * ld], z.x, z.y); });
+        return;
+    }
     double2 v[8];
 #pragma unroll
     for (int m = 0; m < 8; m++) v[m] = ok ? base[(size_t)(tj + m * LM) * ld] : make_double2(0.0, 0.0);
-    fft_lines<SG, false, L>(v, tj, line, lds, 1, tkx, pl, tw);
+    if constexpr (N == 0 || is_pow2(N)) fft_lines<SG, false, N>(v, tj, line, lds, 1, tkx, pl, tw);
     if (ok) {
 #pragma unroll
         for (int m = 0; m < 8; m++) nt_store2(&base[(size_t)(tj + m * LM) * ld], v[m].x, v[m].y);
     }
 }
 
-template <int SG, int L, int TK>
-__global__ void __launch_bounds__(FFT_MAX_THREADS) k_ypass_r(double2 *__restrict__ spec,
+template <int SG, int N, int TK>
+__global__ void __launch_bounds__(col_threads(N)) k_ypass_r(double2 *__restrict__ spec,
                                                              const double2 *__restrict__ tw,
                                                              const Scalars *__restrict__ sc, FftPlan pl, int ld,
                                                              int tkx)
 {
-    k_ypass_r_body<SG, L, TK>(make_uint3(blockIdx.x, blockIdx.y, blockIdx.z), spec, tw, sc, pl, ld, tkx);
+    k_ypass_r_body<SG, N, TK>(make_uint3(blockIdx.x, blockIdx.y, blockIdx.z), spec, tw, sc, pl, ld, tkx);
 }
 
 
-template <bool INV_ONLY = false, int L = 0, int TK = 0>
+template <bool INV_ONLY = false, int N = 0, int TK = 0>
 __device__ __forceinline__ void k_zpoisson_r_body(uint3 blk, double2 *__restrict__ spec,
                                                                 const double2 *__restrict__ tw,
                                                                 const double *__restrict__ ktab,
@@ -1509,35 +1590,46 @@ __device__ __forceinline__ void k_zpoisson_r_body(uint3 blk, double2 *__restrict
 {
     if (halted(sc)) return;
     extern __shared__ double2 lds[];
-    const int n = L ? (1 << L) : pl.n, nh = n / 2 + 1, LM = n / 8, tkx = TK ? TK : tkx_;
+    const int n = N ? N : pl.n, nh = n / 2 + 1, LM = n / 8, tkx = TK ? TK : tkx_;
     const int q0 = blk.x * tkx, j = blk.y;
     const int t = threadIdx.x, line = t % tkx, tj = t / tkx;
     const int q = q0 + line;
     const bool ok = q < nh;
     const size_t rs = spec_plane(n, ld);
     double2 *base = spec + (size_t)j * ld + q;
-    double2 v[8];
+    const double nnn = (double)((long long)n * (long long)n * (long long)n);
+    const double ky = ktab[j], kx = ktab[ok ? q : 0];
+    auto solve = [&](int r, double2 z) {        // the divide by -k^2 and N^3 at row r
+        double kz = ktab[r];
+        double k2 = (kx * kx + ky * ky) + kz * kz;
+        z = make_double2(((-z.x) / k2) / nnn, ((-z.y) / k2) / nnn);
+        if (q == 0 && j == 0 && r == 0) z = make_double2(0.0, 0.0);
+        return z;
+    };
+    if constexpr (N > 0 && !is_pow2(N)) {
+        static_assert(!INV_ONLY, "the generator's inverse runs the other forms");
+        fft_threes<-1, false, N, false>(
+            tj, line, lds, 1, tkx, tw,
+            [&](int p) { return ok ? base[(size_t)p * rs] : make_double2(0.0, 0.0); },
+            [&](int p, double2 z) { lds[rlds<false>(line, p, 1, tkx)] = solve(p, z); });
+        __syncthreads();
+        fft_threes<1, false, N, true>(
+            tj, line, lds, 1, tkx, tw, [&](int p) { return lds[rlds<false>(line, p, 1, tkx)]; },
+            [&](int p, double2 z) { if (ok) nt_store2(&base[(size_t)p * rs], z.x, z.y); });
+    } else {
+        double2 v[8];
 #pragma unroll
-    for (int m = 0; m < 8; m++) v[m] = ok ? base[(size_t)(tj + m * LM) * rs] : make_double2(0.0, 0.0);
-    if constexpr (!INV_ONLY) {
-        fft_lines<-1, false, L>(v, tj, line, lds, 1, tkx, pl, tw);
-        const double nnn = (double)((long long)n * (long long)n * (long long)n);
-        const double ky = ktab[j], kx = ktab[ok ? q : 0];
+        for (int m = 0; m < 8; m++) v[m] = ok ? base[(size_t)(tj + m * LM) * rs] : make_double2(0.0, 0.0);
+        if constexpr (!INV_ONLY) {
+            fft_lines<-1, false, N>(v, tj, line, lds, 1, tkx, pl, tw);
 #pragma unroll
-        for (int m = 0; m < 8; m++) {
-            const int r = tj + m * LM;
-            double kz = ktab[r];
-            double k2 = (kx * kx + ky * ky) + kz * kz;
-            double2 z = v[m];
-            z = make_double2(((-z.x) / k2) / nnn, ((-z.y) / k2) / nnn);
-            if (q == 0 && j == 0 && r == 0) z = make_double2(0.0, 0.0);
-            v[m] = z;
+            for (int m = 0; m < 8; m++) v[m] = solve(tj + m * LM, v[m]);
         }
-    }
-    fft_lines<1, false, L>(v, tj, line, lds, 1, tkx, pl, tw);
-    if (ok) {
+        fft_lines<1, false, N>(v, tj, line, lds, 1, tkx, pl, tw);
+        if (ok) {
 #pragma unroll
-        for (int m = 0; m < 8; m++) nt_store2(&base[(size_t)(tj + m * LM) * rs], v[m].x, v[m].y);
+            for (int m = 0; m < 8; m++) nt_store2(&base[(size_t)(tj + m * LM) * rs], v[m].x, v[m].y);
+        }
     }
 }
 
@@ -1559,19 +1651,19 @@ __global__ void __launch_bounds__(FFT_MAX_THREADS) k_zinv(double2 *__restrict__ 
     k_zpoisson_body<true>(make_uint3(blockIdx.x, blockIdx.y, blockIdx.z), spec, tw, ktab, sc, pl, ld, tkx);
 }
 
-template <int L, int TK>
-__global__ void __launch_bounds__(FFT_MAX_THREADS) k_zpoisson_r(double2 *__restrict__ spec,
+template <int N, int TK>
+__global__ void __launch_bounds__(col_threads(N)) k_zpoisson_r(double2 *__restrict__ spec,
                                                                 const double2 *__restrict__ tw,
                                                                 const double *__restrict__ ktab,
                                                                 const Scalars *__restrict__ sc, FftPlan pl, int ld,
                                                                 int tkx)
 {
-    k_zpoisson_r_body<false, L, TK>(make_uint3(blockIdx.x, blockIdx.y, blockIdx.z), spec, tw, ktab, sc, pl, ld,
+    k_zpoisson_r_body<false, N, TK>(make_uint3(blockIdx.x, blockIdx.y, blockIdx.z), spec, tw, ktab, sc, pl, ld,
                                     tkx);
 }
 
 
-template <int L = 0>
+template <int N = 0>
 __device__ __forceinline__ void k_xinv_r_body(uint3 blk, const double2 *__restrict__ spec,
                                                             double *__restrict__ p, const double2 *__restrict__ tw,
                                                             const Scalars *__restrict__ sc, FftPlan pl, int ppb,
@@ -1579,13 +1671,32 @@ __device__ __forceinline__ void k_xinv_r_body(uint3 blk, const double2 *__restri
 {
     if (halted(sc)) return;
     extern __shared__ double2 lds[];
-    const int n = L ? (1 << L) : pl.n, half = n / 2, LM = n / 8;
+    const int n = N ? N : pl.n, half = n / 2, LM = N ? line_threads(N) : n / 8;
     const int lstride = rline_stride(n);
     const int t = threadIdx.x, pl_ = t / LM, tj = t - pl_ * LM;
     const int pair = blk.x * ppb + pl_;
     const int k = pair / half, j = 2 * (pair - k * half);
     const double2 *s1 = spec + spec_row(k, j, n, ld);
     const double2 *s2 = spec + spec_row(k, j + 1, n, ld);
+    if constexpr (N > 0 && !is_pow2(N)) {
+        // the half spectra of the block's pairs into LDS, each value read once
+        for (int e = t; e < ppb * (half + 1); e += blockDim.x) {
+            const int pq = e / (half + 1), q = e - pq * (half + 1);
+            const int pr = blk.x * ppb + pq, kk = pr / half, jj = 2 * (pr - kk * half);
+            const double2 a = spec[spec_row(kk, jj, n, ld) + q], b = spec[spec_row(kk, jj + 1, n, ld) + q];
+            const bool own = q == 0 || q == half;                  // its own mirror
+            lds[rlds<true>(pq, q, lstride, 1)] = own ? make_double2(a.x, b.x) : make_double2(a.x - b.y, a.y + b.x);
+            if (!own) lds[rlds<true>(pq, n - q, lstride, 1)] = make_double2(a.x + b.y, b.x - a.y);
+        }
+        __syncthreads();
+        fft_threes<1, true, N, true>(
+            tj, pl_, lds, lstride, 1, tw, [&](int q) { return lds[rlds<true>(pl_, q, lstride, 1)]; },
+            [&](int i, double2 z) {
+                __builtin_nontemporal_store(z.x, &p[IDX(i, j, k)]);
+                __builtin_nontemporal_store(z.y, &p[IDX(i, j + 1, k)]);
+            });
+        return;
+    }
     double2 v[8];
     if (LM <= 64) {
         // Each spectrum value is loaded once: positions below n/2 directly,
@@ -1629,7 +1740,7 @@ __device__ __forceinline__ void k_xinv_r_body(uint3 blk, const double2 *__restri
             v[m] = z;
         }
     }
-    fft_lines<1, true, L>(v, tj, pl_, lds, lstride, 1, pl, tw);
+    if constexpr (N == 0 || is_pow2(N)) fft_lines<1, true, N>(v, tj, pl_, lds, lstride, 1, pl, tw);
 #pragma unroll
     for (int m = 0; m < 8; m++) {
         const int i = tj + m * LM;
@@ -1638,15 +1749,15 @@ __device__ __forceinline__ void k_xinv_r_body(uint3 blk, const double2 *__restri
     }
 }
 
-template <int L>
-__global__ void __launch_bounds__(FFT_MAX_THREADS) k_xinv_r(const double2 *__restrict__ spec,
+template <int N>
+__global__ void __launch_bounds__(x_threads(N)) k_xinv_r(const double2 *__restrict__ spec,
                                                             double *__restrict__ p, const double2 *__restrict__ tw,
                                                             const Scalars *__restrict__ sc, FftPlan pl, int ppb,
                                                             int ld)
 {
     // last pairs first: the y inverse pass wrote the highest planes last, and
     // some of them are still in the memory-side cache
-    k_xinv_r_body<L>(make_uint3(gridDim.x - 1 - blockIdx.x, blockIdx.y, blockIdx.z), spec, p, tw, sc, pl, ppb, ld);
+    k_xinv_r_body<N>(make_uint3(gridDim.x - 1 - blockIdx.x, blockIdx.y, blockIdx.z), spec, p, tw, sc, pl, ppb, ld);
 }
 
 
@@ -1979,49 +2090,49 @@ __global__ void __launch_bounds__(PTHREADS) kg_momentum_x2(const GangBox *__rest
 }
 
 // FFT passes: box = the first grid dimension the one-box launch leaves unused.
-template <typename T, bool REGS, int L>
-__global__ void __launch_bounds__(FFT_MAX_THREADS) kg_xfwd(const GangBox *__restrict__ g, FftPlan pl, int ppb, int ld)
+template <typename T, bool REGS, int N>
+__global__ void __launch_bounds__(x_threads(N)) kg_xfwd(const GangBox *__restrict__ g, FftPlan pl, int ppb, int ld)
 {
     const GangBox &B = g[blockIdx.y];
     const uint3 b = make_uint3(blockIdx.x, 0, 0);
     if constexpr (REGS)
-        k_xfwd_r_body<T, L>(b, (const T *)B.f.us, (const T *)B.f.vs, (const T *)B.f.ws, B.f.spec, B.f.tw, B.f.sc, B.c,
+        k_xfwd_r_body<T, N>(b, (const T *)B.f.us, (const T *)B.f.vs, (const T *)B.f.ws, B.f.spec, B.f.tw, B.f.sc, B.c,
                          pl, ppb, ld);
     else
         k_xfwd_body<T>(b, (const T *)B.f.us, (const T *)B.f.vs, (const T *)B.f.ws, B.f.spec, B.f.tw, B.f.sc, B.c, pl,
                        ppb, ld);
 }
 
-template <int SG, bool REGS, int L>
-__global__ void __launch_bounds__(FFT_MAX_THREADS) kg_ypass(const GangBox *__restrict__ g, FftPlan pl, int ld, int tkx)
+template <int SG, bool REGS, int N>
+__global__ void __launch_bounds__(col_threads(N)) kg_ypass(const GangBox *__restrict__ g, FftPlan pl, int ld, int tkx)
 {
     const GangBox &B = g[blockIdx.z];
     const uint3 b = make_uint3(blockIdx.x, blockIdx.y, 0);
     if constexpr (REGS)
-        k_ypass_r_body<SG, L, L ? rtile_n(1 << L) : 0>(b, B.f.spec, B.f.tw, B.f.sc, pl, ld, tkx);
+        k_ypass_r_body<SG, N, N ? rtile_n(N) : 0>(b, B.f.spec, B.f.tw, B.f.sc, pl, ld, tkx);
     else
         k_ypass_body<SG>(b, B.f.spec, B.f.tw, B.f.sc, pl, ld, tkx);
 }
 
-template <bool REGS, int L>
-__global__ void __launch_bounds__(FFT_MAX_THREADS) kg_zpoisson(const GangBox *__restrict__ g, FftPlan pl, int ld,
+template <bool REGS, int N>
+__global__ void __launch_bounds__(col_threads(N)) kg_zpoisson(const GangBox *__restrict__ g, FftPlan pl, int ld,
                                                                int tkx)
 {
     const GangBox &B = g[blockIdx.z];
     const uint3 b = make_uint3(blockIdx.x, blockIdx.y, 0);
     if constexpr (REGS)
-        k_zpoisson_r_body<false, L, L ? rtile_n(1 << L) : 0>(b, B.f.spec, B.f.tw, B.f.ktab, B.f.sc, pl, ld, tkx);
+        k_zpoisson_r_body<false, N, N ? rtile_n(N) : 0>(b, B.f.spec, B.f.tw, B.f.ktab, B.f.sc, pl, ld, tkx);
     else
         k_zpoisson_body<false>(b, B.f.spec, B.f.tw, B.f.ktab, B.f.sc, pl, ld, tkx);
 }
 
-template <bool REGS, int L>
-__global__ void __launch_bounds__(FFT_MAX_THREADS) kg_xinv(const GangBox *__restrict__ g, FftPlan pl, int ppb, int ld)
+template <bool REGS, int N>
+__global__ void __launch_bounds__(x_threads(N)) kg_xinv(const GangBox *__restrict__ g, FftPlan pl, int ppb, int ld)
 {
     const GangBox &B = g[blockIdx.y];
     const uint3 b = make_uint3(blockIdx.x, 0, 0);
     if constexpr (REGS)
-        k_xinv_r_body<L>(b, B.f.spec, B.f.p, B.f.tw, B.f.sc, pl, ppb, ld);
+        k_xinv_r_body<N>(b, B.f.spec, B.f.p, B.f.tw, B.f.sc, pl, ppb, ld);
     else
         k_xinv_body(b, B.f.spec, B.f.p, B.f.tw, B.f.sc, pl, ppb, ld);
 }
@@ -2711,70 +2822,69 @@ static int col_tile(const FftPlan &pl)
     return t;
 }
 
-// The register-resident kernels need radices 8/4/2 only and one thread per
-// 8 elements: n a multiple of 8 with no radix-3 stage.
-static bool plan_regs(const FftPlan &pl)
-{
-    if (pl.n % 8 != 0 || pl.n < 16) return false;
-    for (int s = 0; s < pl.nst; s++)
-        if (pl.R[s] != 8 && pl.R[s] != 4 && pl.R[s] != 2) return false;
-    return true;
-}
+// The lengths the register kernels are compiled for, with the stage plan as
+// constants: the column passes for their default tile (rtile_n) alone, the x
+// passes for any number of line pairs per block.  FFT_SIZES_GANG: also in gang
+// launches (boxes of up to 128^3).
+#define FFT_SIZES_GANG(X) X(32) X(36) X(48) X(54) X(64) X(72) X(96) X(108) X(128)
+#define FFT_SIZES(X) FFT_SIZES_GANG(X) X(144) X(162) X(192) X(216) X(256) X(288) X(324) X(384) X(432) X(486) X(512) X(1024)
 
-// x-line pairs per block (register path): threads = p*n/8 <= 1024, LDS <= LDS_CAP.
-static int rpairs(const FftPlan &pl) { return rpairs_n(pl.n); }
-
-// kx columns per block (register path).
-static int rtile(const FftPlan &pl) { return rtile_n(pl.n); }
-
-// The register kernels are compiled for n = 2^L, 6 <= L <= 10, with the stage
-// plan as constants; the column passes also with their default tile (rtile)
-// as a constant, so another tile (a tuned one, say) runs the kernels compiled
-// for any n, which read the plan at run time.  The x passes take any number of
-// line pairs per block.  reg_log2 gives L when pl is the compiled plan, else 0.
-constexpr int REG_LMIN = 6, REG_LMAX = 10;
-static constexpr int rtile_c(int L) { return rtile_n(1 << L); }
-static int reg_log2(const FftPlan &pl)
+static bool compiled_n(int n, bool gang)
 {
-    int L = 0;
-    while (L < 30 && (1 << L) < pl.n) L++;
-    if ((1 << L) != pl.n || L < REG_LMIN || L > REG_LMAX || pl.nst != cplan_nst(L)) return 0;
-    for (int st = 0; st < pl.nst; st++)
-        if (pl.R[st] != cplan_R(L, st) || pl.Ns[st] != cplan_Ns(L, st) || pl.twoff[st] != cplan_twoff(L, st))
-            return 0;
-    return L;
-}
-// Calls fn(std::integral_constant<int, L>) for L in [REG_LMIN, REG_LMAX], or
-// with 0 for any other L.
-template <typename Fn>
-static void with_log2(int L, Fn &&fn)
-{
-    switch (L) {
-    case 6: fn(std::integral_constant<int, 6>()); break;
-    case 7: fn(std::integral_constant<int, 7>()); break;
-    case 8: fn(std::integral_constant<int, 8>()); break;
-    case 9: fn(std::integral_constant<int, 9>()); break;
-    case 10: fn(std::integral_constant<int, 10>()); break;
-    default: fn(std::integral_constant<int, 0>()); break;
+#define FFT_CASE(N) case N:
+    switch (n) {
+    FFT_SIZES_GANG(FFT_CASE)
+        return true;
+    default: break;
     }
-}
-// The same for the gang kernels, whose boxes are at most 128^3.
-template <typename Fn>
-static void with_log2_gang(int L, Fn &&fn)
-{
-    switch (L) {
-    case 6: fn(std::integral_constant<int, 6>()); break;
-    case 7: fn(std::integral_constant<int, 7>()); break;
-    default: fn(std::integral_constant<int, 0>()); break;
+    if (gang) return false;
+    switch (n) {
+    FFT_SIZES(FFT_CASE)
+        return true;
+    default: return false;
     }
+#undef FFT_CASE
 }
-// L for a column pass of tile tkx.
-static int reg_log2_cols(const FftPlan &pl, int tkx)
+// Calls fn(std::integral_constant<int, N>) for a compiled n, or with 0 for any other.
+template <bool GANG, typename Fn>
+static void with_n(int n, Fn &&fn)
 {
-    const int L = reg_log2(pl);
-    return L && tkx == rtile_c(L) ? L : 0;
+#define FFT_CASE(N) case N: fn(std::integral_constant<int, N>()); return;
+    if constexpr (GANG) {
+        switch (n) {
+        FFT_SIZES_GANG(FFT_CASE)
+        default: break;
+        }
+    } else {
+        switch (n) {
+        FFT_SIZES(FFT_CASE)
+        default: break;
+        }
+    }
+#undef FFT_CASE
+    fn(std::integral_constant<int, 0>());
 }
 
+// A power of two the runtime-plan register kernels take (radices 8/4/2, one
+// thread per 8 elements).
+static bool pow2_regs(const FftPlan &pl) { return pl.n >= 16 && is_pow2(pl.n); }
+
+// Which form an x pass takes, and a column pass of tile tkx: the register
+// kernels where n is compiled (a column pass also needs its default tile) or a
+// power of two, else the LDS-staged kernels.
+static bool x_regs(const FftPlan &pl, bool gang = false) { return compiled_n(pl.n, gang) || pow2_regs(pl); }
+static bool col_regs(const FftPlan &pl, int tkx, bool gang = false)
+{
+    return pow2_regs(pl) || (compiled_n(pl.n, gang) && tkx == rtile_n(pl.n));
+}
+// The length a column pass of tile tkx is compiled for, or 0.
+static int col_n(const FftPlan &pl, int tkx) { return tkx == rtile_n(pl.n) ? pl.n : 0; }
+// Default shapes.
+static int default_pairs(const FftPlan &pl, bool gang = false) { return x_regs(pl, gang) ? rpairs_n(pl.n) : pairs_per_block(pl); }
+static int default_tile(const FftPlan &pl, bool gang = false)
+{
+    return pow2_regs(pl) || compiled_n(pl.n, gang) ? rtile_n(pl.n) : col_tile(pl);
+}
 static int fft_threads(const FftPlan &pl, int nlines)
 {
     int t = nlines * (pl.n / plan_rmin(pl));
@@ -2787,21 +2897,20 @@ static int fft_threads(const FftPlan &pl, int nlines)
 // LDS_MAX bytes of LDS; pairs per block divide the n^2/2 line pairs.
 int knob_default(int knob, const Consts &c, const FftPlan &pl)
 {
-    const bool regs = plan_regs(pl);
     switch (knob) {
     case KNOB_KZ_ACDI: return kz_acdi(c.n, c.mixed);
     case KNOB_KZ_MOM: return kz_momentum(c.n, c.mixed);
     case KNOB_XPAIRS:
-    case KNOB_XIPAIRS: return regs ? rpairs(pl) : pairs_per_block(pl);
-    default: return regs ? rtile(pl) : col_tile(pl);
+    case KNOB_XIPAIRS: return default_pairs(pl);
+    default: return default_tile(pl);
     }
 }
 
 int knob_candidates(int knob, const Consts &c, const FftPlan &pl, int *out, int cap)
 {
     const int n = c.n;
-    const bool regs = plan_regs(pl);
-    const int per_line = regs ? n / 8 : n / plan_rmin(pl);   // threads per line
+    const bool regs = pow2_regs(pl);
+    const int per_line = regs ? n / 8 : n / plan_rmin(pl);   // most threads per line (the LDS-staged form's)
     int k = 0;
     for (int v = 1; v <= 1024 && k < cap; v *= 2) {
         bool ok;
@@ -2814,7 +2923,7 @@ int knob_candidates(int knob, const Consts &c, const FftPlan &pl, int *out, int 
             const size_t lds = sizeof(double2) * (size_t)v * n;
             ok = v <= 16 && v * per_line <= FFT_MAX_THREADS && lds <= LDS_MAX && v <= n / 2 + 1;
         }
-        if (ok) out[k++] = v;
+        if (ok || v == knob_default(knob, c, pl)) out[k++] = v;
     }
     return k;
 }
@@ -2822,61 +2931,53 @@ int knob_candidates(int knob, const Consts &c, const FftPlan &pl, int *out, int 
 void launch_xfwd(const Fields &f, const Consts &c, const FftPlan &pl, const Tuning &tu, hipStream_t s,
                  LaunchInfo *li)
 {
-    if (plan_regs(pl)) {
-        const int ppb = tu.v[KNOB_XPAIRS] ? tu.v[KNOB_XPAIRS] : rpairs(pl), pairs = c.n * c.n / 2;
+    const int ppb = tu.v[KNOB_XPAIRS] ? tu.v[KNOB_XPAIRS] : default_pairs(pl), pairs = c.n * c.n / 2;
+    const dim3 grid(pairs / ppb);
+    const float *us = (const float *)f.us, *vs = (const float *)f.vs, *ws = (const float *)f.ws;
+    if (x_regs(pl)) {
         const size_t shm = sizeof(double2) * (size_t)ppb * rline_stride(c.n);
-        const dim3 grid(pairs / ppb), blk(ppb * (c.n / 8));
-        with_log2(reg_log2(pl), [&](auto LC) {
-            constexpr int L = decltype(LC)::value;
+        const dim3 blk(ppb * line_threads(c.n));
+        with_n<false>(c.n, [&](auto NC) {
+            constexpr int N = decltype(NC)::value;
             if (c.mixed)
-                hipLaunchKernelGGL((k_xfwd_r<float, L>), grid, blk, shm, s, (const float *)f.us,
-                                   (const float *)f.vs, (const float *)f.ws, f.spec, f.tw, f.sc, c, pl, ppb, f.ld);
+                hipLaunchKernelGGL((k_xfwd_r<float, N>), grid, blk, shm, s, us, vs, ws, f.spec, f.tw, f.sc, c, pl, ppb,
+                                   f.ld);
             else
-                hipLaunchKernelGGL((k_xfwd_r<double, L>), grid, blk, shm, s, f.us, f.vs, f.ws, f.spec, f.tw, f.sc, c,
+                hipLaunchKernelGGL((k_xfwd_r<double, N>), grid, blk, shm, s, f.us, f.vs, f.ws, f.spec, f.tw, f.sc, c,
                                    pl, ppb, f.ld);
         });
-        li->name = "xfwd_div"; li->bytes = (c.mixed ? 2.5 : 4.0) * F(c);
-        return;
+    } else {
+        const size_t shm = sizeof(double2) * (size_t)ppb * (c.n + 1);
+        const dim3 blk(fft_threads(pl, ppb));
+        if (c.mixed)
+            hipLaunchKernelGGL(k_xfwd<float>, grid, blk, shm, s, us, vs, ws, f.spec, f.tw, f.sc, c, pl, ppb, f.ld);
+        else
+            hipLaunchKernelGGL(k_xfwd<double>, grid, blk, shm, s, f.us, f.vs, f.ws, f.spec, f.tw, f.sc, c, pl, ppb,
+                               f.ld);
     }
-    int ppb = tu.v[KNOB_XPAIRS] ? tu.v[KNOB_XPAIRS] : pairs_per_block(pl);
-    int pairs = c.n * c.n / 2;
-    size_t shm = sizeof(double2) * (size_t)ppb * (c.n + 1);
-    if (c.mixed)
-        hipLaunchKernelGGL(k_xfwd<float>, dim3(pairs / ppb), dim3(fft_threads(pl, ppb)), shm, s, (const float *)f.us,
-                           (const float *)f.vs, (const float *)f.ws, f.spec, f.tw, f.sc, c, pl, ppb, f.ld);
-    else
-        hipLaunchKernelGGL(k_xfwd<double>, dim3(pairs / ppb), dim3(fft_threads(pl, ppb)), shm, s, f.us, f.vs, f.ws,
-                           f.spec, f.tw, f.sc, c, pl, ppb, f.ld);
     li->name = "xfwd_div"; li->bytes = (c.mixed ? 2.5 : 4.0) * F(c);
 }
 
 void launch_ypass(const Fields &f, const Consts &c, const FftPlan &pl, const Tuning &tu, int inverse,
                   hipStream_t s, LaunchInfo *li)
 {
-    if (plan_regs(pl)) {
-        const int tkx = tu.v[KNOB_YTILE] ? tu.v[KNOB_YTILE] : rtile(pl), nh = c.n / 2 + 1;
-        const dim3 grid((nh + tkx - 1) / tkx, c.n), blk(tkx * (c.n / 8));
-        const size_t shm = sizeof(double2) * (size_t)tkx * c.n;
-        with_log2(reg_log2_cols(pl, tkx), [&](auto LC) {
-            constexpr int L = decltype(LC)::value, TK = L ? rtile_c(L) : 0;
+    const int tkx = tu.v[KNOB_YTILE] ? tu.v[KNOB_YTILE] : default_tile(pl), nh = c.n / 2 + 1;
+    const dim3 grid((nh + tkx - 1) / tkx, c.n);
+    const size_t shm = sizeof(double2) * (size_t)tkx * c.n;
+    if (col_regs(pl, tkx)) {
+        const dim3 blk(tkx * line_threads(c.n));
+        with_n<false>(col_n(pl, tkx), [&](auto NC) {
+            constexpr int N = decltype(NC)::value, TK = N ? rtile_n(N) : 0;
             if (inverse)
-                hipLaunchKernelGGL((k_ypass_r<1, L, TK>), grid, blk, shm, s, f.spec, f.tw, f.sc, pl, f.ld, tkx);
+                hipLaunchKernelGGL((k_ypass_r<1, N, TK>), grid, blk, shm, s, f.spec, f.tw, f.sc, pl, f.ld, tkx);
             else
-                hipLaunchKernelGGL((k_ypass_r<-1, L, TK>), grid, blk, shm, s, f.spec, f.tw, f.sc, pl, f.ld, tkx);
+                hipLaunchKernelGGL((k_ypass_r<-1, N, TK>), grid, blk, shm, s, f.spec, f.tw, f.sc, pl, f.ld, tkx);
         });
-        li->name = inverse ? "y_inv" : "y_fwd";
-        li->bytes = 2.0 * 16.0 * (double)nh * c.n * c.n;
-        return;
+    } else if (inverse) {
+        hipLaunchKernelGGL(k_ypass<1>, grid, dim3(fft_threads(pl, tkx)), shm, s, f.spec, f.tw, f.sc, pl, f.ld, tkx);
+    } else {
+        hipLaunchKernelGGL(k_ypass<-1>, grid, dim3(fft_threads(pl, tkx)), shm, s, f.spec, f.tw, f.sc, pl, f.ld, tkx);
     }
-    int tkx = tu.v[KNOB_YTILE] ? tu.v[KNOB_YTILE] : col_tile(pl);
-    int nh = c.n / 2 + 1;
-    dim3 grid((nh + tkx - 1) / tkx, c.n);
-    size_t shm = sizeof(double2) * (size_t)tkx * c.n;
-    dim3 blk(fft_threads(pl, tkx));
-    if (inverse)
-        hipLaunchKernelGGL(k_ypass<1>, grid, blk, shm, s, f.spec, f.tw, f.sc, pl, f.ld, tkx);
-    else
-        hipLaunchKernelGGL(k_ypass<-1>, grid, blk, shm, s, f.spec, f.tw, f.sc, pl, f.ld, tkx);
     li->name = inverse ? "y_inv" : "y_fwd";
     li->bytes = 2.0 * 16.0 * (double)nh * c.n * c.n;
 }
@@ -2884,24 +2985,19 @@ void launch_ypass(const Fields &f, const Consts &c, const FftPlan &pl, const Tun
 void launch_zpoisson(const Fields &f, const Consts &c, const FftPlan &pl, const Tuning &tu, hipStream_t s,
                      LaunchInfo *li)
 {
-    if (plan_regs(pl)) {
-        const int tkx = tu.v[KNOB_ZTILE] ? tu.v[KNOB_ZTILE] : rtile(pl), nh = c.n / 2 + 1;
-        const dim3 grid((nh + tkx - 1) / tkx, c.n), blk(tkx * (c.n / 8));
-        const size_t shm = sizeof(double2) * (size_t)tkx * c.n;
-        with_log2(reg_log2_cols(pl, tkx), [&](auto LC) {
-            constexpr int L = decltype(LC)::value, TK = L ? rtile_c(L) : 0;
-            hipLaunchKernelGGL((k_zpoisson_r<L, TK>), grid, blk, shm, s, f.spec, f.tw, f.ktab, f.sc, pl, f.ld, tkx);
+    const int tkx = tu.v[KNOB_ZTILE] ? tu.v[KNOB_ZTILE] : default_tile(pl), nh = c.n / 2 + 1;
+    const dim3 grid((nh + tkx - 1) / tkx, c.n);
+    const size_t shm = sizeof(double2) * (size_t)tkx * c.n;
+    if (col_regs(pl, tkx)) {
+        with_n<false>(col_n(pl, tkx), [&](auto NC) {
+            constexpr int N = decltype(NC)::value, TK = N ? rtile_n(N) : 0;
+            hipLaunchKernelGGL((k_zpoisson_r<N, TK>), grid, dim3(tkx * line_threads(c.n)), shm, s, f.spec, f.tw, f.ktab,
+                               f.sc, pl, f.ld, tkx);
         });
-        li->name = "z_poisson";
-        li->bytes = 2.0 * 16.0 * (double)nh * c.n * c.n;
-        return;
+    } else {
+        hipLaunchKernelGGL(k_zpoisson, grid, dim3(fft_threads(pl, tkx)), shm, s, f.spec, f.tw, f.ktab, f.sc, pl, f.ld,
+                           tkx);
     }
-    int tkx = tu.v[KNOB_ZTILE] ? tu.v[KNOB_ZTILE] : col_tile(pl);
-    int nh = c.n / 2 + 1;
-    dim3 grid((nh + tkx - 1) / tkx, c.n);
-    size_t shm = sizeof(double2) * (size_t)tkx * c.n;
-    hipLaunchKernelGGL(k_zpoisson, grid, dim3(fft_threads(pl, tkx)), shm, s, f.spec, f.tw, f.ktab, f.sc, pl,
-                       f.ld, tkx);
     li->name = "z_poisson";
     li->bytes = 2.0 * 16.0 * (double)nh * c.n * c.n;
 }
@@ -2909,21 +3005,18 @@ void launch_zpoisson(const Fields &f, const Consts &c, const FftPlan &pl, const 
 void launch_xinv(const Fields &f, const Consts &c, const FftPlan &pl, const Tuning &tu, hipStream_t s,
                  LaunchInfo *li)
 {
-    if (plan_regs(pl)) {
-        const int ppb = tu.v[KNOB_XIPAIRS] ? tu.v[KNOB_XIPAIRS] : rpairs(pl), pairs = c.n * c.n / 2;
+    const int ppb = tu.v[KNOB_XIPAIRS] ? tu.v[KNOB_XIPAIRS] : default_pairs(pl), pairs = c.n * c.n / 2;
+    if (x_regs(pl)) {
         const size_t shm = sizeof(double2) * (size_t)ppb * rline_stride(c.n);
-        with_log2(reg_log2(pl), [&](auto LC) {
-            hipLaunchKernelGGL((k_xinv_r<decltype(LC)::value>), dim3(pairs / ppb), dim3(ppb * (c.n / 8)), shm, s,
-                               f.spec, f.p, f.tw, f.sc, pl, ppb, f.ld);
+        with_n<false>(c.n, [&](auto NC) {
+            hipLaunchKernelGGL((k_xinv_r<decltype(NC)::value>), dim3(pairs / ppb), dim3(ppb * line_threads(c.n)), shm,
+                               s, f.spec, f.p, f.tw, f.sc, pl, ppb, f.ld);
         });
-        li->name = "x_inv"; li->bytes = 16.0 * (double)(c.n / 2 + 1) * c.n * c.n + F(c);
-        return;
+    } else {
+        const size_t shm = sizeof(double2) * (size_t)ppb * (c.n + 1);
+        hipLaunchKernelGGL(k_xinv, dim3(pairs / ppb), dim3(fft_threads(pl, ppb)), shm, s, f.spec, f.p, f.tw, f.sc, pl,
+                           ppb, f.ld);
     }
-    int ppb = tu.v[KNOB_XIPAIRS] ? tu.v[KNOB_XIPAIRS] : pairs_per_block(pl);
-    int pairs = c.n * c.n / 2;
-    size_t shm = sizeof(double2) * (size_t)ppb * (c.n + 1);
-    hipLaunchKernelGGL(k_xinv, dim3(pairs / ppb), dim3(fft_threads(pl, ppb)), shm, s, f.spec, f.p, f.tw, f.sc, pl,
-                       ppb, f.ld);
     li->name = "x_inv"; li->bytes = 16.0 * (double)(c.n / 2 + 1) * c.n * c.n + F(c);
 }
 
@@ -3030,59 +3123,53 @@ void launch_gang_step(const GangBox *g, int nbox, unsigned euler, const GangLaun
         const int nb = z.cnt, n = z.n, nh = n / 2 + 1, pairs = n * n / 2, ld = z.ld;
         const FftPlan &pl = z.plan;
         const Tuning &tu = z.tune;
-        if (plan_regs(pl)) {
-            const int xp = tu.v[KNOB_XPAIRS] ? tu.v[KNOB_XPAIRS] : rpairs(pl);
-            const int xip = tu.v[KNOB_XIPAIRS] ? tu.v[KNOB_XIPAIRS] : rpairs(pl);
-            const int ty = tu.v[KNOB_YTILE] ? tu.v[KNOB_YTILE] : rtile(pl);
-            const int tz = tu.v[KNOB_ZTILE] ? tu.v[KNOB_ZTILE] : rtile(pl);
-            const size_t shx = sizeof(double2) * (size_t)xp * rline_stride(n);
-            with_log2_gang(reg_log2(pl), [&](auto LC) {
-                constexpr int L = decltype(LC)::value;
+        const int xp = tu.v[KNOB_XPAIRS] ? tu.v[KNOB_XPAIRS] : default_pairs(pl, true);
+        const int xip = tu.v[KNOB_XIPAIRS] ? tu.v[KNOB_XIPAIRS] : default_pairs(pl, true);
+        const int ty = tu.v[KNOB_YTILE] ? tu.v[KNOB_YTILE] : default_tile(pl, true);
+        const int tz = tu.v[KNOB_ZTILE] ? tu.v[KNOB_ZTILE] : default_tile(pl, true);
+        const bool xr = x_regs(pl, true), yr = col_regs(pl, ty, true), zr = col_regs(pl, tz, true);
+        const size_t line = sizeof(double2) * (size_t)(xr ? rline_stride(n) : n + 1);
+        const dim3 gx(pairs / xp, nb), gxi(pairs / xip, nb), gy((nh + ty - 1) / ty, n, nb), gz((nh + tz - 1) / tz, n, nb);
+        const size_t shy = sizeof(double2) * (size_t)ty * n, shz = sizeof(double2) * (size_t)tz * n;
+        const int lt = line_threads(n);
+        if (xr) {
+            with_n<true>(n, [&](auto NC) {
+                constexpr int N = decltype(NC)::value;
                 if (gl.mixed)
-                    hipLaunchKernelGGL((kg_xfwd<float, true, L>), dim3(pairs / xp, nb), dim3(xp * (n / 8)), shx, s, gs,
-                                       pl, xp, ld);
+                    hipLaunchKernelGGL((kg_xfwd<float, true, N>), gx, dim3(xp * lt), xp * line, s, gs, pl, xp, ld);
                 else
-                    hipLaunchKernelGGL((kg_xfwd<double, true, L>), dim3(pairs / xp, nb), dim3(xp * (n / 8)), shx, s,
-                                       gs, pl, xp, ld);
+                    hipLaunchKernelGGL((kg_xfwd<double, true, N>), gx, dim3(xp * lt), xp * line, s, gs, pl, xp, ld);
             });
-            const dim3 gy((nh + ty - 1) / ty, n, nb), gz((nh + tz - 1) / tz, n, nb);
-            const size_t shy = sizeof(double2) * (size_t)ty * n, shz = sizeof(double2) * (size_t)tz * n;
-            with_log2_gang(reg_log2_cols(pl, ty), [&](auto LC) {
-                hipLaunchKernelGGL((kg_ypass<-1, true, decltype(LC)::value>), gy, dim3(ty * (n / 8)), shy, s, gs, pl,
-                                   ld, ty);
-            });
-            with_log2_gang(reg_log2_cols(pl, tz), [&](auto LC) {
-                hipLaunchKernelGGL((kg_zpoisson<true, decltype(LC)::value>), gz, dim3(tz * (n / 8)), shz, s, gs, pl,
-                                   ld, tz);
-            });
-            with_log2_gang(reg_log2_cols(pl, ty), [&](auto LC) {
-                hipLaunchKernelGGL((kg_ypass<1, true, decltype(LC)::value>), gy, dim3(ty * (n / 8)), shy, s, gs, pl,
-                                   ld, ty);
-            });
-            with_log2_gang(reg_log2(pl), [&](auto LC) {
-                hipLaunchKernelGGL((kg_xinv<true, decltype(LC)::value>), dim3(pairs / xip, nb), dim3(xip * (n / 8)),
-                                   sizeof(double2) * (size_t)xip * rline_stride(n), s, gs, pl, xip, ld);
-            });
+        } else if (gl.mixed) {
+            hipLaunchKernelGGL((kg_xfwd<float, false, 0>), gx, dim3(fft_threads(pl, xp)), xp * line, s, gs, pl, xp, ld);
         } else {
-            const int xp = tu.v[KNOB_XPAIRS] ? tu.v[KNOB_XPAIRS] : pairs_per_block(pl);
-            const int xip = tu.v[KNOB_XIPAIRS] ? tu.v[KNOB_XIPAIRS] : pairs_per_block(pl);
-            const int ty = tu.v[KNOB_YTILE] ? tu.v[KNOB_YTILE] : col_tile(pl);
-            const int tz = tu.v[KNOB_ZTILE] ? tu.v[KNOB_ZTILE] : col_tile(pl);
-            const size_t shx = sizeof(double2) * (size_t)xp * (n + 1);
-            if (gl.mixed)
-                hipLaunchKernelGGL((kg_xfwd<float, false, 0>), dim3(pairs / xp, nb), dim3(fft_threads(pl, xp)), shx,
-                                   s, gs, pl, xp, ld);
-            else
-                hipLaunchKernelGGL((kg_xfwd<double, false, 0>), dim3(pairs / xp, nb), dim3(fft_threads(pl, xp)), shx,
-                                   s, gs, pl, xp, ld);
-            const dim3 gy((nh + ty - 1) / ty, n, nb), gz((nh + tz - 1) / tz, n, nb);
-            const size_t shy = sizeof(double2) * (size_t)ty * n, shz = sizeof(double2) * (size_t)tz * n;
-            hipLaunchKernelGGL((kg_ypass<-1, false, 0>), gy, dim3(fft_threads(pl, ty)), shy, s, gs, pl, ld, ty);
-            hipLaunchKernelGGL((kg_zpoisson<false, 0>), gz, dim3(fft_threads(pl, tz)), shz, s, gs, pl, ld, tz);
-            hipLaunchKernelGGL((kg_ypass<1, false, 0>), gy, dim3(fft_threads(pl, ty)), shy, s, gs, pl, ld, ty);
-            hipLaunchKernelGGL((kg_xinv<false, 0>), dim3(pairs / xip, nb), dim3(fft_threads(pl, xip)),
-                               sizeof(double2) * (size_t)xip * (n + 1), s, gs, pl, xip, ld);
+            hipLaunchKernelGGL((kg_xfwd<double, false, 0>), gx, dim3(fft_threads(pl, xp)), xp * line, s, gs, pl, xp, ld);
         }
+        auto ypass = [&](auto SGC) {
+            constexpr int SG = decltype(SGC)::value;
+            if (yr)
+                with_n<true>(col_n(pl, ty), [&](auto NC) {
+                    hipLaunchKernelGGL((kg_ypass<SG, true, decltype(NC)::value>), gy, dim3(ty * lt), shy, s, gs, pl, ld,
+                                       ty);
+                });
+            else
+                hipLaunchKernelGGL((kg_ypass<SG, false, 0>), gy, dim3(fft_threads(pl, ty)), shy, s, gs, pl, ld, ty);
+        };
+        ypass(std::integral_constant<int, -1>());
+        if (zr)
+            with_n<true>(col_n(pl, tz), [&](auto NC) {
+                hipLaunchKernelGGL((kg_zpoisson<true, decltype(NC)::value>), gz, dim3(tz * lt), shz, s, gs, pl, ld, tz);
+            });
+        else
+            hipLaunchKernelGGL((kg_zpoisson<false, 0>), gz, dim3(fft_threads(pl, tz)), shz, s, gs, pl, ld, tz);
+        ypass(std::integral_constant<int, 1>());
+        if (xr)
+            with_n<true>(n, [&](auto NC) {
+                hipLaunchKernelGGL((kg_xinv<true, decltype(NC)::value>), gxi, dim3(xip * lt), xip * line, s, gs, pl, xip,
+                                   ld);
+            });
+        else
+            hipLaunchKernelGGL((kg_xinv<false, 0>), gxi, dim3(fft_threads(pl, xip)), xip * line, s, gs, pl, xip, ld);
         if (fork && q > 0) (void)hipEventRecord(fs->join[q - 1], s);
     }
     s = s0;
@@ -3106,17 +3193,12 @@ void launch_ic_potential(const Fields &f, const Consts &c, const FftPlan &pl, co
     const unsigned g = nblocks(total, BLK) < 65536 ? nblocks(total, BLK) : 65536;
     hipLaunchKernelGGL(k_ic_spectrum, dim3(g), dim3(BLK), 0, s, f.spec, c.n, f.ld, comp, seedmix, kp, kmax);
     const int nh = c.n / 2 + 1;
-    if (plan_regs(pl)) {
-        const int tkx = tu.v[KNOB_ZTILE] ? tu.v[KNOB_ZTILE] : rtile(pl);
-        const size_t shm = sizeof(double2) * (size_t)tkx * c.n;
-        hipLaunchKernelGGL(k_zinv_r, dim3((nh + tkx - 1) / tkx, c.n), dim3(tkx * (c.n / 8)), shm, s, f.spec, f.tw,
-                           f.ktab, f.sc, pl, f.ld, tkx);
-    } else {
-        const int tkx = tu.v[KNOB_ZTILE] ? tu.v[KNOB_ZTILE] : col_tile(pl);
-        const size_t shm = sizeof(double2) * (size_t)tkx * c.n;
-        hipLaunchKernelGGL(k_zinv, dim3((nh + tkx - 1) / tkx, c.n), dim3(fft_threads(pl, tkx)), shm, s, f.spec,
-                           f.tw, f.ktab, f.sc, pl, f.ld, tkx);
-    }
+    const bool regs = pow2_regs(pl);
+    const int tkx = tu.v[KNOB_ZTILE] ? tu.v[KNOB_ZTILE] : regs ? rtile_n(c.n) : col_tile(pl);
+    const size_t shm = sizeof(double2) * (size_t)tkx * c.n;
+    hipLaunchKernelGGL(regs ? k_zinv_r : k_zinv, dim3((nh + tkx - 1) / tkx, c.n),
+                       dim3(regs ? tkx * line_threads(c.n) : fft_threads(pl, tkx)), shm, s, f.spec, f.tw, f.ktab, f.sc, pl,
+                       f.ld, tkx);
     LaunchInfo li;
     launch_ypass(f, c, pl, tu, 1, s, &li);
     Fields g2 = f;

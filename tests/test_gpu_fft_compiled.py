@@ -83,3 +83,32 @@ def test_1024_compiled_equals_generic():
     assert g0 == g1
     assert d0 == d1
     assert np.array_equal(p0, p1)
+
+
+@pytest.mark.parametrize("n", [16, 32, 36, 48, 54, 64, 72, 96, 108, 144, 162, 192, 216, 256, 288, 324, 384, 432,
+                               486])
+def test_compiled_lengths_bit_identical_to_oracle(n):
+    """Every compiled length up to 486 (with a factor 3: n/8, n/6 or n/3 threads
+    per line, stages of whole and of partial rounds of butterflies) against the
+    oracle, and against the column passes' other form (2-column tiles) and
+    the x passes with one pair per block."""
+    rng = np.random.default_rng(n)
+    u, v, w = (np.asfortranarray(rng.standard_normal((n, n, n))) for _ in range(3))
+    dx = 2 * np.pi / (n - 1)
+    kw = dict(nx=n, dt=0.01 * dx, mu=0.004, f1=1.0, f2=0.5, f3=0.25, phiflag=0, inflow=1)
+    o = orc.Oracle(**kw)
+    out = []
+    for shapes in ({}, OTHER_SHAPES):
+        with Solver(**kw) as s:
+            s.set_tuning(**shapes)
+            for f, a in ((1, u), (2, v), (3, w)):
+                s.set_field(f, a)
+            s.step(2)
+            out.append([s.get_field(f) for f in (1, 2, 3, 4)])
+    for f, a in ((1, u), (2, v), (3, w)):
+        o.set_field(f, a)
+    o.step(2)
+    for f, a, b in zip((1, 2, 3, 4), *out):
+        assert np.array_equal(a, o.get_field(f)), f
+        assert np.array_equal(a, b), f
+    o.close()
