@@ -90,7 +90,7 @@ struct Fields {
     double *mtab;                // log/expm1 table (devmath.h layout)
     Scalars *sc;
     double *diag;                // 3 diagnostic sums (kinetic, strain, phase)
-    Scalars *mirror = nullptr;   // host-mapped copy of *sc as the last step left it
+    Scalars *mirror = nullptr;   // host-mapped copy of *sc as the last step of a call left it
     EnsSlot *slot = nullptr;     // host-mapped progress record (ensemble boxes only)
     int ld;                      // spectrum leading dimension (>= n/2+1)
 };
@@ -155,13 +155,23 @@ void launch_zpoisson(const Fields &f, const Consts &c, const FftPlan &pl, const 
 void launch_xinv(const Fields &f, const Consts &c, const FftPlan &pl, const Tuning &tu, hipStream_t s,
                  LaunchInfo *li);
 void launch_project(const Fields &f, const Consts &c, hipStream_t s, LaunchInfo *li);
+// Whether launch_project has formed the plane sums of this box, which launch_reduce otherwise forms.
+bool project_sums_planes(const Consts &c);
 void launch_reduce(const Fields &f, const Consts &c, hipStream_t s, LaunchInfo *li);
-void launch_finalize(const Fields &f, const Consts &c, hipStream_t s, LaunchInfo *li);
+// publish: write the scalars to f.mirror too (the last step of a call).
+void launch_finalize(const Fields &f, const Consts &c, bool publish, hipStream_t s, LaunchInfo *li);
+// The x and y passes of small boxes, plane by plane, in place of launch_xfwd and
+// the forward launch_ypass, and of the inverse pair.
+bool plane_passes(const Consts &c, const FftPlan &pl, const Tuning &tu);
+bool plane_fwd_alone(const Consts &c);   // the forward pair too, in a box stepped alone
+void launch_plane_fwd(const Fields &f, const Consts &c, hipStream_t s, LaunchInfo *li);
+void launch_plane_inv(const Fields &f, const Consts &c, hipStream_t s, LaunchInfo *li);
 // The launches of a gang step: the grid of each shared pass and, per size n,
 // its boxes [off, off + cnt) with the FFT plan, spectrum row length and
 // launch shapes of that size (the FFT passes take one launch per size).
 struct GangSize {
     int off, cnt, n, ld;
+    bool planes;                         // plane_passes
     FftPlan plan;
     Tuning tune;
 };
@@ -186,8 +196,9 @@ struct GangStreams {
 // One step of the gang (descriptors g in device memory, laid out by
 // gang_layout; bit b of euler: box b takes its Euler first step) on stream s;
 // with fs holding a side stream per size beyond the first, the sizes' FFT
-// passes run on their own streams between a fork and a join.
-void launch_gang_step(const GangBox *g, int nbox, unsigned euler, const GangLaunch &gl, hipStream_t s,
+// passes run on their own streams between a fork and a join.  publish: each
+// box's scalars to its mirror too.
+void launch_gang_step(const GangBox *g, int nbox, unsigned euler, bool publish, const GangLaunch &gl, hipStream_t s,
                       const GangStreams *fs = nullptr);
 void launch_debug_math(int op, size_t count, const double *x, double *y, const double *mtab, hipStream_t s);
 // Drop counting: label the phi >= 0.5 cells (26-connected, periodic) by the

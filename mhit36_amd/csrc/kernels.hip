@@ -17,6 +17,10 @@ namespace mhit {
 
 constexpr int BLK = 256;
 
+// A kernel of a halted run writes nothing.  The FFT passes, the projection and
+// the sums read the flag at the start and test it just before the first store,
+// so that no load waits for it: 0.2-0.4 us of a 64^3 box's 4 to 7 us kernels.
+// (The marching passes gain nothing by it and their main loops compile worse.)
 __device__ __forceinline__ bool halted(const Scalars *sc) { return sc->halted != 0; }
 
 static inline unsigned nblocks(size_t work, int blk) { return (unsigned)((work + blk - 1) / blk); }
@@ -1450,13 +1454,86 @@ __device__ __forceinline__ int mirror_lane(int tj, int LM)
     return (int)(threadIdx.x & 63) - tj + ((LM - tj) & (LM - 1));
 }
 
+// Poisson right-hand side (main.f90:715-750) at points (i, j, k) and (i, j+1, k).
+template <typename T>
+__device__ __forceinline__ double2 poisson_rhs(const T *__restrict__ us, const T *__restrict__ vs,
+                                               const T *__restrict__ ws, int i, int j, int k, int kp, int n, double cdiv,
+                                               int fp32)
+{
+    const int ip = i + 1 == n ? 0 : i + 1;
+    double rr[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        int jj = j + h;
+        int jp = jj + 1 == n ? 0 : jj + 1;
+        size_t id = IDX(i, jj, k);
+        double r = cdiv * ((double)us[IDX(ip, jj, k)] - (double)us[id]);
+        r = r + cdiv * ((double)vs[IDX(i, jp, k)] - (double)vs[id]);
+        r = r + cdiv * ((double)ws[IDX(i, jj, kp)] - (double)ws[id]);
+        if (fp32) r = (double)(float)r;
+        rr[h] = r;
+    }
+    return make_double2(rr[0], rr[1]);
+}
+
+// The spectrum of two real lines transformed as one, a thread's 8 positions of
+// it in v, split into the lines' half spectra (q = 0 .. n/2); z[n-q] comes from
+// the mirror lane.  put(line, q, re, im).
+template <typename Put>
+__device__ __forceinline__ void split_pair(const double2 (&v)[8], int tj, int LM, int half, Put &&put)
+{
+    const int src = mirror_lane(tj, LM);
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+        const int q = tj + m * LM;
+        double2 zm = lane_get2(v[7 - m], src);
+        if (tj == 0) zm = v[(8 - m) & 7];
+        const double a = v[m].x, b = v[m].y, cc = zm.x, d = zm.y;
+        put(0, q, (a + cc) * 0.5, (b - d) * 0.5);
+        put(1, q, (b + d) * 0.5, (cc - a) * 0.5);
+    }
+    if (tj == 0) {                        // q = n/2, its own mirror
+        const double a = v[4].x, b = v[4].y, cc = v[4].x, d = v[4].y;
+        put(0, half, (a + cc) * 0.5, (b - d) * 0.5);
+        put(1, half, (b + d) * 0.5, (cc - a) * 0.5);
+    }
+}
+
+// The reverse: a thread's 8 positions of the joint spectrum of the half spectra
+// s1, s2.  Each value is loaded once: positions below n/2 directly, their
+// mirrors (slots 4..7) from the mirror lane by a permute.
+__device__ __forceinline__ void join_pair(const double2 *s1, const double2 *s2, double2 (&v)[8], int tj, int LM, int half)
+{
+    double2 A[4], B[4];
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+        A[m] = s1[tj + m * LM];
+        B[m] = s2[tj + m * LM];
+    }
+    const int src = mirror_lane(tj, LM);
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+        const double2 a = A[m], b = B[m];
+        v[m] = tj + m * LM == 0 ? make_double2(a.x, b.x) : make_double2(a.x - b.y, a.y + b.x);
+    }
+#pragma unroll
+    for (int m = 4; m < 8; m++) {
+        double2 a = lane_get2(A[7 - m], src), b = lane_get2(B[7 - m], src);
+        if (tj == 0) {
+            if (m == 4) { a = s1[half]; b = s2[half]; }
+            else { a = A[8 - m]; b = B[8 - m]; }
+        }
+        v[m] = (tj == 0 && m == 4) ? make_double2(a.x, b.x) : make_double2(a.x + b.y, b.x - a.y);
+    }
+}
+
 template <typename T, int N = 0>
 __device__ __forceinline__ void k_xfwd_r_body(uint3 blk,
     const T *__restrict__ us, const T *__restrict__ vs, const T *__restrict__ ws,
     double2 *__restrict__ spec, const double2 *__restrict__ tw, const Scalars *__restrict__ sc,
     Consts c, FftPlan pl, int ppb, int ld)
 {
-    if (halted(sc)) return;
+    const bool stop = halted(sc);
     extern __shared__ double2 lds[];
     const int n = N ? N : c.n, half = n / 2, nh = n / 2 + 1, LM = N ? line_threads(N) : n / 8;
     const int lstride = rline_stride(n);
@@ -1465,22 +1542,7 @@ __device__ __forceinline__ void k_xfwd_r_body(uint3 blk,
     const int k = pair / half, j = 2 * (pair - k * half);
     const int kp = k + 1 == n ? 0 : k + 1;
     const double cdiv = c.rho * c.dxi / c.dt;
-    auto rhs = [&](int i) {                     // Poisson right-hand side at points (i, j, k) and (i, j+1, k)
-        const int ip = i + 1 == n ? 0 : i + 1;
-        double rr[2];
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            int jj = j + h;
-            int jp = jj + 1 == n ? 0 : jj + 1;
-            size_t id = IDX(i, jj, k);
-            double r = cdiv * ((double)us[IDX(ip, jj, k)] - (double)us[id]);
-            r = r + cdiv * ((double)vs[IDX(i, jp, k)] - (double)vs[id]);
-            r = r + cdiv * ((double)ws[IDX(i, jj, kp)] - (double)ws[id]);
-            if (c.fp32_rhs) r = (double)(float)r;
-            rr[h] = r;
-        }
-        return make_double2(rr[0], rr[1]);
-    };
+    auto rhs = [&](int i) { return poisson_rhs(us, vs, ws, i, j, k, kp, n, cdiv, c.fp32_rhs); };
     double2 v[8];
     if constexpr (N > 0 && !is_pow2(N)) {
         fft_threes<-1, true, N, false>(tj, pl_, lds, lstride, 1, tw, rhs, [&](int p, double2 z) {
@@ -1491,31 +1553,17 @@ __device__ __forceinline__ void k_xfwd_r_body(uint3 blk,
 #pragma unroll
         for (int m = 0; m < 8; m++) v[m] = rhs(tj + m * LM);
         fft_lines<-1, true, N>(v, tj, pl_, lds, lstride, 1, pl, tw);
+        if (stop) return;
         if (LM <= 64) {
-            // split z into the two real lines' half spectra (q = 0 .. n/2); z[n-q]
-            // from the mirror lane instead of a round trip through LDS
-            const int src = mirror_lane(tj, LM);
             double2 *r1 = spec + spec_row(k, j, n, ld), *r2 = spec + spec_row(k, j + 1, n, ld);
-#pragma unroll
-            for (int m = 0; m < 4; m++) {
-                const int q = tj + m * LM;
-                double2 zm = lane_get2(v[7 - m], src);
-                if (tj == 0) zm = v[(8 - m) & 7];
-                const double a = v[m].x, b = v[m].y, cc = zm.x, d = zm.y;
-                nt_store2(&r1[q], (a + cc) * 0.5, (b - d) * 0.5);
-                nt_store2(&r2[q], (b + d) * 0.5, (cc - a) * 0.5);
-            }
-            if (tj == 0) {                        // q = n/2, its own mirror
-                const double a = v[4].x, b = v[4].y, cc = v[4].x, d = v[4].y;
-                nt_store2(&r1[half], (a + cc) * 0.5, (b - d) * 0.5);
-                nt_store2(&r2[half], (b + d) * 0.5, (cc - a) * 0.5);
-            }
+            split_pair(v, tj, LM, half, [&](int h, int q, double re, double im) { nt_store2(&(h ? r2 : r1)[q], re, im); });
             return;
         }
 #pragma unroll
         for (int m = 0; m < 8; m++) lds[rlds<true>(pl_, tj + m * LM, lstride, 1)] = v[m];
         __syncthreads();
     }
+    if (stop) return;
     for (int e = t; e < ppb * nh; e += blockDim.x) {
         int pq = e / nh, q = e - pq * nh;
         int pr = blk.x * ppb + pq;
@@ -1547,7 +1595,7 @@ __device__ __forceinline__ void k_ypass_r_body(uint3 blk, double2 *__restrict__ 
                                                              const Scalars *__restrict__ sc, FftPlan pl, int ld,
                                                              int tkx_)
 {
-    if (halted(sc)) return;
+    const bool stop = halted(sc);
     extern __shared__ double2 lds[];
     const int n = N ? N : pl.n, nh = n / 2 + 1, LM = n / 8, tkx = TK ? TK : tkx_;
     const int q0 = blk.x * tkx, k = blk.y;
@@ -1558,14 +1606,14 @@ __device__ __forceinline__ void k_ypass_r_body(uint3 blk, double2 *__restrict__ 
         fft_threes<SG, false, N, false>(
             tj, line, lds, 1, tkx, tw,
             [&](int p) { return ok ? base[(size_t)p * ld] : make_double2(0.0, 0.0); },
-            [&](int p, double2 z) { if (ok) nt_store2(&base[(size_t)p * ld], z.x, z.y); });
+            [&](int p, double2 z) { if (ok && !stop) nt_store2(&base[(size_t)p * ld], z.x, z.y); });
         return;
     }
     double2 v[8];
 #pragma unroll
     for (int m = 0; m < 8; m++) v[m] = ok ? base[(size_t)(tj + m * LM) * ld] : make_double2(0.0, 0.0);
     if constexpr (N == 0 || is_pow2(N)) fft_lines<SG, false, N>(v, tj, line, lds, 1, tkx, pl, tw);
-    if (ok) {
+    if (ok && !stop) {
 #pragma unroll
         for (int m = 0; m < 8; m++) nt_store2(&base[(size_t)(tj + m * LM) * ld], v[m].x, v[m].y);
     }
@@ -1588,7 +1636,7 @@ __device__ __forceinline__ void k_zpoisson_r_body(uint3 blk, double2 *__restrict
                                                                 const Scalars *__restrict__ sc, FftPlan pl, int ld,
                                                                 int tkx_)
 {
-    if (halted(sc)) return;
+    const bool stop = halted(sc);
     extern __shared__ double2 lds[];
     const int n = N ? N : pl.n, nh = n / 2 + 1, LM = n / 8, tkx = TK ? TK : tkx_;
     const int q0 = blk.x * tkx, j = blk.y;
@@ -1615,7 +1663,7 @@ __device__ __forceinline__ void k_zpoisson_r_body(uint3 blk, double2 *__restrict
         __syncthreads();
         fft_threes<1, false, N, true>(
             tj, line, lds, 1, tkx, tw, [&](int p) { return lds[rlds<false>(line, p, 1, tkx)]; },
-            [&](int p, double2 z) { if (ok) nt_store2(&base[(size_t)p * rs], z.x, z.y); });
+            [&](int p, double2 z) { if (ok && !stop) nt_store2(&base[(size_t)p * rs], z.x, z.y); });
     } else {
         double2 v[8];
 #pragma unroll
@@ -1626,7 +1674,7 @@ __device__ __forceinline__ void k_zpoisson_r_body(uint3 blk, double2 *__restrict
             for (int m = 0; m < 8; m++) v[m] = solve(tj + m * LM, v[m]);
         }
         fft_lines<1, false, N>(v, tj, line, lds, 1, tkx, pl, tw);
-        if (ok) {
+        if (ok && !stop) {
 #pragma unroll
             for (int m = 0; m < 8; m++) nt_store2(&base[(size_t)(tj + m * LM) * rs], v[m].x, v[m].y);
         }
@@ -1669,7 +1717,7 @@ __device__ __forceinline__ void k_xinv_r_body(uint3 blk, const double2 *__restri
                                                             const Scalars *__restrict__ sc, FftPlan pl, int ppb,
                                                             int ld)
 {
-    if (halted(sc)) return;
+    const bool stop = halted(sc);
     extern __shared__ double2 lds[];
     const int n = N ? N : pl.n, half = n / 2, LM = N ? line_threads(N) : n / 8;
     const int lstride = rline_stride(n);
@@ -1692,6 +1740,7 @@ __device__ __forceinline__ void k_xinv_r_body(uint3 blk, const double2 *__restri
         fft_threes<1, true, N, true>(
             tj, pl_, lds, lstride, 1, tw, [&](int q) { return lds[rlds<true>(pl_, q, lstride, 1)]; },
             [&](int i, double2 z) {
+                if (stop) return;
                 __builtin_nontemporal_store(z.x, &p[IDX(i, j, k)]);
                 __builtin_nontemporal_store(z.y, &p[IDX(i, j + 1, k)]);
             });
@@ -1699,29 +1748,7 @@ __device__ __forceinline__ void k_xinv_r_body(uint3 blk, const double2 *__restri
     }
     double2 v[8];
     if (LM <= 64) {
-        // Each spectrum value is loaded once: positions below n/2 directly,
-        // their mirrors (slots 4..7) from the mirror lane by a permute.
-        double2 A[4], B[4];
-#pragma unroll
-        for (int m = 0; m < 4; m++) {
-            A[m] = s1[tj + m * LM];
-            B[m] = s2[tj + m * LM];
-        }
-        const int src = mirror_lane(tj, LM);
-#pragma unroll
-        for (int m = 0; m < 4; m++) {
-            const double2 a = A[m], b = B[m];
-            v[m] = tj + m * LM == 0 ? make_double2(a.x, b.x) : make_double2(a.x - b.y, a.y + b.x);
-        }
-#pragma unroll
-        for (int m = 4; m < 8; m++) {
-            double2 a = lane_get2(A[7 - m], src), b = lane_get2(B[7 - m], src);
-            if (tj == 0) {
-                if (m == 4) { a = s1[half]; b = s2[half]; }
-                else { a = A[8 - m]; b = B[8 - m]; }
-            }
-            v[m] = (tj == 0 && m == 4) ? make_double2(a.x, b.x) : make_double2(a.x + b.y, b.x - a.y);
-        }
+        join_pair(s1, s2, v, tj, LM, half);
     } else {
 #pragma unroll
         for (int m = 0; m < 8; m++) {
@@ -1741,6 +1768,7 @@ __device__ __forceinline__ void k_xinv_r_body(uint3 blk, const double2 *__restri
         }
     }
     if constexpr (N == 0 || is_pow2(N)) fft_lines<1, true, N>(v, tj, pl_, lds, lstride, 1, pl, tw);
+    if (stop) return;
 #pragma unroll
     for (int m = 0; m < 8; m++) {
         const int i = tj + m * LM;
@@ -1758,6 +1786,156 @@ __global__ void __launch_bounds__(x_threads(N)) k_xinv_r(const double2 *__restri
     // last pairs first: the y inverse pass wrote the highest planes last, and
     // some of them are still in the memory-side cache
     k_xinv_r_body<N>(make_uint3(gridDim.x - 1 - blockIdx.x, blockIdx.y, blockIdx.z), spec, p, tw, sc, pl, ppb, ld);
+}
+
+
+// ---------------------------------------------------------------------------
+// Small boxes (n <= PLANE_MAX): the x and y passes of a plane in one block, the
+// plane's half spectrum (n rows of n/2+1) in LDS between them.  These passes are
+// bound by the latency of a launch and a memory round trip each, not by what
+// they move (times at plane_fwd_alone).  Arithmetic and its order are those of
+// the separate passes.  Threads past the last line repeat the last line's work
+// and store nothing to memory.
+// ---------------------------------------------------------------------------
+constexpr int PLANE_MAX = 64;
+__host__ __device__ constexpr int plane_threads(int n) { return ((n / 2 + 1) * line_threads(n) + 63) / 64 * 64; }
+__host__ __device__ constexpr size_t plane_lds(int n)     // x lines in exchange order, then the spectrum rows
+{
+    return sizeof(double2) * ((size_t)(n / 2) * rline_stride(n) + (size_t)n * (n / 2 + 1));
+}
+
+template <typename T, int N>
+__device__ __forceinline__ void k_plane_fwd_body(int k, const T *__restrict__ us, const T *__restrict__ vs,
+                                                 const T *__restrict__ ws, double2 *__restrict__ spec,
+                                                 const double2 *__restrict__ tw, const Scalars *__restrict__ sc,
+                                                 const Consts &c, int ld)
+{
+    const bool stop = halted(sc);
+    extern __shared__ double2 lds[];
+    constexpr int n = N, half = N / 2, nh = half + 1, LM = line_threads(N), lstride = rline_stride(N);
+    double2 *xl = lds, *rows = lds + half * lstride;
+    const int t = threadIdx.x;
+    {
+        const int pl_ = min(t / LM, half - 1), tj = t % LM, j = 2 * pl_;
+        const int kp = k + 1 == n ? 0 : k + 1;
+        const double cdiv = c.rho * c.dxi / c.dt;
+        auto rhs = [&](int i) { return poisson_rhs(us, vs, ws, i, j, k, kp, n, cdiv, c.fp32_rhs); };
+        if constexpr (is_pow2(N)) {
+            double2 v[8];
+#pragma unroll
+            for (int m = 0; m < 8; m++) v[m] = rhs(tj + m * LM);
+            fft_regs_c<-1, true, N>(v, tj, pl_, xl, lstride, 1, tw);
+            split_pair(v, tj, LM, half, [&](int h, int q, double re, double im) {
+                rows[(j + h) * nh + q] = make_double2(re, im);
+            });
+        } else {
+            fft_threes<-1, true, N, false>(tj, pl_, xl, lstride, 1, tw, rhs, [&](int p, double2 z) {
+                xl[rlds<true>(pl_, p, lstride, 1)] = z;
+            });
+            __syncthreads();
+            for (int e = t; e < half * nh; e += blockDim.x) {
+                const int pq = e / nh, q = e - pq * nh, mq = q == 0 ? 0 : n - q;
+                const double2 zq = xl[rlds<true>(pq, q, lstride, 1)], zm = xl[rlds<true>(pq, mq, lstride, 1)];
+                const double a = zq.x, b = zq.y, cc = zm.x, d = zm.y;
+                rows[2 * pq * nh + q] = make_double2((a + cc) * 0.5, (b - d) * 0.5);
+                rows[(2 * pq + 1) * nh + q] = make_double2((b + d) * 0.5, (cc - a) * 0.5);
+            }
+        }
+    }
+    __syncthreads();
+    const int line = t % nh, tj = min(t / nh, LM - 1);
+    const bool ok = t < nh * LM && !stop;
+    double2 *out = spec + spec_row(k, 0, n, ld) + line;
+    if constexpr (is_pow2(N)) {
+        double2 v[8];
+#pragma unroll
+        for (int m = 0; m < 8; m++) v[m] = rows[(tj + m * LM) * nh + line];
+        __syncthreads();
+        fft_regs_c<-1, false, N>(v, tj, line, rows, 1, nh, tw);
+        if (ok) {
+#pragma unroll
+            for (int m = 0; m < 8; m++) nt_store2(&out[(size_t)(tj + m * LM) * ld], v[m].x, v[m].y);
+        }
+    } else {
+        fft_threes<-1, false, N, true>(
+            tj, line, rows, 1, nh, tw, [&](int p) { return rows[p * nh + line]; },
+            [&](int p, double2 z) { if (ok) nt_store2(&out[(size_t)p * ld], z.x, z.y); });
+    }
+}
+
+template <int N>
+__device__ __forceinline__ void k_plane_inv_body(int k, const double2 *__restrict__ spec, double *__restrict__ p,
+                                                 const double2 *__restrict__ tw, const Scalars *__restrict__ sc, int ld)
+{
+    const bool stop = halted(sc);
+    extern __shared__ double2 lds[];
+    constexpr int n = N, half = N / 2, nh = half + 1, LM = line_threads(N), lstride = rline_stride(N);
+    double2 *xl = lds, *rows = lds + half * lstride;
+    const int t = threadIdx.x;
+    {
+        const int line = t % nh, tj = min(t / nh, LM - 1);
+        const double2 *in = spec + spec_row(k, 0, n, ld) + line;
+        if constexpr (is_pow2(N)) {
+            double2 v[8];
+#pragma unroll
+            for (int m = 0; m < 8; m++) v[m] = in[(size_t)(tj + m * LM) * ld];
+            fft_regs_c<1, false, N>(v, tj, line, rows, 1, nh, tw);
+#pragma unroll
+            for (int m = 0; m < 8; m++) rows[(tj + m * LM) * nh + line] = v[m];
+        } else {
+            fft_threes<1, false, N, false>(
+                tj, line, rows, 1, nh, tw, [&](int r) { return in[(size_t)r * ld]; },
+                [&](int r, double2 z) { rows[r * nh + line] = z; });
+        }
+    }
+    __syncthreads();
+    const int pl_ = min(t / LM, half - 1), tj = t % LM, j = 2 * pl_;
+    const bool ok = t < half * LM && !stop;
+    if constexpr (is_pow2(N)) {
+        double2 v[8];
+        join_pair(rows + j * nh, rows + (j + 1) * nh, v, tj, LM, half);
+        fft_regs_c<1, true, N>(v, tj, pl_, xl, lstride, 1, tw);
+        if (ok) {
+#pragma unroll
+            for (int m = 0; m < 8; m++) {
+                const int i = tj + m * LM;
+                __builtin_nontemporal_store(v[m].x, &p[IDX(i, j, k)]);
+                __builtin_nontemporal_store(v[m].y, &p[IDX(i, j + 1, k)]);
+            }
+        }
+    } else {
+        for (int e = t; e < half * nh; e += blockDim.x) {
+            const int pq = e / nh, q = e - pq * nh;
+            const double2 a = rows[2 * pq * nh + q], b = rows[(2 * pq + 1) * nh + q];
+            const bool own = q == 0 || q == half;
+            xl[rlds<true>(pq, q, lstride, 1)] = own ? make_double2(a.x, b.x) : make_double2(a.x - b.y, a.y + b.x);
+            if (!own) xl[rlds<true>(pq, n - q, lstride, 1)] = make_double2(a.x + b.y, b.x - a.y);
+        }
+        __syncthreads();
+        fft_threes<1, true, N, true>(
+            tj, pl_, xl, lstride, 1, tw, [&](int q) { return xl[rlds<true>(pl_, q, lstride, 1)]; },
+            [&](int i, double2 z) {
+                if (!ok) return;
+                __builtin_nontemporal_store(z.x, &p[IDX(i, j, k)]);
+                __builtin_nontemporal_store(z.y, &p[IDX(i, j + 1, k)]);
+            });
+    }
+}
+
+template <typename T, int N>
+__global__ void __launch_bounds__(plane_threads(N)) k_plane_fwd(
+    const T *__restrict__ us, const T *__restrict__ vs, const T *__restrict__ ws,
+    double2 *__restrict__ spec, const double2 *__restrict__ tw, const Scalars *__restrict__ sc, Consts c, int ld)
+{
+    k_plane_fwd_body<T, N>(blockIdx.x, us, vs, ws, spec, tw, sc, c, ld);
+}
+
+template <int N>
+__global__ void __launch_bounds__(plane_threads(N)) k_plane_inv(const double2 *__restrict__ spec,
+                                                                double *__restrict__ p, const double2 *__restrict__ tw,
+                                                                const Scalars *__restrict__ sc, int ld)
+{
+    k_plane_inv_body<N>(blockIdx.x, spec, p, tw, sc, ld);
 }
 
 
@@ -1856,15 +2034,162 @@ __device__ __forceinline__ double wave_max(double x)
     return x;
 }
 
-// DIRECT: the line sums' lane exchanges through lane_xor (small n, where a
-// lane holds one or two points of its line and the reduction is the work).
-template <typename T, bool DIRECT>
+// Four (or two) reductions over the 64 lanes at once, each in the order of
+// wave_sum / wave_max: the first exchange puts two lines' halves side by side
+// in one register and the next four lines' quarters, so the later steps run
+// once for all of them.  On return the 16 lanes of row r hold line
+// reduced_line(r): a quarter of the instructions of four butterflies.
+template <typename Op>
+__device__ __forceinline__ double halves(double x, double y, Op op)      // lanes 0-31 x, 32-63 y
+{
+    const unsigned long long a = (unsigned long long)__double_as_longlong(x), b = (unsigned long long)__double_as_longlong(y);
+    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)a, (unsigned)b, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(a >> 32), (unsigned)(b >> 32), false, false);
+    return op(__longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0])),
+              __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1])));
+}
+template <typename Op>
+__device__ __forceinline__ double quarters(double x, double y, Op op)    // even rows of 16 lanes x, odd y
+{
+    const unsigned long long a = (unsigned long long)__double_as_longlong(x), b = (unsigned long long)__double_as_longlong(y);
+    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)a, (unsigned)b, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(a >> 32), (unsigned)(b >> 32), false, false);
+    return op(__longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0])),
+              __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1])));
+}
+template <int LPW, typename Op>
+__device__ __forceinline__ double reduce_lines(const double (&x)[LPW], Op op)
+{
+    static_assert(LPW == 2 || LPW == 4, "two halves or four quarters");
+    double r = halves(x[0], x[1], op);
+    if constexpr (LPW == 4) r = quarters(r, halves(x[2], x[3], op), op);
+    else r = op(r, lane_xor<16>(r));
+    r = op(r, lane_xor<8>(r));
+    r = op(r, lane_xor<4>(r));
+    r = op(r, lane_xor<2>(r));
+    return op(r, lane_xor<1>(r));
+}
+template <int LPW>
+__device__ __forceinline__ int reduced_line(int lane)
+{
+    return LPW == 4 ? 2 * ((lane >> 4) & 1) + (lane >> 5) : lane >> 5;
+}
+
+// A wavefront owns LPW consecutive x-lines of a plane, whose p(j-1) is mostly
+// the line before, and reduces them together.  ONE: lines of at most 64 points,
+// one per lane (without a loop over the line a lane's value is its sum and
+// maximum, and four lines fit the registers; two do otherwise).  PLANE (with
+// ONE): a block owns a whole plane and forms its plane sums too, in the order of
+// k_reduce_planes.
+template <typename T, int LPW, bool ONE, bool PLANE>
+__device__ __forceinline__ void k_project_lines(uint3 blk,
+    const T *__restrict__ us, const T *__restrict__ vs, const T *__restrict__ ws,
+    const double *__restrict__ p, T *__restrict__ u, T *__restrict__ v, T *__restrict__ w,
+    double *__restrict__ lsum, double *__restrict__ lmax, const Scalars *__restrict__ sc, Consts c)
+{
+    const bool stop = halted(sc);
+    const int n = c.n;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, per = n / LPW;
+    int j0, k;
+    if constexpr (PLANE) {
+        j0 = wave * LPW;
+        k = blk.x;
+    } else {
+        const unsigned g = blk.x * (BLK / 64) + wave;
+        if (g >= (unsigned)(per * n)) return;
+        k = g / per;
+        j0 = (g - k * per) * LPW;
+    }
+    const int km = k == 0 ? n - 1 : k - 1, jm = j0 == 0 ? n - 1 : j0 - 1;
+    const double dtr = c.dt / c.rho, dxi = c.dxi;
+    double sum[3][LPW], comp[3][LPW], top[3][LPW];     // comp: Neumaier compensation (FP32 storage only)
+#pragma unroll
+    for (int m = 0; m < 3; m++)
+#pragma unroll
+        for (int q = 0; q < LPW; q++) { sum[m][q] = comp[m][q] = 0.0; top[m][q] = -__builtin_inf(); }
+    auto points = [&](int i) {
+        const int im = i == 0 ? n - 1 : i - 1;
+        T a[3][LPW];
+        double pc[LPW + 1], px[LPW], pz[LPW];          // p at rows j0-1.., at i-1, at k-1
+        pc[0] = p[IDX(i, jm, k)];
+#pragma unroll
+        for (int q = 0; q < LPW; q++) {
+            const size_t id = IDX(i, j0 + q, k);
+            a[0][q] = us[id]; a[1][q] = vs[id]; a[2][q] = ws[id];
+            pc[q + 1] = p[id];
+            px[q] = p[IDX(im, j0 + q, k)];
+            pz[q] = p[IDX(i, j0 + q, km)];
+        }
+#pragma unroll
+        for (int q = 0; q < LPW; q++) {
+            const double p0 = pc[q + 1];
+            const T t[3] = {(T)((double)a[0][q] - dtr * (p0 - px[q]) * dxi),
+                            (T)((double)a[1][q] - dtr * (p0 - pc[q]) * dxi),
+                            (T)((double)a[2][q] - dtr * (p0 - pz[q]) * dxi)};
+            const size_t id = IDX(i, j0 + q, k);
+            if (!stop) {
+                __builtin_nontemporal_store(t[0], &u[id]);
+                __builtin_nontemporal_store(t[1], &v[id]);
+                __builtin_nontemporal_store(t[2], &w[id]);
+            }
+#pragma unroll
+            for (int m = 0; m < 3; m++) {
+                const double x = t[m];
+                if constexpr (sizeof(T) == 4) neumaier(sum[m][q], comp[m][q], x);
+                else sum[m][q] = sum[m][q] + x;
+                top[m][q] = ONE ? x : nanmax(top[m][q], x);
+                if constexpr (ONE && sizeof(T) == 4) sum[m][q] = sum[m][q] + comp[m][q];
+            }
+        }
+    };
+    if constexpr (ONE) {
+        if (lane < n) points(lane);
+    } else {
+        for (int i = lane; i < n; i += 64) points(i);
+    }
+    if (stop) return;
+    const auto add = [](double x, double y) { return x + y; };
+    const auto most = [](double x, double y) { return nanmax(x, y); };
+    const size_t nn = (size_t)n * n;
+    __shared__ double plane[PLANE ? 6 : 1][PLANE ? 64 : 1];
+#pragma unroll
+    for (int m = 0; m < 3; m++) {
+        if constexpr (!ONE && sizeof(T) == 4)
+#pragma unroll
+            for (int q = 0; q < LPW; q++) sum[m][q] = sum[m][q] + comp[m][q];
+        const double a = reduce_lines(sum[m], add), b = reduce_lines(top[m], most);
+        if ((lane & (LPW == 4 ? 15 : 31)) == 0) {
+            const int j = j0 + reduced_line<LPW>(lane);
+            if constexpr (PLANE) {
+                plane[m][j] = a;
+                plane[3 + m][j] = b;
+            } else {
+                lsum[m * nn + (size_t)k * n + j] = a;
+                lmax[m * nn + (size_t)k * n + j] = b;
+            }
+        }
+    }
+    if constexpr (PLANE) {                     // lsum, lmax: the plane sums and maxima here
+        __syncthreads();
+        for (int m = wave; m < 6; m += (int)(blockDim.x >> 6)) {
+            if (m < 3) {
+                const double a = wave_sum(lane < n ? 0.0 + plane[m][lane] : 0.0);
+                if (lane == 0) lsum[m * n + k] = a;
+            } else {
+                const double b = wave_max(lane < n ? plane[m][lane] : -__builtin_inf());
+                if (lane == 0) lmax[(m - 3) * n + k] = b;
+            }
+        }
+    }
+}
+
+template <typename T>
 __device__ __forceinline__ void k_project_body(uint3 blk,
     const T *__restrict__ us, const T *__restrict__ vs, const T *__restrict__ ws,
     const double *__restrict__ p, T *__restrict__ u, T *__restrict__ v, T *__restrict__ w,
     double *__restrict__ lsum, double *__restrict__ lmax, const Scalars *__restrict__ sc, Consts c)
 {
-    if (halted(sc)) return;
+    const bool stop = halted(sc);
     const int n = c.n;
     const int lane = threadIdx.x & 63;
     const size_t line = ((size_t)blk.x * BLK + threadIdx.x) >> 6;
@@ -1882,6 +2207,7 @@ __device__ __forceinline__ void k_project_body(uint3 blk,
         const T tu = (T)((double)us[id] - dtr * (p0 - p[IDX(im, j, k)]) * dxi);
         const T tv = (T)((double)vs[id] - dtr * (p0 - p[IDX(i, jm, k)]) * dxi);
         const T tw = (T)((double)ws[id] - dtr * (p0 - p[IDX(i, j, km)]) * dxi);
+        if (stop) return;
         __builtin_nontemporal_store(tu, &u[id]);
         __builtin_nontemporal_store(tv, &v[id]);
         __builtin_nontemporal_store(tw, &w[id]);
@@ -1894,8 +2220,8 @@ __device__ __forceinline__ void k_project_body(uint3 blk,
         mu_ = nanmax(mu_, uu); mv = nanmax(mv, vv); mw = nanmax(mw, ww);
     }
     if constexpr (sizeof(T) == 4) { su = su + cu; sv = sv + cv; sw = sw + cw; }
-    su = wave_sum<DIRECT>(su); sv = wave_sum<DIRECT>(sv); sw = wave_sum<DIRECT>(sw);
-    mu_ = wave_max<DIRECT>(mu_); mv = wave_max<DIRECT>(mv); mw = wave_max<DIRECT>(mw);
+    su = wave_sum<false>(su); sv = wave_sum<false>(sv); sw = wave_sum<false>(sw);
+    mu_ = wave_max<false>(mu_); mv = wave_max<false>(mv); mw = wave_max<false>(mw);
     if (lane == 0) {
         const size_t nn = (size_t)n * n;
         lsum[line] = su; lsum[nn + line] = sv; lsum[2 * nn + line] = sw;
@@ -1903,14 +2229,32 @@ __device__ __forceinline__ void k_project_body(uint3 blk,
     }
 }
 
-template <typename T, bool DIRECT>
-__global__ void __launch_bounds__(BLK) k_project(
+// The forms of the projection: lines per wavefront, and whether a block forms
+// its plane's sums (small boxes; lsum, lmax are then psum, pmax).
+struct ProjectForm {
+    int lpw;
+    bool plane;
+};
+__host__ __device__ constexpr ProjectForm project_form(int n)
+{
+    return n <= 48 && n % 4 == 0 ? ProjectForm{4, true} : n <= 128 ? ProjectForm{2, false} : ProjectForm{0, false};
+}
+__host__ __device__ constexpr int gang_lpw(int n) { return n <= 64 && n % 4 == 0 ? 4 : 2; }
+__host__ __device__ constexpr unsigned project_blocks(int n)
+{
+    const ProjectForm f = project_form(n);
+    return f.plane ? n : f.lpw ? (unsigned)((n / f.lpw * n + BLK / 64 - 1) / (BLK / 64)) : (unsigned)(((size_t)n * n * 64 + BLK - 1) / BLK);
+}
+
+template <typename T, int LPW, bool PLANE>
+__global__ void __launch_bounds__(PLANE ? 1024 : BLK) k_project(
     const T *__restrict__ us, const T *__restrict__ vs, const T *__restrict__ ws,
     const double *__restrict__ p, T *__restrict__ u, T *__restrict__ v, T *__restrict__ w,
     double *__restrict__ lsum, double *__restrict__ lmax, const Scalars *__restrict__ sc, Consts c)
 {
-    k_project_body<T, DIRECT>(make_uint3(blockIdx.x, blockIdx.y, blockIdx.z), us, vs, ws, p, u, v, w, lsum, lmax,
-                              sc, c);
+    const uint3 b = make_uint3(blockIdx.x, blockIdx.y, blockIdx.z);
+    if constexpr (LPW > 0) k_project_lines<T, LPW, PLANE, PLANE>(b, us, vs, ws, p, u, v, w, lsum, lmax, sc, c);
+    else k_project_body<T>(b, us, vs, ws, p, u, v, w, lsum, lmax, sc, c);
 }
 
 
@@ -1920,19 +2264,20 @@ __device__ __forceinline__ void k_reduce_planes_body(uint3 blk, const double *__
                                                       double *__restrict__ psum, double *__restrict__ pmax,
                                                       const Scalars *__restrict__ sc, int n)
 {
-    if (halted(sc)) return;
+    const bool stop = halted(sc);
     const int k = blk.x, comp = blk.y, lane = threadIdx.x;
     const size_t nn = (size_t)n * n;
     const double *ls = lsum + comp * nn + (size_t)k * n;
     const double *lm = lmax + comp * nn + (size_t)k * n;
     double s = 0.0, m = -__builtin_inf();
+#pragma unroll 4
     for (int j = lane; j < n; j += 64) {
         s = s + ls[j];
         m = nanmax(m, lm[j]);
     }
     s = wave_sum(s);
     m = wave_max(m);
-    if (lane == 0) {
+    if (lane == 0 && !stop) {
         psum[comp * n + k] = s;
         pmax[comp * n + k] = m;
     }
@@ -1947,23 +2292,34 @@ __global__ void __launch_bounds__(64) k_reduce_planes(const double *__restrict__
 
 
 // Means (main.f90:906-913), signed umax (937-941), CFL (942-945), halt flag.
-__device__ __forceinline__ void k_finalize_body(uint3 blk, const double *__restrict__ psum, const double *__restrict__ pmax,
-                                                 Scalars *__restrict__ sc, Consts c, Scalars *mirror, EnsSlot *slot)
+// One wavefront per sum and maximum.  publish: the last step of a call, which
+// the host waits for through the mirror (a write to host memory and the fence
+// behind it cost about 1 us).
+constexpr int FIN_THREADS = 6 * 64;
+__device__ __forceinline__ void k_finalize_body(const double *__restrict__ psum, const double *__restrict__ pmax,
+                                                Scalars *__restrict__ sc, const Consts &c, Scalars *mirror, EnsSlot *slot,
+                                                int publish)
 {
-    if (sc->halted) return;
-    const int n = c.n, lane = threadIdx.x;
-    double s[3], m[3];
-#pragma unroll
-    for (int comp = 0; comp < 3; comp++) {
-        double a = 0.0, b = -__builtin_inf();
-        for (int k = lane; k < n; k += 64) {
-            a = a + psum[comp * n + k];
-            b = nanmax(b, pmax[comp * n + k]);
-        }
-        s[comp] = wave_sum(a);
-        m[comp] = wave_max(b);
+    const bool stop = sc->halted != 0;
+    const int n = c.n, lane = threadIdx.x & 63, q = threadIdx.x >> 6;
+    __shared__ double part[6];
+    if (q < 3) {
+        double a = 0.0;
+#pragma unroll 4
+        for (int k = lane; k < n; k += 64) a = a + psum[q * n + k];
+        a = wave_sum(a);
+        if (lane == 0) part[q] = a;
+    } else {
+        double b = -__builtin_inf();
+#pragma unroll 4
+        for (int k = lane; k < n; k += 64) b = nanmax(b, pmax[(q - 3) * n + k]);
+        b = wave_max(b);
+        if (lane == 0) part[q] = b;
     }
-    if (lane == 0) {
+    __syncthreads();
+    if (stop) return;
+    if (threadIdx.x == 0) {
+        const double s[3] = {part[0], part[1], part[2]}, m[3] = {part[3], part[4], part[5]};
         const double dn = (double)n;
         double gu = s[0] / dn / dn / dn;
         double gv = s[1] / dn / dn / dn;
@@ -1986,16 +2342,17 @@ __device__ __forceinline__ void k_finalize_body(uint3 blk, const double *__restr
             sc->halted = 1;
             sc->status = status;
         }
-        // the host's copy, its step count last: what mhit_step waits for
-        mirror->umean = gu;
-        mirror->vmean = gv;
-        mirror->wmean = gw;
-        mirror->gumax = gumax;
-        mirror->cou = cou;
-        mirror->halted = halt;
-        mirror->status = status;
-        __threadfence_system();
-        *(volatile int *)&mirror->steps = steps;
+        if (publish || halt) {             // the host's copy, its step count last
+            mirror->umean = gu;
+            mirror->vmean = gv;
+            mirror->wmean = gw;
+            mirror->gumax = gumax;
+            mirror->cou = cou;
+            mirror->halted = halt;
+            mirror->status = status;
+            __threadfence_system();
+            *(volatile int *)&mirror->steps = steps;
+        }
         if (slot) {
             slot->clk[steps % CLK_RING] = wall_clock64();
             if (halt) slot->halted = 1;
@@ -2005,10 +2362,11 @@ __device__ __forceinline__ void k_finalize_body(uint3 blk, const double *__restr
     }
 }
 
-__global__ void __launch_bounds__(64) k_finalize(const double *__restrict__ psum, const double *__restrict__ pmax,
-                                                 Scalars *__restrict__ sc, Consts c, Scalars *mirror, EnsSlot *slot)
+__global__ void __launch_bounds__(FIN_THREADS) k_finalize(const double *__restrict__ psum, const double *__restrict__ pmax,
+                                                         Scalars *__restrict__ sc, Consts c, Scalars *mirror,
+                                                         EnsSlot *slot, int publish)
 {
-    k_finalize_body(make_uint3(blockIdx.x, blockIdx.y, blockIdx.z), psum, pmax, sc, c, mirror, slot);
+    k_finalize_body(psum, pmax, sc, c, mirror, slot, publish);
 }
 
 // ---------------------------------------------------------------------------
@@ -2137,13 +2495,34 @@ __global__ void __launch_bounds__(x_threads(N)) kg_xinv(const GangBox *__restric
         k_xinv_body(b, B.f.spec, B.f.p, B.f.tw, B.f.sc, pl, ppb, ld);
 }
 
+template <typename T, int N>
+__global__ void __launch_bounds__(plane_threads(N)) kg_plane_fwd(const GangBox *__restrict__ g, int ld)
+{
+    const GangBox &B = g[blockIdx.y];
+    k_plane_fwd_body<T, N>(blockIdx.x, (const T *)B.f.us, (const T *)B.f.vs, (const T *)B.f.ws, B.f.spec, B.f.tw, B.f.sc,
+                           B.c, ld);
+}
+
+template <int N>
+__global__ void __launch_bounds__(plane_threads(N)) kg_plane_inv(const GangBox *__restrict__ g, int ld)
+{
+    const GangBox &B = g[blockIdx.y];
+    k_plane_inv_body<N>(blockIdx.x, B.f.spec, B.f.p, B.f.tw, B.f.sc, ld);
+}
+
+// A gang's boxes do not form their plane sums here (a launch has one block size).
 template <typename T>
 __global__ void __launch_bounds__(BLK) kg_project(const GangBox *__restrict__ g, int nbox, GangGrid gg)
 {
     unsigned l;
     const GangBox &B = g[gang_block(gg, nbox, l)];
-    k_project_body<T, true>(make_uint3(l, 0, 0), (const T *)B.f.us, (const T *)B.f.vs, (const T *)B.f.ws, B.f.p,
-                      (T *)B.f.u, (T *)B.f.v, (T *)B.f.w, B.f.lsum, B.f.lmax, B.f.sc, B.c);
+    const uint3 b = make_uint3(l, 0, 0);
+    const T *us = (const T *)B.f.us, *vs = (const T *)B.f.vs, *ws = (const T *)B.f.ws;
+    T *u = (T *)B.f.u, *v = (T *)B.f.v, *w = (T *)B.f.w;
+    if (gang_lpw(B.c.n) == 4)
+        k_project_lines<T, 4, true, false>(b, us, vs, ws, B.f.p, u, v, w, B.f.lsum, B.f.lmax, B.f.sc, B.c);
+    else
+        k_project_lines<T, 2, false, false>(b, us, vs, ws, B.f.p, u, v, w, B.f.lsum, B.f.lmax, B.f.sc, B.c);
 }
 
 __global__ void __launch_bounds__(64) kg_reduce_planes(const GangBox *__restrict__ g, int nbox, GangGrid gg)
@@ -2155,10 +2534,10 @@ __global__ void __launch_bounds__(64) kg_reduce_planes(const GangBox *__restrict
                          B.c.n);
 }
 
-__global__ void __launch_bounds__(64) kg_finalize(const GangBox *__restrict__ g)
+__global__ void __launch_bounds__(FIN_THREADS) kg_finalize(const GangBox *__restrict__ g, int publish)
 {
     const GangBox &B = g[blockIdx.x];
-    k_finalize_body(make_uint3(0, 0, 0), B.f.psum, B.f.pmax, B.f.sc, B.c, B.f.mirror, B.f.slot);
+    k_finalize_body(B.f.psum, B.f.pmax, B.f.sc, B.c, B.f.mirror, B.f.slot, publish);
 }
 
 
@@ -2826,7 +3205,8 @@ static int col_tile(const FftPlan &pl)
 // constants: the column passes for their default tile (rtile_n) alone, the x
 // passes for any number of line pairs per block.  FFT_SIZES_GANG: also in gang
 // launches (boxes of up to 128^3).
-#define FFT_SIZES_GANG(X) X(32) X(36) X(48) X(54) X(64) X(72) X(96) X(108) X(128)
+#define FFT_SIZES_PLANE(X) X(32) X(36) X(48) X(54) X(64)
+#define FFT_SIZES_GANG(X) FFT_SIZES_PLANE(X) X(72) X(96) X(108) X(128)
 #define FFT_SIZES(X) FFT_SIZES_GANG(X) X(144) X(162) X(192) X(216) X(256) X(288) X(324) X(384) X(432) X(486) X(512) X(1024)
 
 static bool compiled_n(int n, bool gang)
@@ -2865,6 +3245,17 @@ static void with_n(int n, Fn &&fn)
     fn(std::integral_constant<int, 0>());
 }
 
+template <typename Fn>
+static void with_plane_n(int n, Fn &&fn)
+{
+#define FFT_CASE(N) case N: static_assert(N <= PLANE_MAX, "a plane fits one block"); fn(std::integral_constant<int, N>()); return;
+    switch (n) {
+    FFT_SIZES_PLANE(FFT_CASE)
+    default: return;
+    }
+#undef FFT_CASE
+}
+
 // A power of two the runtime-plan register kernels take (radices 8/4/2, one
 // thread per 8 elements).
 static bool pow2_regs(const FftPlan &pl) { return pl.n >= 16 && is_pow2(pl.n); }
@@ -2890,6 +3281,23 @@ static int fft_threads(const FftPlan &pl, int nlines)
     int t = nlines * (pl.n / plan_rmin(pl));
     t = ((t + 63) / 64) * 64;
     return t < 64 ? 64 : t;
+}
+
+// Whether a box's x and y passes run plane by plane in one block: a small
+// compiled length whose x and y shapes are the defaults (a shape set by hand
+// asks for the separate passes).
+// One box: n blocks leave most CUs idle, and the forward passes, whose threads
+// load eleven values per point pair, gain only at 32^3 and in FP32 up to 48^3
+// (forward pair / in one, us: 32^3 11.1 / 9.2, 48^3 FP32 9.7 / 8.7, FP64 9.7 /
+// 14.9, 64^3 FP32 10.6 / 12.0, FP64 12.3 / 16.1); the inverse passes gain at every
+// size (64^3 10.0 / 8.1).  A gang fills the CUs: 8 boxes of 64^3 20.4 / 15.6 and
+// 18.1 / 10.1.
+bool plane_fwd_alone(const Consts &c) { return c.n <= 32 || (c.mixed && c.n <= 48); }
+bool plane_passes(const Consts &c, const FftPlan &pl, const Tuning &tu)
+{
+    auto def = [&](int knob, int d) { return tu.v[knob] == 0 || tu.v[knob] == d; };
+    return c.n <= PLANE_MAX && compiled_n(c.n, true) && def(KNOB_XPAIRS, default_pairs(pl)) &&
+           def(KNOB_XIPAIRS, default_pairs(pl)) && def(KNOB_YTILE, default_tile(pl));
 }
 
 // Tunable launch shapes.  Every candidate satisfies what the kernels assume:
@@ -2958,6 +3366,30 @@ void launch_xfwd(const Fields &f, const Consts &c, const FftPlan &pl, const Tuni
     li->name = "xfwd_div"; li->bytes = (c.mixed ? 2.5 : 4.0) * F(c);
 }
 
+void launch_plane_fwd(const Fields &f, const Consts &c, hipStream_t s, LaunchInfo *li)
+{
+    with_plane_n(c.n, [&](auto NC) {
+        constexpr int N = decltype(NC)::value;
+        const dim3 grid(N), blk(plane_threads(N));
+        if (c.mixed)
+            hipLaunchKernelGGL((k_plane_fwd<float, N>), grid, blk, plane_lds(N), s, (const float *)f.us,
+                               (const float *)f.vs, (const float *)f.ws, f.spec, f.tw, f.sc, c, f.ld);
+        else
+            hipLaunchKernelGGL((k_plane_fwd<double, N>), grid, blk, plane_lds(N), s, f.us, f.vs, f.ws, f.spec, f.tw, f.sc,
+                               c, f.ld);
+    });
+    li->name = "plane_fwd"; li->bytes = (c.mixed ? 2.5 : 4.0) * F(c);
+}
+
+void launch_plane_inv(const Fields &f, const Consts &c, hipStream_t s, LaunchInfo *li)
+{
+    with_plane_n(c.n, [&](auto NC) {
+        constexpr int N = decltype(NC)::value;
+        hipLaunchKernelGGL(k_plane_inv<N>, dim3(N), dim3(plane_threads(N)), plane_lds(N), s, f.spec, f.p, f.tw, f.sc, f.ld);
+    });
+    li->name = "plane_inv"; li->bytes = 16.0 * (double)(c.n / 2 + 1) * c.n * c.n + F(c);
+}
+
 void launch_ypass(const Fields &f, const Consts &c, const FftPlan &pl, const Tuning &tu, int inverse,
                   hipStream_t s, LaunchInfo *li)
 {
@@ -3020,24 +3452,24 @@ void launch_xinv(const Fields &f, const Consts &c, const FftPlan &pl, const Tuni
     li->name = "x_inv"; li->bytes = 16.0 * (double)(c.n / 2 + 1) * c.n * c.n + F(c);
 }
 
+template <typename T>
+static void launch_project_t(const Fields &f, const Consts &c, hipStream_t s)
+{
+    const ProjectForm form = project_form(c.n);
+    auto kern = form.plane ? k_project<T, 4, true> : form.lpw == 2 ? k_project<T, 2, false> : k_project<T, 0, false>;
+    const dim3 grid(project_blocks(c.n)), blk(form.plane ? c.n / form.lpw * 64 : BLK);
+    hipLaunchKernelGGL(kern, grid, blk, 0, s, (const T *)f.us, (const T *)f.vs, (const T *)f.ws, f.p, (T *)f.u, (T *)f.v,
+                       (T *)f.w, form.plane ? f.psum : f.lsum, form.plane ? f.pmax : f.lmax, f.sc, c);
+}
+
 void launch_project(const Fields &f, const Consts &c, hipStream_t s, LaunchInfo *li)
 {
-    size_t threads = (size_t)c.n * c.n * 64;
-    // lines of up to 128 points: the line sums' exchanges are the work, so the
-    // direct lane exchanges (for 8 points per lane at 512 the crossbar form
-    // measured 2% faster)
-    const bool direct = c.n <= 128;
-    const dim3 grid(nblocks(threads, BLK));
-    if (c.mixed) {
-        auto kern = direct ? k_project<float, true> : k_project<float, false>;
-        hipLaunchKernelGGL(kern, grid, dim3(BLK), 0, s, (const float *)f.us, (const float *)f.vs, (const float *)f.ws,
-                           f.p, (float *)f.u, (float *)f.v, (float *)f.w, f.lsum, f.lmax, f.sc, c);
-    } else {
-        auto kern = direct ? k_project<double, true> : k_project<double, false>;
-        hipLaunchKernelGGL(kern, grid, dim3(BLK), 0, s, f.us, f.vs, f.ws, f.p, f.u, f.v, f.w, f.lsum, f.lmax, f.sc, c);
-    }
+    if (c.mixed) launch_project_t<float>(f, c, s);
+    else launch_project_t<double>(f, c, s);
     li->name = "project"; li->bytes = (c.mixed ? 4.0 : 7.0) * F(c);
 }
+
+bool project_sums_planes(const Consts &c) { return project_form(c.n).plane; }
 
 void launch_reduce(const Fields &f, const Consts &c, hipStream_t s, LaunchInfo *li)
 {
@@ -3045,9 +3477,10 @@ void launch_reduce(const Fields &f, const Consts &c, hipStream_t s, LaunchInfo *
     li->name = "reduce_planes"; li->bytes = 6.0 * 8.0 * c.n * c.n;
 }
 
-void launch_finalize(const Fields &f, const Consts &c, hipStream_t s, LaunchInfo *li)
+void launch_finalize(const Fields &f, const Consts &c, bool publish, hipStream_t s, LaunchInfo *li)
 {
-    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(64), 0, s, f.psum, f.pmax, f.sc, c, f.mirror, f.slot);
+    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(FIN_THREADS), 0, s, f.psum, f.pmax, f.sc, c, f.mirror, f.slot,
+                       publish ? 1 : 0);
     li->name = "finalize"; li->bytes = 6.0 * 8.0 * c.n;
 }
 
@@ -3070,7 +3503,7 @@ void gang_layout(const GangBox *d, int nbox, const GangSize *sizes, GangLaunch *
             ((n + ATX - 1) / ATX) * ((n + ATY - 1) / ATY) * (n / ka),
             gl->mixed ? ((n + 2 * PTX - 1) / (2 * PTX)) * ((n + PTY - 1) / PTY) * (n / km)
                       : ((n + MTX - 1) / MTX) * ((n + MTY - 1) / MTY) * (n / km),
-            (int)nblocks((size_t)n * n * 64, BLK), 3 * n};
+            (int)nblocks((size_t)n / gang_lpw(n) * n, BLK / 64), 3 * n};
         for (int q = 0; q < GP_COUNT; q++) gl->grid[q].first[b + 1] = gl->grid[q].first[b] + blocks[q];
         if (gl->nsize == 0 || gl->size[gl->nsize - 1].n != n) {
             GangSize &z = gl->size[gl->nsize++];
@@ -3078,6 +3511,7 @@ void gang_layout(const GangBox *d, int nbox, const GangSize *sizes, GangLaunch *
             z.off = b;
             z.cnt = 0;
             z.n = n;
+            z.planes = plane_passes(d[b].c, z.plan, z.tune);
         }
         gl->size[gl->nsize - 1].cnt++;
     }
@@ -3086,7 +3520,7 @@ void gang_layout(const GangBox *d, int nbox, const GangSize *sizes, GangLaunch *
 // One step of a gang laid out by gang_layout (device descriptors g[0..nbox)),
 // with the launch shapes of the one-box passes above: the shared passes once,
 // the FFT passes once per size, on that size's boxes.
-void launch_gang_step(const GangBox *g, int nbox, unsigned euler, const GangLaunch &gl, hipStream_t s0,
+void launch_gang_step(const GangBox *g, int nbox, unsigned euler, bool publish, const GangLaunch &gl, hipStream_t s0,
                       const GangStreams *fs)
 {
     const bool fork = fs && gl.nsize > 1 && fs->n >= gl.nsize - 1;
@@ -3132,7 +3566,16 @@ void launch_gang_step(const GangBox *g, int nbox, unsigned euler, const GangLaun
         const dim3 gx(pairs / xp, nb), gxi(pairs / xip, nb), gy((nh + ty - 1) / ty, n, nb), gz((nh + tz - 1) / tz, n, nb);
         const size_t shy = sizeof(double2) * (size_t)ty * n, shz = sizeof(double2) * (size_t)tz * n;
         const int lt = line_threads(n);
-        if (xr) {
+        const bool planes = z.planes;
+        if (planes) {
+            with_plane_n(n, [&](auto NC) {
+                constexpr int N = decltype(NC)::value;
+                if (gl.mixed)
+                    hipLaunchKernelGGL((kg_plane_fwd<float, N>), dim3(N, nb), dim3(plane_threads(N)), plane_lds(N), s, gs, ld);
+                else
+                    hipLaunchKernelGGL((kg_plane_fwd<double, N>), dim3(N, nb), dim3(plane_threads(N)), plane_lds(N), s, gs, ld);
+            });
+        } else if (xr) {
             with_n<true>(n, [&](auto NC) {
                 constexpr int N = decltype(NC)::value;
                 if (gl.mixed)
@@ -3155,15 +3598,20 @@ void launch_gang_step(const GangBox *g, int nbox, unsigned euler, const GangLaun
             else
                 hipLaunchKernelGGL((kg_ypass<SG, false, 0>), gy, dim3(fft_threads(pl, ty)), shy, s, gs, pl, ld, ty);
         };
-        ypass(std::integral_constant<int, -1>());
+        if (!planes) ypass(std::integral_constant<int, -1>());
         if (zr)
             with_n<true>(col_n(pl, tz), [&](auto NC) {
                 hipLaunchKernelGGL((kg_zpoisson<true, decltype(NC)::value>), gz, dim3(tz * lt), shz, s, gs, pl, ld, tz);
             });
         else
             hipLaunchKernelGGL((kg_zpoisson<false, 0>), gz, dim3(fft_threads(pl, tz)), shz, s, gs, pl, ld, tz);
-        ypass(std::integral_constant<int, 1>());
-        if (xr)
+        if (!planes) ypass(std::integral_constant<int, 1>());
+        if (planes)
+            with_plane_n(n, [&](auto NC) {
+                constexpr int N = decltype(NC)::value;
+                hipLaunchKernelGGL(kg_plane_inv<N>, dim3(N, nb), dim3(plane_threads(N)), plane_lds(N), s, gs, ld);
+            });
+        else if (xr)
             with_n<true>(n, [&](auto NC) {
                 hipLaunchKernelGGL((kg_xinv<true, decltype(NC)::value>), gxi, dim3(xip * lt), xip * line, s, gs, pl, xip,
                                    ld);
@@ -3181,7 +3629,7 @@ void launch_gang_step(const GangBox *g, int nbox, unsigned euler, const GangLaun
     else
         hipLaunchKernelGGL(kg_project<double>, dim3((unsigned)gp.first[nbox]), dim3(BLK), 0, s, g, nbox, gp);
     hipLaunchKernelGGL(kg_reduce_planes, dim3((unsigned)gr.first[nbox]), dim3(64), 0, s, g, nbox, gr);
-    hipLaunchKernelGGL(kg_finalize, dim3(nbox), dim3(64), 0, s, g);
+    hipLaunchKernelGGL(kg_finalize, dim3(nbox), dim3(FIN_THREADS), 0, s, g, publish ? 1 : 0);
 }
 
 // Inverse 3-D transform of the half spectrum into `out` (n^3, x fastest):

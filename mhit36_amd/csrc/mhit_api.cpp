@@ -98,7 +98,7 @@ struct Arena {
 constexpr size_t HOST_BLOCK = (size_t)4 << 20;
 constexpr int HOST_BLOCKS = 32, SLOTS_PER_PAGE = 64;
 struct HostSlot {
-    Scalars mirror;       // written by the last kernel of every step
+    Scalars mirror;       // written by the last kernel of a call's last step
     Scalars copy;         // landing place of read_scalars
     char pad[256 - 2 * sizeof(Scalars)];
 };
@@ -960,7 +960,8 @@ extern "C" int mhit_kernel_stats(mhit_ctx *c, mhit_kstat *out, int max_entries, 
 // ---------------------------------------------------------------------------
 // One timestep, main.f90:329-946
 // ---------------------------------------------------------------------------
-static void enqueue_step(mhit_ctx *c)
+// publish: the step's scalars go to the host mirror too.
+static void enqueue_step(mhit_ctx *c, bool publish)
 {
     Fields &f = c->f;
     const Consts &k = c->kc;
@@ -972,19 +973,28 @@ static void enqueue_step(mhit_ctx *c)
         std::swap(f.phi, f.phin);
     }
     timed(c, [&](LaunchInfo *li) { launch_momentum(f, k, c->tune, alpha, beta, s, li); });
-    timed(c, [&](LaunchInfo *li) { launch_xfwd(f, k, c->plan, c->tune, s, li); });
-    timed(c, [&](LaunchInfo *li) { launch_ypass(f, k, c->plan, c->tune, 0, s, li); });
+    const bool planes = plane_passes(k, c->plan, c->tune);
+    if (planes && plane_fwd_alone(k)) {
+        timed(c, [&](LaunchInfo *li) { launch_plane_fwd(f, k, s, li); });
+    } else {
+        timed(c, [&](LaunchInfo *li) { launch_xfwd(f, k, c->plan, c->tune, s, li); });
+        timed(c, [&](LaunchInfo *li) { launch_ypass(f, k, c->plan, c->tune, 0, s, li); });
+    }
     timed(c, [&](LaunchInfo *li) { launch_zpoisson(f, k, c->plan, c->tune, s, li); });
-    timed(c, [&](LaunchInfo *li) { launch_ypass(f, k, c->plan, c->tune, 1, s, li); });
-    timed(c, [&](LaunchInfo *li) { launch_xinv(f, k, c->plan, c->tune, s, li); });
+    if (planes) {
+        timed(c, [&](LaunchInfo *li) { launch_plane_inv(f, k, s, li); });
+    } else {
+        timed(c, [&](LaunchInfo *li) { launch_ypass(f, k, c->plan, c->tune, 1, s, li); });
+        timed(c, [&](LaunchInfo *li) { launch_xinv(f, k, c->plan, c->tune, s, li); });
+    }
     timed(c, [&](LaunchInfo *li) { launch_project(f, k, s, li); });
-    timed(c, [&](LaunchInfo *li) { launch_reduce(f, k, s, li); });
-    timed(c, [&](LaunchInfo *li) { launch_finalize(f, k, s, li); });
+    if (!project_sums_planes(k)) timed(c, [&](LaunchInfo *li) { launch_reduce(f, k, s, li); });
+    timed(c, [&](LaunchInfo *li) { launch_finalize(f, k, publish, s, li); });
     c->nsteps_since_init++;
 }
 
 // Waits for the steps enqueued since dev_steps and reads the scalars they left,
-// from the pinned mirror that each step's last kernel writes.  A short wait
+// from the pinned mirror that the last step's last kernel writes.  A short wait
 // polls the mirror's step count, up to about the time of the driver's own
 // wake-up; then, or when steps halted (a halted step writes nothing), the
 // stream is synchronised.  One step of a 32^3 box per call: 83 us, 132 us with
@@ -1012,7 +1022,7 @@ extern "C" int mhit_step(mhit_ctx *c, int nsteps, mhit_diag *d)
     auto t0 = std::chrono::steady_clock::now();
     double *phi0 = c->f.phi, *phin0 = c->f.phin;
     const int since0 = c->nsteps_since_init, steps0 = c->dev_steps;
-    for (int st = 0; st < nsteps; st++) enqueue_step(c);
+    for (int st = 0; st < nsteps; st++) enqueue_step(c, st == nsteps - 1);
     HIPCHK(hipGetLastError());
     Scalars s1;
     int rc = wait_steps(c, nsteps, &s1);
@@ -1123,7 +1133,7 @@ extern "C" int mhit_step_batch(mhit_ctx *const *ctx, int nbox, int nsteps, mhit_
             if (since0[order[j]] == 0) euler |= 1u << j;
         for (int st = 0; st < nsteps; st++) {
             const GangBox *g = lead->gang + (run[0]->kc.phiflag && (st & 1) ? GANG_MAX : 0);
-            launch_gang_step(g, m, st == 0 ? euler : 0u, gl, s, &lead->gang_fs);
+            launch_gang_step(g, m, st == 0 ? euler : 0u, st == nsteps - 1, gl, s, &lead->gang_fs);
         }
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(s));
@@ -1433,8 +1443,11 @@ static int tune_impl(mhit_ctx *c, double *ms_h, double *ms_t)
         double ms = 0.0;
         rc = tune_time(c, knob, best, a, b, 3, &ms);
     }
+    const bool planes = plane_passes(c->kc, c->plan, Tuning());
     for (int knob = 0; knob < KNOB_COUNT && rc == MHIT_OK; knob++) {
         if (knob == KNOB_KZ_ACDI && !c->kc.phiflag) continue;
+        // a small box's x and y passes run plane by plane, and have no shape
+        if (planes && (knob == KNOB_XPAIRS || knob == KNOB_XIPAIRS || knob == KNOB_YTILE)) continue;
         int cand[12];
         const int nc = knob_candidates(knob, c->kc, c->plan, cand, 12);
         const int def = knob_default(knob, c->kc, c->plan);
@@ -1843,7 +1856,7 @@ static int capture_step(mhit_ctx *c, hipGraphExec_t *out)
     double *phi = c->f.phi, *phin = c->f.phin;
     const int since = c->nsteps_since_init;
     HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeRelaxed));
-    enqueue_step(c);
+    enqueue_step(c, false);
     hipError_t e1 = hipStreamEndCapture(c->stream, &g);
     c->f.phi = phi;
     c->f.phin = phin;
@@ -2080,7 +2093,7 @@ static int gang_launch(mhit_ens *e, EnsGang *g, unsigned euler)
     const GangBox *d = g->dev + (size_t)g->slot * 2 * GANG_MAX + (par ? GANG_MAX : 0);
     const int m = (int)g->members.size();
     if (euler || !e->cfg.use_graphs || g->steady < GANG_STEADY) {
-        launch_gang_step(d, m, euler, g->gl, g->stream);
+        launch_gang_step(d, m, euler, false, g->gl, g->stream);
         HIPCHK(hipGetLastError());
         return MHIT_OK;
     }
@@ -2088,7 +2101,7 @@ static int gang_launch(mhit_ens *e, EnsGang *g, unsigned euler)
     if (!x) {
         hipGraph_t gr = nullptr;
         HIPCHK(hipStreamBeginCapture(g->stream, hipStreamCaptureModeRelaxed));
-        launch_gang_step(d, m, 0u, g->gl, g->stream);
+        launch_gang_step(d, m, 0u, false, g->gl, g->stream);
         HIPCHK(hipStreamEndCapture(g->stream, &gr));
         hipError_t ei = hipGraphInstantiate(&x, gr, nullptr, nullptr, 0);
         (void)hipGraphDestroy(gr);
@@ -2305,7 +2318,7 @@ extern "C" int mhit_ens_progress(mhit_ens *e, int *n_active, int *n_queued)
                                                     : r->g_ab2[c->kc.phiflag ? r->launched % 2 : 0];
                 if (hipGraphLaunch(g, c->stream) != hipSuccess) return MHIT_ERR_HIP;
             } else {
-                enqueue_step(c);
+                enqueue_step(c, false);
             }
             r->launched++;
         }
