@@ -142,6 +142,8 @@ struct Tuning {
 // Valid values of `knob` for this box (at most `cap`), and the heuristic's value.
 int knob_candidates(int knob, const Consts &c, const FftPlan &pl, int *out, int cap);
 int knob_default(int knob, const Consts &c, const FftPlan &pl);
+// Whether the default form of this box's pass has no such shape (small boxes).
+bool knob_unused(int knob, const Consts &c, const FftPlan &pl);
 
 void launch_acdi(const Fields &f, const Consts &c, const Tuning &tu, hipStream_t s, LaunchInfo *li);
 void launch_momentum(const Fields &f, const Consts &c, const Tuning &tu, double alpha, double beta,

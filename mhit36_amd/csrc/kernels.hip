@@ -75,6 +75,8 @@ constexpr int HS0 = ATHREADS / 2, HP0 = 3 * ATHREADS / 4;   // first thread of e
 static_assert(HS0 + NHS <= HP0 && HP0 + NHP <= ATHREADS, "one ring cell per thread at most");
 
 __device__ __forceinline__ int wrap(int a, int n) { a %= n; return a < 0 ? a + n : a; }
+// The same for an index less than one period outside.
+__device__ __forceinline__ int wrap_once(int a, int n) { return a < 0 ? a + n : a >= n ? a - n : a; }
 
 // FP64: the project's own table-driven log (bit-identical to the oracle;
 // `tab` is the block's LDS copy of the table) and IEEE division.  FP32 (the
@@ -128,6 +130,67 @@ __device__ __forceinline__ T *at_off(T *base, unsigned off)
     return reinterpret_cast<T *>(reinterpret_cast<char *>(base) + off * (unsigned)sizeof(T));
 }
 
+// psi = eps log(phi / (1 - phi))
+template <typename T>
+__device__ __forceinline__ T acdi_psi(T f, T eps, T en, const double *tab)
+{
+    T val = f < (T)1.0 ? f : (T)1.0;
+    if constexpr (sizeof(T) == 4) val = val > (T)0.0 ? val : (T)0.0;   // FP32 phi: no log of a negative
+    return eps * tlog(tdiv(val + en, ((T)1.0 - val) + en), tab);
+}
+// The sharpening flux a(psi) n at a cell: g* the undivided gradient of psi, pc0
+// psi and f phi at the cell.  The factor 1/4 (1 - tanh^2(psi/(2 eps))) of the flux
+// comes from the cell's phi, no tanh: psi = eps log(A/B), A = val + enum,
+// B = (1 - val) + enum, so it is A B / (A + B)^2 exactly (and, like the
+// tanh form, goes to 0 with A as phi nears -enum).  A NaN psi (phi below
+// -enum) stays NaN, as tanh(NaN) would.
+template <typename T>
+__device__ __forceinline__ void acdi_flux(T gx, T gy, T gz, T pc0, T f, T en, T tiny, T &sx, T &sy, T &sz)
+{
+    T normod = tdiv((T)1.0, tsqrt((gx * gx + gy * gy) + gz * gz) + tiny);
+    T val = f < (T)1.0 ? f : (T)1.0;
+    if constexpr (sizeof(T) == 4) val = val > (T)0.0 ? val : (T)0.0;   // as psi's FP32 clamp
+    const T A = val + en, B = ((T)1.0 - val) + en, S = A + B;
+    const T a = pc0 != pc0 ? pc0 : tdiv(A * B, S * S);
+    sx = a * (gx * normod);
+    sy = a * (gy * normod);
+    sz = a * (gz * normod);
+}
+// phi^{n+1} at a cell: phi there (f0) and at its neighbours, the velocity at the
+// cell's faces and the differences of the flux components over two cells.  The
+// expressions of the march's output stencil, which has them in place: through
+// this function its FP64 form spills 20 values instead of 14 (512^3: 1.59 against
+// 1.44 ms).
+template <typename T>
+__device__ __forceinline__ T acdi_advance(T f0, T fxp, T fxm, T fyp, T fym, T fzp, T fzm, T uip, T u0, T vjp, T v0,
+                                          T wkp, T w0, T dsx, T dsy, T dsz, T gamma, T eps, T dxi, T ddxi, T dt)
+{
+    if constexpr (sizeof(T) == 4) {
+        const T hd = (T)0.5 * dxi;
+        const T A = __builtin_fmaf(uip, fxp + f0, -(u0 * (f0 + fxm)));
+        const T B = __builtin_fmaf(vjp, fyp + f0, -(v0 * (f0 + fym)));
+        const T C = __builtin_fmaf(wkp, fzp + f0, -(w0 * (f0 + fzm)));
+        const T lap = ((fxp + fxm) + (fyp + fym)) + __builtin_fmaf((T)-6.0, f0, fzp + fzm);
+        const T sdiv = (dsx + dsy) + dsz;
+        const T r2 = __builtin_fmaf(gamma * eps * ddxi, lap, -hd * (((A + B) + C) + gamma * sdiv));
+        return __builtin_fmaf(dt, r2, f0);
+    } else {
+        T A = uip * (T)0.5 * (fxp + f0) - u0 * (T)0.5 * (f0 + fxm);
+        T B = vjp * (T)0.5 * (fyp + f0) - v0 * (T)0.5 * (f0 + fym);
+        T C = wkp * (T)0.5 * (fzp + f0) - w0 * (T)0.5 * (f0 + fzm);
+        T r = (-(A * dxi) - B * dxi) - C * dxi;
+        T dxx = eps * ((fxp - (T)2.0 * f0) + fxm) * ddxi;
+        T dyy = eps * ((fyp - (T)2.0 * f0) + fym) * ddxi;
+        T dzz = eps * ((fzp - (T)2.0 * f0) + fzm) * ddxi;
+        T rphi = r + gamma * ((dxx + dyy) + dzz);
+        T X = dsx * (T)0.5 * dxi;
+        T Y = dsy * (T)0.5 * dxi;
+        T Z = dsz * (T)0.5 * dxi;
+        T r2 = rphi - gamma * ((X + Y) + Z);
+        return f0 + dt * r2;
+    }
+}
+
 // MARCH3: the march unrolled by three planes (the one-box FP64 pass); else
 // one plane per iteration with the registers copied forward (FP32, and the
 // gang pass, whose per-box addressing would not fit the unrolled march in 128
@@ -171,26 +234,9 @@ __device__ __forceinline__ void k_acdi_body(uint3 blk,
     const int hP = (hc.y + 2) * APX + (hc.x + 2), hS = (hc.y + 1) * ASX + (hc.x + 1);
 
     auto ld_phi = [&](unsigned off, int m) { return ld_off(phi + nn * (size_t)wrap(m, n), off); };
-    auto psi_of = [&](T f) {                  // psi = eps log(phi / (1 - phi))
-        T val = f < (T)1.0 ? f : (T)1.0;
-        if constexpr (sizeof(T) == 4) val = val > (T)0.0 ? val : (T)0.0;   // FP32 phi: no log of a negative
-        return eps * tlog(tdiv(val + en, ((T)1.0 - val) + en), tabL);
-    };
-    // Normal and a(psi) at a cell: g* the undivided gradient of psi, pc0 psi
-    // and f phi at the cell.  The factor 1/4 (1 - tanh^2(psi/(2 eps))) of the flux
-    // comes from the cell's phi, no tanh: psi = eps log(A/B), A = val + enum,
-    // B = (1 - val) + enum, so it is A B / (A + B)^2 exactly (and, like the
-    // tanh form, goes to 0 with A as phi nears -enum).  A NaN psi (phi below
-    // -enum) stays NaN, as tanh(NaN) would.
+    auto psi_of = [&](T f) { return acdi_psi(f, eps, en, tabL); };
     auto sharp = [&](T gx, T gy, T gz, T pc0, T f, T &sx, T &sy, T &sz) {
-        T normod = tdiv((T)1.0, tsqrt((gx * gx + gy * gy) + gz * gz) + tiny);
-        T val = f < (T)1.0 ? f : (T)1.0;
-        if constexpr (sizeof(T) == 4) val = val > (T)0.0 ? val : (T)0.0;   // as psi's FP32 clamp
-        const T A = val + en, B = ((T)1.0 - val) + en, S = A + B;
-        const T a = pc0 != pc0 ? pc0 : tdiv(A * B, S * S);
-        sx = a * (gx * normod);
-        sy = a * (gy * normod);
-        sz = a * (gz * normod);
+        acdi_flux(gx, gy, gz, pc0, f, en, tiny, sx, sy, sz);
     };
 
     if constexpr (sizeof(T) == 8) {
@@ -384,6 +430,113 @@ __global__ void __launch_bounds__(ATHREADS, sizeof(T) == 4 ? 8 : 4) k_acdi(
     Consts c, int kz)
 {
     k_acdi_body<T>(xcd_block(), u, v, w, phi, phin, sc, mtab, c, kz);
+}
+
+
+// ---------------------------------------------------------------------------
+// The phase field of a small box, where a march of a few planes is bound by its
+// serial chain (four planes of psi before the first output, 1.6 us per plane):
+// a block owns BTX x BTY x BTZ cells, forms psi on them and two cells around,
+// then the flux on them and the face neighbours, then the output: three steps
+// with a barrier between, in exchange for psi at 3 cells per cell instead of
+// 1.4 plus the prologue.  March / box, us (event times): FP64 32^3 12.2 / 8.5,
+// 64^3 13.1 / 12.2, 72^3 22.2 / 18.0, 96^3 22.7 / 25.2; FP32 32^3 8.4 / 6.8,
+// 72^3 12.5 / 11.7, 96^3 12.9 / 15.3: used up to 72^3.
+// ---------------------------------------------------------------------------
+constexpr int BTX = 16, BTY = 8, BTZ = 4, BTHREADS = BTX * BTY * BTZ;
+constexpr int BPX = BTX + 4, BPY = BTY + 4, BPZ = BTZ + 4, BPSI = BPX * BPY * BPZ;
+constexpr int BRX = 2 * BTY * BTZ, BRY = 2 * BTX * BTZ, BRZ = 2 * BTX * BTY;      // face neighbours
+static_assert(BRX + BRY + BRZ <= BTHREADS, "one face neighbour per thread at most");
+
+template <typename T>
+__global__ void __launch_bounds__(BTHREADS) k_acdi_box(
+    const T *__restrict__ u, const T *__restrict__ v, const T *__restrict__ w,
+    const T *__restrict__ phi, T *__restrict__ phin, const Scalars *__restrict__ sc, const double *__restrict__ mtab,
+    Consts c)
+{
+    constexpr int NTAB = sizeof(T) == 8 ? TAB_LHI + 2 * 129 : 1, Q = (BPSI + BTHREADS - 1) / BTHREADS;
+    static_assert(NTAB <= BTHREADS, "one table entry per thread");
+    __shared__ double tabL[NTAB];
+    __shared__ T psiL[BPSI], phL[BPSI];
+    __shared__ T sxL[BTZ * BTY * (BTX + 2)], syL[BTZ * (BTY + 2) * BTX], szL[(BTZ + 2) * BTY * BTX];
+    const bool stop = halted(sc);
+    const int n = c.n, tid = threadIdx.x;
+    const int i0 = blockIdx.x * BTX, j0 = blockIdx.y * BTY, k0 = blockIdx.z * BTZ;
+    const T eps = c.eps, en = c.enumr, dxi = c.dxi, ddxi = c.ddxi, tiny = (T)1.0E-16f;
+    const T um = sc->umean, vm = sc->vmean, wm = sc->wmean, gamma = c.gamma_factor * sc->gumax;
+    const unsigned nn = (unsigned)n * n;
+    // a tile reaches BTX + 1 past its first cell: below 2n from n = 18 on
+    auto per = [&](int a) { return n >= BTX + 2 ? wrap_once(a, n) : wrap(a, n); };
+    auto off = [&](int x, int y, int z) {
+        return (unsigned)per(i0 + x) + (unsigned)n * (unsigned)per(j0 + y) + nn * (unsigned)per(k0 + z);
+    };
+    // this thread's cell, and every load of the pass
+    const int x = tid % BTX, y = tid / BTX % BTY, z = tid / (BTX * BTY);
+    const unsigned own = off(x, y, z);
+    const T u0 = ld_off(u, own), v0 = ld_off(v, own), w0 = ld_off(w, own);
+    const T uip = ld_off(u, off(x + 1, y, z)), vjp = ld_off(v, off(x, y + 1, z)), wkp = ld_off(w, off(x, y, z + 1));
+    T f[Q];
+    bool need[Q];
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+        const int e = tid + q * BTHREADS, px = e % BPX - 2, py = e / BPX % BPY - 2, pz = e / (BPX * BPY) - 2;
+        // psi is read up to two cells away in all: face neighbours of the face neighbours
+        const int d = max(max(-px, px - (BTX - 1)), 0) + max(max(-py, py - (BTY - 1)), 0) + max(max(-pz, pz - (BTZ - 1)), 0);
+        need[q] = e < BPSI && d <= 2;
+        f[q] = need[q] ? ld_off(phi, off(px, py, pz)) : (T)0.0;
+    }
+    if constexpr (sizeof(T) == 8) {
+        if (tid < NTAB) tabL[tid] = mtab[tid];
+        __syncthreads();
+    }
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+        if (need[q]) {
+            psiL[tid + q * BTHREADS] = acdi_psi(f[q], eps, en, tabL);
+            phL[tid + q * BTHREADS] = f[q];
+        }
+    __syncthreads();
+    auto at = [&](int a, int b, int d) { return a + 2 + BPX * (b + 2 + BPY * (d + 2)); };
+    auto flux = [&](int e, T &sx, T &sy, T &sz) {
+        acdi_flux(psiL[e + 1] - psiL[e - 1], psiL[e + BPX] - psiL[e - BPX], psiL[e + BPX * BPY] - psiL[e - BPX * BPY],
+                  psiL[e], phL[e], en, tiny, sx, sy, sz);
+    };
+    const int e0 = at(x, y, z);
+    {
+        T sx, sy, sz;
+        flux(e0, sx, sy, sz);
+        sxL[x + 1 + (BTX + 2) * (y + BTY * z)] = sx;
+        syL[x + BTX * (y + 1 + (BTY + 2) * z)] = sy;
+        szL[x + BTX * (y + BTY * (z + 1))] = sz;
+    }
+    if (tid < BRX + BRY + BRZ) {
+        int h = tid;
+        T sx, sy, sz;
+        if (h < BRX) {
+            const int a = h & 1 ? BTX : -1, b = (h >> 1) % BTY, d = (h >> 1) / BTY;
+            flux(at(a, b, d), sx, sy, sz);
+            sxL[a + 1 + (BTX + 2) * (b + BTY * d)] = sx;
+        } else if (h < BRX + BRY) {
+            h -= BRX;
+            const int b = h & 1 ? BTY : -1, a = (h >> 1) % BTX, d = (h >> 1) / BTX;
+            flux(at(a, b, d), sx, sy, sz);
+            syL[a + BTX * (b + 1 + (BTY + 2) * d)] = sy;
+        } else {
+            h -= BRX + BRY;
+            const int d = h & 1 ? BTZ : -1, a = (h >> 1) % BTX, b = (h >> 1) / BTX;
+            flux(at(a, b, d), sx, sy, sz);
+            szL[a + BTX * (b + BTY * (d + 1))] = sz;
+        }
+    }
+    __syncthreads();
+    if (stop || i0 + x >= n || j0 + y >= n || k0 + z >= n) return;
+    const int ex = x + 1 + (BTX + 2) * (y + BTY * z), ey = x + BTX * (y + 1 + (BTY + 2) * z),
+              ez = x + BTX * (y + BTY * (z + 1));
+    const T r = acdi_advance(phL[e0], phL[e0 + 1], phL[e0 - 1], phL[e0 + BPX], phL[e0 - BPX], phL[e0 + BPX * BPY],
+                             phL[e0 - BPX * BPY], uip - um, u0 - um, vjp - vm, v0 - vm, wkp - wm, w0 - wm,
+                             sxL[ex + 1] - sxL[ex - 1], syL[ey + BTX] - syL[ey - BTX], szL[ez + BTX * BTY] - szL[ez - BTX * BTY],
+                             gamma, eps, dxi, ddxi, (T)c.dt);
+    __builtin_nontemporal_store(r, at_off(phin, own));
 }
 
 
@@ -909,6 +1062,113 @@ __global__ void __launch_bounds__(PTHREADS) k_momentum_x2(
     Consts c, double ALPHA, double BETA, int kz)
 {
     k_momentum_x2_body<PHI, T>(xcd_block(), u, v, w, phi, us, vs, ws, ruo, rvo, rwo, sinf, cosf, sc, c, ALPHA, BETA, kz);
+}
+
+
+// ---------------------------------------------------------------------------
+// The same pass without a march, for boxes whose march is a few planes long and
+// then bound by its chain of barriers, not by memory: one point per thread,
+// every neighbour loaded from the caches, the CSF force formed at the point and
+// at its three lower neighbours.  49 loads per point, all in flight at once,
+// and no barrier.  mom_point on 3 x 3 neighbourhoods (row stride 3, the point
+// at 4): the results are those of k_momentum bit for bit.  March / point with
+// the phase field, us (event times): FP64 32^3 10.9 / 6.7, 64^3 14.3 / 13.0,
+// 72^3 21.7 / 20.0 but without the phase field 18.0 at either, 96^3 29.7 / 32.9;
+// FP32 32^3 11.5 / 6.6, 64^3 13.2 / 8.9, 96^3 22.1 / 18.2, 108^3 28.3 / 29.5:
+// used up to 64^3 and 96^3.  Bound by the L1: 49 loads of 512 bytes per wavefront.
+// At most 4 waves per SIMD, or the compiler saves registers and waits for
+// the loads in groups (FP64 32^3 7.9 us).
+// ---------------------------------------------------------------------------
+constexpr int DTX = 32, DTY = 8;
+
+template <int PHI, typename T>
+__device__ __forceinline__ void k_momentum_point_body(uint3 blk,
+    const T *__restrict__ u, const T *__restrict__ v, const T *__restrict__ w, const T *__restrict__ phi,
+    T *__restrict__ us, T *__restrict__ vs, T *__restrict__ ws,
+    T *__restrict__ ruo, T *__restrict__ rvo, T *__restrict__ rwo,
+    const double *__restrict__ sinf, const double *__restrict__ cosf, const Scalars *__restrict__ sc,
+    const Consts &c, double ALPHA, double BETA)
+{
+    const bool stop = halted(sc);
+    const int n = c.n;
+    const int i = blk.x * DTX + threadIdx.x % DTX, j = blk.y * DTY + threadIdx.x / DTX, k = blk.z;
+    if (i >= n || j >= n) return;
+    // periodic neighbours: columns, rows and planes -1 (and -2 for phi), 0, +1, as offsets
+    const int im = i == 0 ? n - 1 : i - 1, ip = i + 1 == n ? 0 : i + 1;
+    const int jm = j == 0 ? n - 1 : j - 1, jp = j + 1 == n ? 0 : j + 1;
+    const int km = k == 0 ? n - 1 : k - 1, kp = k + 1 == n ? 0 : k + 1;
+    const unsigned nn = (unsigned)n * n;
+    const unsigned r0 = (unsigned)n * j, rm = (unsigned)n * jm, rp = (unsigned)n * jp;
+    const unsigned z0 = nn * k, zm = nn * km, zp = nn * kp;
+    const T um = sc->umean, vm = sc->vmean, wm = sc->wmean;
+    T U0[9] = {}, V0[9] = {}, W0[9] = {}, Up[9] = {}, Vp[9] = {}, Wp[9] = {};
+    auto at = [](const T *f, unsigned off) { return ld_off(f, off); };
+    U0[4] = at(u, z0 + r0 + i) - um; U0[5] = at(u, z0 + r0 + ip) - um; U0[3] = at(u, z0 + r0 + im) - um;
+    U0[7] = at(u, z0 + rp + i) - um; U0[1] = at(u, z0 + rm + i) - um; U0[2] = at(u, z0 + rm + ip) - um;
+    V0[4] = at(v, z0 + r0 + i) - vm; V0[5] = at(v, z0 + r0 + ip) - vm; V0[3] = at(v, z0 + r0 + im) - vm;
+    V0[7] = at(v, z0 + rp + i) - vm; V0[1] = at(v, z0 + rm + i) - vm; V0[6] = at(v, z0 + rp + im) - vm;
+    W0[4] = at(w, z0 + r0 + i) - wm; W0[5] = at(w, z0 + r0 + ip) - wm; W0[3] = at(w, z0 + r0 + im) - wm;
+    W0[7] = at(w, z0 + rp + i) - wm; W0[1] = at(w, z0 + rm + i) - wm;
+    Up[4] = at(u, zp + r0 + i) - um;
+    Vp[4] = at(v, zp + r0 + i) - vm;
+    Wp[4] = at(w, zp + r0 + i) - wm; Wp[3] = at(w, zp + r0 + im) - wm; Wp[1] = at(w, zp + rm + i) - wm;
+    const T uzm = at(u, zm + r0 + i) - um, uxpm = at(u, zm + r0 + ip) - um;
+    const T vzm = at(v, zm + r0 + i) - vm, vypm = at(v, zm + rp + i) - vm;
+    const T wzm = at(w, zm + r0 + i) - wm;
+    const unsigned t = z0 + r0 + i;
+    const T ro0 = ruo[t], ro1 = rvo[t], ro2 = rwo[t];
+    MomK<T> q;
+    q.dxi = (T)c.dxi; q.ddxi = (T)c.ddxi; q.mu = (T)c.mu; q.rhoi = (T)c.rhoi;
+    q.f1 = (T)c.f1; q.f2 = (T)c.f2; q.f3 = (T)c.f3;
+    q.dt = (T)c.dt; q.alpha = (T)ALPHA; q.beta = (T)BETA;
+    T FX[9] = {}, FY[9] = {}, FZ[9] = {}, fzm = 0;
+    if constexpr (PHI) {
+        const T sig6 = (T)((T)6.0 * c.sigma), eps = (T)c.eps, epsi = (T)c.epsi, dxi = q.dxi, ddxi = q.ddxi;
+        const int imm = im == 0 ? n - 1 : im - 1, jmm = jm == 0 ? n - 1 : jm - 1, kmm = km == 0 ? n - 1 : km - 1;
+        const unsigned rmm = (unsigned)n * jmm, zmm = nn * kmm;
+        // CSF force at a cell centre: sigma 6 chem times half the difference of the pair (p, m) / dx
+        auto chem = [&](T f0, T fxp, T fxm, T fyp, T fym, T fzp, T fzm_) {
+            T t1 = f0 * ((T)1.0 - f0) * ((T)1.0 - (T)2.0 * f0) * epsi;
+            T s6 = (((((fxp + fxm) + fyp) + fym) + fzp) + fzm_) - (T)6.0 * f0;
+            return t1 - eps * s6 * ddxi;
+        };
+        auto part = [&](T ch, T fp, T fm) { return sig6 * ch * ((T)0.5 * (fp - fm) * dxi); };
+        const T f0 = at(phi, z0 + r0 + i), fx = at(phi, z0 + r0 + ip), fX = at(phi, z0 + r0 + im);
+        const T fy = at(phi, z0 + rp + i), fY = at(phi, z0 + rm + i), fz = at(phi, zp + r0 + i), fZ = at(phi, zm + r0 + i);
+        const T fXX = at(phi, z0 + r0 + imm), fXy = at(phi, z0 + rp + im), fXY = at(phi, z0 + rm + im),
+                fXz = at(phi, zp + r0 + im), fXZ = at(phi, zm + r0 + im);
+        const T fYY = at(phi, z0 + rmm + i), fYx = at(phi, z0 + rm + ip), fYz = at(phi, zp + rm + i),
+                fYZ = at(phi, zm + rm + i);
+        const T fZZ = at(phi, zmm + r0 + i), fZx = at(phi, zm + r0 + ip), fZy = at(phi, zm + rp + i);
+        const T c0 = chem(f0, fx, fX, fy, fY, fz, fZ);
+        FX[4] = part(c0, fx, fX);
+        FY[4] = part(c0, fy, fY);
+        FZ[4] = part(c0, fz, fZ);
+        FX[3] = part(chem(fX, f0, fXX, fXy, fXY, fXz, fXZ), f0, fXX);
+        FY[1] = part(chem(fY, fYx, fXY, f0, fYY, fYz, fYZ), f0, fYY);
+        fzm = part(chem(fZ, fZx, fXZ, fZy, fYZ, f0, fZZ), f0, fZZ);
+    }
+    T o[6];
+    mom_point<PHI, 3, 3>(U0, V0, W0, Up, Vp, Wp, 4, uzm, vzm, wzm, uxpm, vypm, FX, FY, FZ, fzm, 4, (T)sinf[k], (T)cosf[j],
+                         (T)sinf[i], (T)cosf[k], (T)sinf[j], (T)cosf[i], ro0, ro1, ro2, q, o);
+    if (stop) return;
+    __builtin_nontemporal_store(o[0], &us[t]);
+    __builtin_nontemporal_store(o[1], &vs[t]);
+    __builtin_nontemporal_store(o[2], &ws[t]);
+    __builtin_nontemporal_store(o[3], &ruo[t]);
+    __builtin_nontemporal_store(o[4], &rvo[t]);
+    __builtin_nontemporal_store(o[5], &rwo[t]);
+}
+
+template <int PHI, typename T>
+__global__ void __launch_bounds__(DTX * DTY) __attribute__((amdgpu_waves_per_eu(1, 4))) k_momentum_point(
+    const T *__restrict__ u, const T *__restrict__ v, const T *__restrict__ w, const T *__restrict__ phi,
+    T *__restrict__ us, T *__restrict__ vs, T *__restrict__ ws,
+    T *__restrict__ ruo, T *__restrict__ rvo, T *__restrict__ rwo,
+    const double *__restrict__ sinf, const double *__restrict__ cosf, const Scalars *__restrict__ sc,
+    Consts c, double ALPHA, double BETA)
+{
+    k_momentum_point_body<PHI, T>(xcd_block(), u, v, w, phi, us, vs, ws, ruo, rvo, rwo, sinf, cosf, sc, c, ALPHA, BETA);
 }
 
 
@@ -3131,43 +3391,67 @@ static int kz_momentum(int n, int mixed, int boxes = 1)
     return march_kz(n, ((n + tx - 1) / tx) * ((n + ty - 1) / ty), mixed ? 768 : 1024, mixed ? 3 : 1, 32, boxes);
 }
 
+// The forms of small boxes take no slab height: they run unless one was set by
+// hand that differs from the default.
+static bool kz_default(const Tuning &tu, int knob, int kz) { return tu.v[knob] == 0 || tu.v[knob] == kz; }
+static bool acdi_in_boxes(const Consts &c, const Tuning &tu)
+{
+    return c.n <= 72 && kz_default(tu, KNOB_KZ_ACDI, kz_acdi(c.n, c.mixed));
+}
+static bool momentum_by_point(const Consts &c, const Tuning &tu)
+{
+    return c.n <= (c.mixed ? 96 : 64) && kz_default(tu, KNOB_KZ_MOM, kz_momentum(c.n, c.mixed));
+}
+
+template <typename T>
+static void launch_acdi_t(const Fields &f, const Consts &c, int kz, bool boxes, hipStream_t s)
+{
+    const int n = c.n;
+    const T *u = (const T *)f.u, *v = (const T *)f.v, *w = (const T *)f.w, *phi = (const T *)f.phi;
+    if (boxes)
+        hipLaunchKernelGGL(k_acdi_box<T>, dim3((n + BTX - 1) / BTX, (n + BTY - 1) / BTY, (n + BTZ - 1) / BTZ),
+                           dim3(BTHREADS), 0, s, u, v, w, phi, (T *)f.phin, f.sc, f.mtab, c);
+    else
+        hipLaunchKernelGGL(k_acdi<T>, dim3((n + ATX - 1) / ATX, (n + ATY - 1) / ATY, n / kz), dim3(ATHREADS), 0, s, u, v, w,
+                           phi, (T *)f.phin, f.sc, f.mtab, c, kz);
+}
+
 void launch_acdi(const Fields &f, const Consts &c, const Tuning &tu, hipStream_t s, LaunchInfo *li)
 {
-    const int n = c.n, kz = tu.v[KNOB_KZ_ACDI] ? tu.v[KNOB_KZ_ACDI] : kz_acdi(n, c.mixed);
-    dim3 grid((n + ATX - 1) / ATX, (n + ATY - 1) / ATY, n / kz);
-    if (c.mixed)
-        hipLaunchKernelGGL(k_acdi<float>, grid, dim3(ATHREADS), 0, s, (const float *)f.u, (const float *)f.v,
-                           (const float *)f.w, (const float *)f.phi, (float *)f.phin, f.sc, f.mtab, c, kz);
-    else
-        hipLaunchKernelGGL(k_acdi<double>, grid, dim3(ATHREADS), 0, s, f.u, f.v, f.w, f.phi, f.phin, f.sc, f.mtab, c,
-                           kz);
+    const int kz = tu.v[KNOB_KZ_ACDI] ? tu.v[KNOB_KZ_ACDI] : kz_acdi(c.n, c.mixed);
+    const bool boxes = acdi_in_boxes(c, tu);
+    if (c.mixed) launch_acdi_t<float>(f, c, kz, boxes, s);
+    else launch_acdi_t<double>(f, c, kz, boxes, s);
     li->name = "acdi"; li->bytes = (c.mixed ? 2.5 : 5.0) * F(c);
+}
+
+template <int PHI, typename T>
+static void launch_momentum_t(const Fields &f, const Consts &c, int kz, bool point, double alpha, double beta,
+                              hipStream_t s)
+{
+    const int n = c.n;
+    const T *u = (const T *)f.u, *v = (const T *)f.v, *w = (const T *)f.w, *ph = (const T *)f.phi;
+    T *us = (T *)f.us, *vs = (T *)f.vs, *ws = (T *)f.ws, *ru = (T *)f.ruo, *rv = (T *)f.rvo, *rw = (T *)f.rwo;
+    if (point)
+        hipLaunchKernelGGL((k_momentum_point<PHI, T>), dim3((n + DTX - 1) / DTX, (n + DTY - 1) / DTY, n), dim3(DTX * DTY),
+                           0, s, u, v, w, ph, us, vs, ws, ru, rv, rw, f.sinf, f.cosf, f.sc, c, alpha, beta);
+    else if constexpr (sizeof(T) == 4)
+        hipLaunchKernelGGL((k_momentum_x2<PHI, T>), dim3((n + 2 * PTX - 1) / (2 * PTX), (n + PTY - 1) / PTY, n / kz),
+                           dim3(PTHREADS), 0, s, u, v, w, ph, us, vs, ws, ru, rv, rw, f.sinf, f.cosf, f.sc, c, alpha, beta,
+                           kz);
+    else
+        hipLaunchKernelGGL((k_momentum<PHI, T>), dim3((n + MTX - 1) / MTX, (n + MTY - 1) / MTY, n / kz), dim3(MTHREADS), 0,
+                           s, u, v, w, ph, us, vs, ws, ru, rv, rw, f.sinf, f.cosf, f.sc, c, alpha, beta, kz);
 }
 
 void launch_momentum(const Fields &f, const Consts &c, const Tuning &tu, double alpha, double beta, hipStream_t s,
                      LaunchInfo *li)
 {
-    const int n = c.n, kz = tu.v[KNOB_KZ_MOM] ? tu.v[KNOB_KZ_MOM] : kz_momentum(n, c.mixed);
-    dim3 grid((n + MTX - 1) / MTX, (n + MTY - 1) / MTY, n / kz);
-    if (c.mixed) {
-        using T = float;
-        const T *u = (const T *)f.u, *v = (const T *)f.v, *w = (const T *)f.w, *ph = (const T *)f.phi;
-        T *us = (T *)f.us, *vs = (T *)f.vs, *ws = (T *)f.ws, *ru = (T *)f.ruo, *rv = (T *)f.rvo, *rw = (T *)f.rwo;
-        const dim3 g2((n + 2 * PTX - 1) / (2 * PTX), (n + PTY - 1) / PTY, n / kz);
-        if (c.phiflag)
-            hipLaunchKernelGGL((k_momentum_x2<1, T>), g2, dim3(PTHREADS), 0, s, u, v, w, ph, us, vs, ws, ru, rv, rw,
-                               f.sinf, f.cosf, f.sc, c, alpha, beta, kz);
-        else
-            hipLaunchKernelGGL((k_momentum_x2<0, T>), g2, dim3(PTHREADS), 0, s, u, v, w, ph, us, vs, ws, ru, rv, rw,
-                               f.sinf, f.cosf, f.sc, c, alpha, beta, kz);
-    } else {
-        if (c.phiflag)
-            hipLaunchKernelGGL((k_momentum<1, double>), grid, dim3(MTHREADS), 0, s, f.u, f.v, f.w, f.phi, f.us, f.vs,
-                               f.ws, f.ruo, f.rvo, f.rwo, f.sinf, f.cosf, f.sc, c, alpha, beta, kz);
-        else
-            hipLaunchKernelGGL((k_momentum<0, double>), grid, dim3(MTHREADS), 0, s, f.u, f.v, f.w, f.phi, f.us, f.vs,
-                               f.ws, f.ruo, f.rvo, f.rwo, f.sinf, f.cosf, f.sc, c, alpha, beta, kz);
-    }
+    const int kz = tu.v[KNOB_KZ_MOM] ? tu.v[KNOB_KZ_MOM] : kz_momentum(c.n, c.mixed);
+    const bool point = momentum_by_point(c, tu);
+    auto launch = c.mixed ? (c.phiflag ? launch_momentum_t<1, float> : launch_momentum_t<0, float>)
+                          : (c.phiflag ? launch_momentum_t<1, double> : launch_momentum_t<0, double>);
+    launch(f, c, kz, point, alpha, beta, s);
     li->name = "momentum"; li->bytes = (c.mixed ? (c.phiflag ? 6.5 : 6.0) : (c.phiflag ? 13.0 : 12.0)) * F(c);
 }
 
@@ -3311,6 +3595,16 @@ int knob_default(int knob, const Consts &c, const FftPlan &pl)
     case KNOB_XPAIRS:
     case KNOB_XIPAIRS: return default_pairs(pl);
     default: return default_tile(pl);
+    }
+}
+
+bool knob_unused(int knob, const Consts &c, const FftPlan &pl)
+{
+    switch (knob) {
+    case KNOB_KZ_ACDI: return acdi_in_boxes(c, Tuning());
+    case KNOB_KZ_MOM: return momentum_by_point(c, Tuning());
+    case KNOB_ZTILE: return false;
+    default: return plane_passes(c, pl, Tuning());
     }
 }
 

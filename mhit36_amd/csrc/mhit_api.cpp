@@ -1443,11 +1443,9 @@ static int tune_impl(mhit_ctx *c, double *ms_h, double *ms_t)
         double ms = 0.0;
         rc = tune_time(c, knob, best, a, b, 3, &ms);
     }
-    const bool planes = plane_passes(c->kc, c->plan, Tuning());
     for (int knob = 0; knob < KNOB_COUNT && rc == MHIT_OK; knob++) {
         if (knob == KNOB_KZ_ACDI && !c->kc.phiflag) continue;
-        // a small box's x and y passes run plane by plane, and have no shape
-        if (planes && (knob == KNOB_XPAIRS || knob == KNOB_XIPAIRS || knob == KNOB_YTILE)) continue;
+        if (knob_unused(knob, c->kc, c->plan)) continue;
         int cand[12];
         const int nc = knob_candidates(knob, c->kc, c->plan, cand, 12);
         const int def = knob_default(knob, c->kc, c->plan);
