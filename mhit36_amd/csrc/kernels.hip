@@ -545,266 +545,29 @@ __global__ void __launch_bounds__(BTHREADS) k_acdi_box(
 // CSF force (phi^{n+1}) interpolated to the faces, AB2/Euler advance
 // and rhs_o <- rhs, in one pass.
 //
-// A block owns an MTX x MTY column and marches kz planes in z.  LDS rings
-// hold u, v, w on an (MTX+2) x (MTY+2) box (planes k-1..k+1), phi on an
-// (MTX+3) x (MTY+3) box (planes k-1..k+1) and the
-// CSF cell-centre force on an (MTX+1) x (MTY+1) box for planes k-1 and k, so
-// every input is read from HBM once per block (plus the halo) and every CSF
-// force is formed once.
+// A block owns an MTX x MTY column and marches kz planes in z.  LDS rings hold
+// u, v, w on an (MTX+2) x (MTY+2) box and phi on an (MTX+3) x (MTY+3) box,
+// three planes each, so every input is read from memory once per block (plus
+// the halo).  What a point needs of plane k-1 (its u, v, w, u(i+1), v(j+1), its
+// phi and the z force) it has seen at that plane and keeps in registers, so
+// the slot of plane k-1 is free for the plane being stored and one barrier a
+// plane is enough.  A thread forms the CSF force of its own cell, and MTX + MTY
+// threads one of the cells before the tile in x or y too; the face averages
+// take the neighbour's part from the lane before (x) or from LDS (y).
+// Bound by memory: 13 values a point.  512 threads, because a taller tile reads
+// less halo (rows of u: 18/16 instead of 10/8) and with one barrier the two
+// blocks of a CU still cover each other's waits.  256^3 and 512^3 with phi:
+// 394 and 3056 us (8 rows, two barriers a plane) -> 360 and 2907 (8 rows, one
+// barrier) -> 348 and 2730 (16 rows); 351 and 2742 with 32 rows.  Without phi:
+// 345 and 2588 -> 325 and 2638 -> 308 and 2435.  13 (12) values at the 5.4 TB/s
+// of a large copy are 2585 (2390) us at 512^3.
 // ---------------------------------------------------------------------------
-constexpr int MTX = 32, MTY = 8, MTHREADS = MTX * MTY;
-constexpr int MUX = MTX + 2, MUY = MTY + 2;       // u/v/w box
-constexpr int MPX = MTX + 3, MPY = MTY + 3;       // phi box
-constexpr int MFX = MTX + 1, MFY = MTY + 1;       // force box
-static_assert(MUX * MUY <= 2 * MTHREADS && MPX * MPY <= 2 * MTHREADS, "box loads assume <= 2 elements per thread");
-
-template <int PHI, typename T>
-__device__ __forceinline__ void k_momentum_body(uint3 blk,
-    const T *__restrict__ u, const T *__restrict__ v, const T *__restrict__ w,
-    const T *__restrict__ phi,
-    T *__restrict__ us, T *__restrict__ vs, T *__restrict__ ws,
-    T *__restrict__ ruo, T *__restrict__ rvo, T *__restrict__ rwo,
-    const double *__restrict__ sinf, const double *__restrict__ cosf, const Scalars *__restrict__ sc,
-    Consts c, double ALPHA, double BETA, int kz)
-{
-    if (halted(sc)) return;
-    __shared__ T UL[3][3][MUY * MUX];
-    __shared__ T PL[PHI ? 3 : 1][PHI ? MPY * MPX : 1];
-    // CSF force of plane k, only where the face interpolation reads it: the x
-    // part at x = -1..MTX-1, the y part at y = -1..MTY-1, the z part at the
-    // points themselves (tile coordinates); the z part of plane k-1 at the
-    // thread's own point is carried in a register (fzm).
-    __shared__ T FXL[PHI ? MTY * (MTX + 1) : 1];
-    __shared__ T FYL[PHI ? (MTY + 1) * MTX : 1];
-    __shared__ T FZL[PHI ? MTY * MTX : 1];
-    const int n = c.n;
-    const int tid = threadIdx.x;
-    const int i0 = blk.x * MTX, j0 = blk.y * MTY, k0 = blk.z * kz;
-    const T um = sc->umean, vm = sc->vmean, wm = sc->wmean;
-    const T dxi = (T)c.dxi, ddxi = (T)c.ddxi, mu = (T)c.mu, rhoi = (T)c.rhoi;
-    const T f1 = (T)c.f1, f2 = (T)c.f2, f3 = (T)c.f3;
-
-    // Box elements of this thread (<= 2 per box) and their x/y offsets.
-    size_t uoff[2], foff[2];
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-        int e = tid + q * MTHREADS;
-        uoff[q] = (size_t)wrap(i0 - 1 + e % MUX, n) + (size_t)n * wrap(j0 - 1 + e / MUX, n);
-        foff[q] = (size_t)wrap(i0 - 2 + e % MPX, n) + (size_t)n * wrap(j0 - 2 + e / MPX, n);
-    }
-    const size_t nn = (size_t)n * n;
-    // Loads run one plane ahead into registers (pu, pp) and are stored into
-    // the LDS rings an iteration later, so their latency overlaps compute.
-    T pu[2][3], pp[2];
-    auto fetch_u = [&](int m) {
-        const size_t zoff = nn * (size_t)wrap(m, n);
-#pragma unroll
-        for (int q = 0; q < 2; q++) {
-            if (tid + q * MTHREADS < MUX * MUY) {
-                size_t g = uoff[q] + zoff;
-                pu[q][0] = u[g]; pu[q][1] = v[g]; pu[q][2] = w[g];
-            }
-        }
-    };
-    auto store_u = [&](int m) {
-        const int slot = (m - k0 + 1) % 3;
-#pragma unroll
-        for (int q = 0; q < 2; q++) {
-            int e = tid + q * MTHREADS;
-            if (e < MUX * MUY) {
-                UL[slot][0][e] = pu[q][0] - um;
-                UL[slot][1][e] = pu[q][1] - vm;
-                UL[slot][2][e] = pu[q][2] - wm;
-            }
-        }
-    };
-    auto fetch_phi = [&](int m) {
-        if constexpr (PHI) {
-            const size_t zoff = nn * (size_t)wrap(m, n);
-#pragma unroll
-            for (int q = 0; q < 2; q++)
-                if (tid + q * MTHREADS < MPX * MPY) pp[q] = phi[foff[q] + zoff];
-        }
-    };
-    auto store_phi = [&](int m) {
-        if constexpr (PHI) {
-            const int slot = (m - k0 + 2) % 3;
-#pragma unroll
-            for (int q = 0; q < 2; q++) {
-                int e = tid + q * MTHREADS;
-                if (e < MPX * MPY) PL[slot][e] = pp[q];
-            }
-        }
-    };
-    auto load_u = [&](int m) { fetch_u(m); store_u(m); };
-    auto load_phi = [&](int m) { fetch_phi(m); store_phi(m); };
-    auto force = [&](int m) {           // CSF force at cell centres (first half) on plane m
-        if constexpr (PHI) {
-            const int ps = (m - k0 + 2) % 3, psm = (m - 1 - k0 + 2) % 3, psp = (m + 1 - k0 + 2) % 3;
-            const T sig6 = (T)((T)6.0 * c.sigma), eps = (T)c.eps, epsi = (T)c.epsi;
-            for (int e = tid; e < MFX * MFY; e += MTHREADS) {
-                int fx_ = e % MFX, fy_ = e / MFX;              // cell x = fx_-1, y = fy_-1 in the tile
-                if (fx_ == 0 && fy_ == 0) continue;             // the corner cell is never read
-                int pc = (fy_ + 1) * MPX + (fx_ + 1);
-                T f0 = PL[ps][pc];
-                T fxp = PL[ps][pc + 1], fxm = PL[ps][pc - 1];
-                T fyp = PL[ps][pc + MPX], fym = PL[ps][pc - MPX];
-                T fzp = PL[psp][pc], fzm = PL[psm][pc];
-                T t1 = f0 * ((T)1.0 - f0) * ((T)1.0 - (T)2.0 * f0) * epsi;
-                T s6 = (((((fxp + fxm) + fyp) + fym) + fzp) + fzm) - (T)6.0 * f0;
-                T chem = t1 - eps * s6 * ddxi;
-                if (fy_ > 0) FXL[(fy_ - 1) * MFX + fx_] = sig6 * chem * ((T)0.5 * (fxp - fxm) * dxi);
-                if (fx_ > 0) FYL[fy_ * MTX + (fx_ - 1)] = sig6 * chem * ((T)0.5 * (fyp - fym) * dxi);
-                if (fx_ > 0 && fy_ > 0) FZL[(fy_ - 1) * MTX + (fx_ - 1)] = sig6 * chem * ((T)0.5 * (fzp - fzm) * dxi);
-            }
-        }
-    };
-
-    // prologue: u planes k0-1, k0; phi planes k0-2 .. k0; force on plane k0-1;
-    // plane k0+1 fetched into registers
-    load_u(k0 - 1);
-    load_u(k0);
-    load_phi(k0 - 2);
-    load_phi(k0 - 1);
-    load_phi(k0);
-    fetch_u(k0 + 1);
-    fetch_phi(k0 + 1);
-    __syncthreads();
-    force(k0 - 1);
-    __syncthreads();      // force(k0-1) reads phi(k0-2), whose slot phi(k0+1) takes next
-
-    const int tx = tid % MTX, ty = tid / MTX;
-    const int i = i0 + tx, j = j0 + ty;
-    const bool active = (i < n) && (j < n);
-    const int kend = min(k0 + kz, n);
-    const int uc = (ty + 1) * MUX + (tx + 1);
-    const int fxc = ty * MFX + (tx + 1);       // x part at x = tx (FXL[fxc-1]: x = tx-1)
-    const int fyc = (ty + 1) * MTX + tx;       // y part at y = ty (FYL[fyc-MTX]: y = ty-1)
-    const int fzc = ty * MTX + tx;
-    T fzm = (T)0.0;                            // z part of the force at plane k-1, this point
-    if constexpr (PHI) fzm = FZL[fzc];
-    const size_t cxy = (size_t)(i < n ? i : 0) + (size_t)n * (j < n ? j : 0);
-    T ro[3] = {(T)0.0, (T)0.0, (T)0.0};
-    if (active) {
-        ro[0] = ruo[cxy + nn * (size_t)k0];
-        ro[1] = rvo[cxy + nn * (size_t)k0];
-        ro[2] = rwo[cxy + nn * (size_t)k0];
-    }
-    // Ring slots (3 each): u plane m in (m-k0+1)%3, phi plane m in (m-k0+2)%3.
-    // phi(k+1) replaces phi(k-2), last read by force(k-1) before the previous
-    // iteration's second barrier; u(k+1) replaces u(k-2), and force(k) the
-    // force of plane k-1, both last read by output(k-1) before this
-    // iteration's first barrier.
-    for (int k = k0; k < kend; k++) {
-        store_phi(k + 1);
-        if (k + 1 < kend) fetch_phi(k + 2);
-        __syncthreads();
-        force(k);
-        store_u(k + 1);
-        if (k + 1 < kend) fetch_u(k + 2);
-        const T ro0 = ro[0], ro1 = ro[1], ro2 = ro[2];
-        if (active && k + 1 < kend) {
-            ro[0] = __builtin_nontemporal_load(&ruo[cxy + nn * (size_t)(k + 1)]);
-            ro[1] = __builtin_nontemporal_load(&rvo[cxy + nn * (size_t)(k + 1)]);
-            ro[2] = __builtin_nontemporal_load(&rwo[cxy + nn * (size_t)(k + 1)]);
-        }
-        __syncthreads();
-        if (active) {
-            const int s0 = (k - k0 + 1) % 3, sm = (k - k0) % 3, sp = (k - k0 + 2) % 3;
-            const T *U0 = UL[s0][0], *V0 = UL[s0][1], *W0 = UL[s0][2];
-            const T *Um = UL[sm][0], *Vm = UL[sm][1], *Wm = UL[sm][2];
-            const T *Up = UL[sp][0], *Vp = UL[sp][1], *Wp = UL[sp][2];
-            const T u0 = U0[uc], v0 = V0[uc], w0 = W0[uc];
-            const T uxp = U0[uc + 1], uxm = U0[uc - 1], uyp = U0[uc + MUX], uym = U0[uc - MUX];
-            const T uzp = Up[uc], uzm = Um[uc];
-            const T vxp = V0[uc + 1], vxm = V0[uc - 1], vyp = V0[uc + MUX], vym = V0[uc - MUX];
-            const T vzp = Vp[uc], vzm = Vm[uc];
-            const T wxp = W0[uc + 1], wxm = W0[uc - 1], wyp = W0[uc + MUX], wym = W0[uc - MUX];
-            const T wzp = Wp[uc], wzm = Wm[uc];
-            T h11 = (uxp + u0) * (uxp + u0) - (u0 + uxm) * (u0 + uxm);
-            T h12 = (uyp + u0) * (vyp + V0[uc + MUX - 1]) - (u0 + uym) * (v0 + vxm);
-            T h13 = (uzp + u0) * (wzp + Wp[uc - 1]) - (u0 + uzm) * (w0 + wxm);
-            T h21 = (uxp + U0[uc + 1 - MUX]) * (vxp + v0) - (u0 + uym) * (v0 + vxm);
-            T h22 = (vyp + v0) * (vyp + v0) - (v0 + vym) * (v0 + vym);
-            T h23 = (wzp + Wp[uc - MUX]) * (vzp + v0) - (w0 + wym) * (v0 + vzm);
-            T h31 = (wxp + w0) * (uxp + Um[uc + 1]) - (w0 + wxm) * (u0 + uzm);
-            T h32 = (vyp + Vm[uc + MUX]) * (wyp + w0) - (v0 + vzm) * (w0 + wym);
-            T h33 = (wzp + w0) * (wzp + w0) - (w0 + wzm) * (w0 + wzm);
-            h11 = h11 * (T)0.25 * dxi; h12 = h12 * (T)0.25 * dxi; h13 = h13 * (T)0.25 * dxi;
-            h21 = h21 * (T)0.25 * dxi; h22 = h22 * (T)0.25 * dxi; h23 = h23 * (T)0.25 * dxi;
-            h31 = h31 * (T)0.25 * dxi; h32 = h32 * (T)0.25 * dxi; h33 = h33 * (T)0.25 * dxi;
-            T ru = -((h11 + h12) + h13);
-            T rv = -((h21 + h22) + h23);
-            T rw = -((h31 + h32) + h33);
-            h11 = mu * ((uxp - (T)2.0 * u0) + uxm) * ddxi;
-            h12 = mu * ((uyp - (T)2.0 * u0) + uym) * ddxi;
-            h13 = mu * ((uzp - (T)2.0 * u0) + uzm) * ddxi;
-            h21 = mu * ((vxp - (T)2.0 * v0) + vxm) * ddxi;
-            h22 = mu * ((vyp - (T)2.0 * v0) + vym) * ddxi;
-            h23 = mu * ((vzp - (T)2.0 * v0) + vzm) * ddxi;
-            h31 = mu * ((wxp - (T)2.0 * w0) + wxm) * ddxi;
-            h32 = mu * ((wyp - (T)2.0 * w0) + wym) * ddxi;
-            h33 = mu * ((wzp - (T)2.0 * w0) + wzm) * ddxi;
-            ru = ru + ((h11 + h12) + h13) * rhoi;
-            rv = rv + ((h21 + h22) + h23) * rhoi;
-            rw = rw + ((h31 + h32) + h33) * rhoi;
-            ru = (ru + f3 * (T)sinf[k]) + f2 * (T)cosf[j];
-            rv = (rv + f1 * (T)sinf[i]) + f3 * (T)cosf[k];
-            rw = (rw + f2 * (T)sinf[j]) + f1 * (T)cosf[i];
-            if constexpr (PHI) {
-                const T fz0 = FZL[fzc];
-                ru = ru + (T)0.5 * (FXL[fxc - 1] + FXL[fxc]) * rhoi;
-                rv = rv + (T)0.5 * (FYL[fyc - MTX] + FYL[fyc]) * rhoi;
-                rw = rw + (T)0.5 * (fzm + fz0) * rhoi;
-                fzm = fz0;
-            }
-            const T dt = (T)c.dt, alpha = (T)ALPHA, beta = (T)BETA;
-            const size_t t = cxy + nn * (size_t)k;
-            __builtin_nontemporal_store(u0 + dt * (alpha * ru - beta * ro0), &us[t]);
-            __builtin_nontemporal_store(v0 + dt * (alpha * rv - beta * ro1), &vs[t]);
-            __builtin_nontemporal_store(w0 + dt * (alpha * rw - beta * ro2), &ws[t]);
-            __builtin_nontemporal_store(ru, &ruo[t]);
-            __builtin_nontemporal_store(rv, &rvo[t]);
-            __builtin_nontemporal_store(rw, &rwo[t]);
-        }
-    }
-}
-
-template <int PHI, typename T>
-__global__ void __launch_bounds__(MTHREADS) k_momentum(
-    const T *__restrict__ u, const T *__restrict__ v, const T *__restrict__ w,
-    const T *__restrict__ phi,
-    T *__restrict__ us, T *__restrict__ vs, T *__restrict__ ws,
-    T *__restrict__ ruo, T *__restrict__ rvo, T *__restrict__ rwo,
-    const double *__restrict__ sinf, const double *__restrict__ cosf, const Scalars *__restrict__ sc,
-    Consts c, double ALPHA, double BETA, int kz)
-{
-    k_momentum_body<PHI, T>(xcd_block(), u, v, w, phi, us, vs, ws, ruo, rvo, rwo, sinf, cosf, sc, c, ALPHA, BETA, kz);
-}
-
-
-// ---------------------------------------------------------------------------
-// The same pass with two x-points per thread, used for FP32 state (in FP64
-// the pair needs 220 VGPRs and 95 KB of LDS: one wave per SIMD): 64 x 8 points
-// per block, every global load and store a float2 (the u/v/w and phi boxes
-// start at the even column i0-2, so pairs never straddle the periodic seam),
-// half the memory instructions per byte of the one-point form.  Each point's
-// arithmetic is mom_point below, written exactly as in k_momentum, so the
-// results are those of k_momentum<PHI, T> bit for bit.
-// ---------------------------------------------------------------------------
-constexpr int PTX = 32, PTY = 8, PTHREADS = PTX * PTY;   // threads; 2 points each in x
-constexpr int PBX = 2 * PTX + 4, PUY = PTY + 2;           // u/v/w box row (68) and rows (10)
-constexpr int PPY = PTY + 3;                              // phi box rows (11), same row as u/v/w
-constexpr int PFX = 2 * PTX + 1, PFY = PTY + 1;           // force box (65 x 9)
-static_assert((PBX / 2) * PUY <= 2 * PTHREADS && (PBX / 2) * PPY <= 2 * PTHREADS, "two pairs per thread");
-static_assert(PFX * PFY <= 3 * PTHREADS, "three force points per thread");
-
 template <typename T>
 struct MomK {
     T dxi, ddxi, mu, rhoi, f1, f2, f3, dt, alpha, beta;
 };
 
-// The momentum point, main.f90:513-696 (as in k_momentum).  U0..W0: plane
+// The momentum point, main.f90:513-696.  U0..W0: plane
 // k, Up..Wp: plane k+1, with row stride SX; uzm..wzm, uxpm (u at k-1, i+1)
 // and vypm (v at k-1, j+1) from plane k-1; FX/FY/FZ the force of plane k and
 // fzm its z part at plane k-1 (row stride FXS).
@@ -865,6 +628,247 @@ __device__ __forceinline__ void mom_point(const T *U0, const T *V0, const T *W0,
     out[4] = rv;
     out[5] = rw;
 }
+
+constexpr int MTX = 32, MTY = 16, MTHREADS = MTX * MTY;
+constexpr int MUX = MTX + 2, MUY = MTY + 2;       // u/v/w box
+constexpr int MPX = MTX + 3, MPY = MTY + 3;       // phi box
+static_assert(MUX * MUY <= 2 * MTHREADS && MPX * MPY <= 2 * MTHREADS, "box loads assume <= 2 elements per thread");
+static_assert(MTX == 32 && MTX + MTY <= MTHREADS, "two tile rows per wavefront; one edge cell per thread");
+
+// The value of the previous lane (x - 1 in the tile; lane 0 gets 0).
+__device__ __forceinline__ double prev_lane(double x)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x138, 0xf, 0xf, true);     // wave_shr:1
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x138, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+
+template <int PHI, typename T>
+__device__ __forceinline__ void k_momentum_body(uint3 blk,
+    const T *__restrict__ u, const T *__restrict__ v, const T *__restrict__ w,
+    const T *__restrict__ phi,
+    T *__restrict__ us, T *__restrict__ vs, T *__restrict__ ws,
+    T *__restrict__ ruo, T *__restrict__ rvo, T *__restrict__ rwo,
+    const double *__restrict__ sinf, const double *__restrict__ cosf, const Scalars *__restrict__ sc,
+    Consts c, double ALPHA, double BETA, int kz)
+{
+    if (halted(sc)) return;
+    __shared__ T UL[3][3][MUY * MUX];
+    __shared__ T PL[PHI ? 3 : 1][PHI ? MPY * MPX : 1];
+    __shared__ T FXL[PHI ? 2 : 1][PHI ? MTY : 1];
+    __shared__ T FYL[PHI ? 2 : 1][PHI ? (MTY + 1) * MTX : 1];
+    const int n = c.n;
+    const int tid = threadIdx.x;
+    const int i0 = blk.x * MTX, j0 = blk.y * MTY, k0 = blk.z * kz;
+    const T um = sc->umean, vm = sc->vmean, wm = sc->wmean;
+    MomK<T> q;
+    q.dxi = (T)c.dxi; q.ddxi = (T)c.ddxi; q.mu = (T)c.mu; q.rhoi = (T)c.rhoi;
+    q.f1 = (T)c.f1; q.f2 = (T)c.f2; q.f3 = (T)c.f3;
+    q.dt = (T)c.dt; q.alpha = (T)ALPHA; q.beta = (T)BETA;
+
+    // Box elements of this thread (<= 2 per box) and their x/y offsets.
+    unsigned uoff[2], foff[2];
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        const int e = tid + r * MTHREADS;
+        uoff[r] = (unsigned)wrap(i0 - 1 + e % MUX, n) + (unsigned)n * wrap(j0 - 1 + e / MUX, n);
+        foff[r] = (unsigned)wrap(i0 - 2 + e % MPX, n) + (unsigned)n * wrap(j0 - 2 + e / MPX, n);
+    }
+    const size_t nn = (size_t)n * n;
+    // Loads run one plane ahead into registers (pu, pp) and are stored into
+    // the LDS rings an iteration later, so their latency overlaps compute.
+    T pu[2][3], pp[2];
+    auto fetch_u = [&](int m) {
+        const size_t zoff = nn * (size_t)wrap(m, n);
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            if (tid + r * MTHREADS < MUX * MUY) {
+                const size_t g = uoff[r] + zoff;
+                pu[r][0] = u[g]; pu[r][1] = v[g]; pu[r][2] = w[g];
+            }
+        }
+    };
+    auto store_u = [&](int slot) {
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            const int e = tid + r * MTHREADS;
+            if (e < MUX * MUY) {
+                UL[slot][0][e] = pu[r][0] - um;
+                UL[slot][1][e] = pu[r][1] - vm;
+                UL[slot][2][e] = pu[r][2] - wm;
+            }
+        }
+    };
+    auto fetch_phi = [&](int m) {
+        if constexpr (PHI) {
+            const size_t zoff = nn * (size_t)wrap(m, n);
+#pragma unroll
+            for (int r = 0; r < 2; r++)
+                if (tid + r * MTHREADS < MPX * MPY) pp[r] = phi[foff[r] + zoff];
+        }
+    };
+    auto store_phi = [&](int slot) {
+        if constexpr (PHI) {
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+                const int e = tid + r * MTHREADS;
+                if (e < MPX * MPY) PL[slot][e] = pp[r];
+            }
+        }
+    };
+    const int tx = tid % MTX, ty = tid / MTX;
+    const int i = i0 + tx, j = j0 + ty;
+    const bool active = (i < n) && (j < n);
+    const int kend = min(k0 + kz, n);
+    const int uc = (ty + 1) * MUX + (tx + 1), pc = (ty + 2) * MPX + (tx + 2);
+    // The cell before the tile in x (row tid) or y (column tid - MTY) whose force this thread forms too.
+    const bool edge_x = tid < MTY, edge = tid < MTX + MTY;
+    const int ec = edge_x ? (tid + 2) * MPX + 1 : MPX + (tid - MTY + 2);
+    const T sig6 = (T)((T)6.0 * c.sigma), eps = (T)c.eps, epsi = (T)c.epsi;
+    auto chem = [&](const T *P0, const T *Pp, int e, T fzm) {
+        const T f0 = P0[e];
+        T t1 = f0 * ((T)1.0 - f0) * ((T)1.0 - (T)2.0 * f0) * epsi;
+        T s6 = (((((P0[e + 1] + P0[e - 1]) + P0[e + MPX]) + P0[e - MPX]) + Pp[e]) + fzm) - (T)6.0 * f0;
+        return t1 - eps * s6 * q.ddxi;
+    };
+    auto part = [&](T ch, T fp, T fm) { return sig6 * ch * ((T)0.5 * (fp - fm) * q.dxi); };
+    // phi of the plane below at the thread's own and edge cell; its own forces
+    // at the plane and, in z, at the plane below
+    T fown = (T)0.0, fedge = (T)0.0, FX[9] = {}, FY[9] = {}, FZ[9] = {}, fzm = (T)0.0;
+    auto force = [&](int s0, int sp, int buf) {
+        if constexpr (PHI) {
+            const T *P0 = PL[s0], *Pp = PL[sp];
+            {
+                const T ch = chem(P0, Pp, pc, fown);
+                FX[4] = part(ch, P0[pc + 1], P0[pc - 1]);
+                FY[4] = part(ch, P0[pc + MPX], P0[pc - MPX]);
+                FZ[4] = part(ch, Pp[pc], fown);
+                FYL[buf][(ty + 1) * MTX + tx] = FY[4];
+                fown = P0[pc];
+            }
+            if (edge) {
+                const T ch = chem(P0, Pp, ec, fedge);
+                if (edge_x) FXL[buf][tid] = part(ch, P0[ec + 1], P0[ec - 1]);
+                else FYL[buf][tid - MTY] = part(ch, P0[ec + MPX], P0[ec - MPX]);
+                fedge = P0[ec];
+            }
+        }
+    };
+    const size_t cxy = (size_t)(i < n ? i : 0) + (size_t)n * (j < n ? j : 0);
+    const int ic = i < n ? i : 0, jc = j < n ? j : 0;
+
+    // prologue: slot of plane m in either ring: (m - k0) % 3
+    fetch_u(k0);
+    T um1[5];           // at plane k - 1: u, v, w, u(i+1), v(j+1)
+    {
+        const size_t zm = nn * (size_t)wrap(k0 - 1, n);
+        um1[0] = u[cxy + zm] - um;
+        um1[1] = v[cxy + zm] - vm;
+        um1[2] = w[cxy + zm] - wm;
+        um1[3] = u[zm + (size_t)n * jc + (ic + 1 == n ? 0 : ic + 1)] - um;
+        um1[4] = v[zm + (size_t)n * (jc + 1 == n ? 0 : jc + 1) + ic] - vm;
+    }
+    T fzz = (T)0.0;
+    if constexpr (PHI) {
+        fzz = phi[cxy + nn * (size_t)wrap(k0 - 2, n)];
+        fetch_phi(k0 - 1); store_phi(2);
+        fetch_phi(k0); store_phi(0);
+        fetch_phi(k0 + 1); store_phi(1);
+    }
+    store_u(0);
+    fetch_u(k0 + 1);
+    if (k0 + 1 < kend) fetch_phi(k0 + 2);
+    T ro[3] = {(T)0.0, (T)0.0, (T)0.0};
+    if (active) {
+        ro[0] = ruo[cxy + nn * (size_t)k0];
+        ro[1] = rvo[cxy + nn * (size_t)k0];
+        ro[2] = rwo[cxy + nn * (size_t)k0];
+    }
+    __syncthreads();
+    if constexpr (PHI) {
+        fzm = part(chem(PL[2], PL[0], pc, fzz), PL[0][pc], fzz);
+        fown = PL[2][pc];
+        if (edge) fedge = PL[2][ec];
+    }
+    force(0, 1, 0);
+    // One barrier a plane.  What is stored before the barrier of plane k (u of
+    // k+1, phi of k+2) takes the slots of u(k-2) and phi(k-1), last read before
+    // the barrier of plane k-1; force(k+1) writes the buffer that output(k-1)
+    // read, before this barrier too.
+    int sa = 0, sb = 1, sn = 2, buf = 0;       // slots of planes k, k+1 and the free one
+    const T sj = (T)sinf[jc], cj = (T)cosf[jc], si = (T)sinf[ic], ci = (T)cosf[ic];
+    for (int k = k0; k < kend; k++) {
+        const bool more = k + 1 < kend;
+        store_u(sb);
+        if (more) {
+            if constexpr (PHI) {
+                store_phi(sn);
+                if (k + 2 < kend) fetch_phi(k + 3);
+            }
+            fetch_u(k + 2);
+        }
+        const T ro0 = ro[0], ro1 = ro[1], ro2 = ro[2];
+        if (active && more) {
+            ro[0] = __builtin_nontemporal_load(&ruo[cxy + nn * (size_t)(k + 1)]);
+            ro[1] = __builtin_nontemporal_load(&rvo[cxy + nn * (size_t)(k + 1)]);
+            ro[2] = __builtin_nontemporal_load(&rwo[cxy + nn * (size_t)(k + 1)]);
+        }
+        __syncthreads();
+        if constexpr (PHI) {
+            FX[3] = prev_lane(FX[4]);
+            if (tx == 0) FX[3] = FXL[buf][ty];
+            FY[1] = FYL[buf][ty * MTX + tx];
+        }
+        const T *U0 = UL[sa][0], *V0 = UL[sa][1], *W0 = UL[sa][2];
+        T o[6];
+        mom_point<PHI, MUX, 3>(U0, V0, W0, UL[sb][0], UL[sb][1], UL[sb][2], uc, um1[0], um1[1], um1[2], um1[3],
+                               um1[4], FX, FY, FZ, fzm, 4, (T)sinf[k], cj, si, (T)cosf[k], sj, ci, ro0, ro1, ro2, q, o);
+        um1[0] = U0[uc]; um1[1] = V0[uc]; um1[2] = W0[uc]; um1[3] = U0[uc + 1]; um1[4] = V0[uc + MUX];
+        fzm = FZ[4];
+        if (active) {
+            const size_t t = cxy + nn * (size_t)k;
+            __builtin_nontemporal_store(o[0], &us[t]);
+            __builtin_nontemporal_store(o[1], &vs[t]);
+            __builtin_nontemporal_store(o[2], &ws[t]);
+            __builtin_nontemporal_store(o[3], &ruo[t]);
+            __builtin_nontemporal_store(o[4], &rvo[t]);
+            __builtin_nontemporal_store(o[5], &rwo[t]);
+        }
+        buf ^= 1;
+        if (more) force(sb, sn, buf);
+        const int t = sa;
+        sa = sb; sb = sn; sn = t;
+    }
+}
+
+template <int PHI, typename T>
+__global__ void __launch_bounds__(MTHREADS, 4) k_momentum(
+    const T *__restrict__ u, const T *__restrict__ v, const T *__restrict__ w,
+    const T *__restrict__ phi,
+    T *__restrict__ us, T *__restrict__ vs, T *__restrict__ ws,
+    T *__restrict__ ruo, T *__restrict__ rvo, T *__restrict__ rwo,
+    const double *__restrict__ sinf, const double *__restrict__ cosf, const Scalars *__restrict__ sc,
+    Consts c, double ALPHA, double BETA, int kz)
+{
+    k_momentum_body<PHI, T>(xcd_block(), u, v, w, phi, us, vs, ws, ruo, rvo, rwo, sinf, cosf, sc, c, ALPHA, BETA, kz);
+}
+
+
+// ---------------------------------------------------------------------------
+// The same pass with two x-points per thread, used for FP32 state (in FP64
+// the pair needs 220 VGPRs and 95 KB of LDS: one wave per SIMD): 64 x 8 points
+// per block, every global load and store a float2 (the u/v/w and phi boxes
+// start at the even column i0-2, so pairs never straddle the periodic seam),
+// half the memory instructions per byte of the one-point form.  Each point's
+// arithmetic is mom_point, as in k_momentum, so the
+// results are those of k_momentum<PHI, T> bit for bit.
+// ---------------------------------------------------------------------------
+constexpr int PTX = 32, PTY = 8, PTHREADS = PTX * PTY;   // threads; 2 points each in x
+constexpr int PBX = 2 * PTX + 4, PUY = PTY + 2;           // u/v/w box row (68) and rows (10)
+constexpr int PPY = PTY + 3;                              // phi box rows (11), same row as u/v/w
+constexpr int PFX = 2 * PTX + 1, PFY = PTY + 1;           // force box (65 x 9)
+static_assert((PBX / 2) * PUY <= 2 * PTHREADS && (PBX / 2) * PPY <= 2 * PTHREADS, "two pairs per thread");
+static_assert(PFX * PFY <= 3 * PTHREADS, "three force points per thread");
 
 template <typename T> struct Pair2;
 template <> struct Pair2<float> { typedef float2 type; };
@@ -2674,7 +2678,7 @@ __global__ void __launch_bounds__(ATHREADS, sizeof(T) == 4 ? 8 : 4) kg_acdi(cons
 // euler: bit b set when box b takes its first (Euler) step, main.f90:323-324.
 // The CSF force uses phi^{n+1} (main.f90:604-658): the buffer the phase pass
 // of this step has just written, phin in the step's descriptor.
-// At most 128 VGPRs (4 waves per SIMD), as the one-box kernel compiles to.
+// At most 128 VGPRs (4 waves per SIMD), as in the one-box kernel.
 template <int PHI, typename T>
 __global__ void __launch_bounds__(MTHREADS, 4) kg_momentum(const GangBox *__restrict__ g, int nbox, unsigned euler,
                                                         GangGrid gg)
@@ -3376,10 +3380,10 @@ static int march_kz(int n, int tiles, int slots, int extra, int most, int boxes 
 // target of 2048 blocks, the rule before):
 //   phase field FP64   64^3: 13.1 / 13.1 / 22.3  128^3: 32.5 / 32.5 / 54.9  256^3: 184 / 184 / 195
 //   phase field FP32   64^3: 9.2 / 9.2 / 14.0    128^3: 17.8 / 17.8 / 22.8  256^3: 86.4 / 86.4 / 86.4
-//   momentum FP64      64^3: 14.4 / 14.4 / 25.3  128^3: 52.6 / 52.6 / 56.3  256^3: 386 / 380 / 386
+//   momentum FP64      72^3: 24.3 / 22.0         128^3: 45.6 / 45.6         256^3: 342 / 342
 //   momentum FP32      64^3: 13.1 / 13.1 / 25.9  128^3: 31.9 / 31.9 / 35.4  256^3: 192 / 192 / 201
 // A phase-field block recomputes 4 planes of psi in its prologue; two FP64
-// blocks are resident per CU, of FP32's four the last adds little.  A momentum
+// blocks are resident per CU (as of the momentum pass), of FP32's four the last adds little.  A momentum
 // block's prologue reads planes that its neighbour has just read.
 static int kz_acdi(int n, int mixed, int boxes = 1)
 {
@@ -3388,7 +3392,7 @@ static int kz_acdi(int n, int mixed, int boxes = 1)
 static int kz_momentum(int n, int mixed, int boxes = 1)
 {
     const int tx = mixed ? 2 * PTX : MTX, ty = mixed ? PTY : MTY;
-    return march_kz(n, ((n + tx - 1) / tx) * ((n + ty - 1) / ty), mixed ? 768 : 1024, mixed ? 3 : 1, 32, boxes);
+    return march_kz(n, ((n + tx - 1) / tx) * ((n + ty - 1) / ty), mixed ? 768 : 512, mixed ? 3 : 1, 32, boxes);
 }
 
 // The forms of small boxes take no slab height: they run unless one was set by
