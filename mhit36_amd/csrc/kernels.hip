@@ -789,6 +789,7 @@ __device__ __forceinline__ void k_momentum_body(uint3 blk,
         fzm = part(chem(PL[2], PL[0], pc, fzz), PL[0][pc], fzz);
         fown = PL[2][pc];
         if (edge) fedge = PL[2][ec];
+        __syncthreads();          // the first plane's store takes slot 2
     }
     force(0, 1, 0);
     // One barrier a plane.  What is stored before the barrier of plane k (u of
