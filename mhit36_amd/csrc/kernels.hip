@@ -642,6 +642,10 @@ __device__ __forceinline__ double prev_lane(double x)
     const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x138, 0xf, 0xf, true);
     return __hiloint2double(hi, lo);
 }
+__device__ __forceinline__ float prev_lane(float x)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x138, 0xf, 0xf, true));
+}
 
 template <int PHI, typename T>
 __device__ __forceinline__ void k_momentum_body(uint3 blk,
@@ -861,15 +865,18 @@ __global__ void __launch_bounds__(MTHREADS, 4) k_momentum(
 // per block, every global load and store a float2 (the u/v/w and phi boxes
 // start at the even column i0-2, so pairs never straddle the periodic seam),
 // half the memory instructions per byte of the one-point form.  Each point's
-// arithmetic is mom_point, as in k_momentum, so the
-// results are those of k_momentum<PHI, T> bit for bit.
+// arithmetic is mom_point, as in k_momentum, so the results are those of
+// k_momentum<PHI, T> bit for bit.  One barrier a plane as there: with phi
+// 192^3 102 -> 88 us, 256^3 211 -> 185, 512^3 1450 -> 1414; without it the
+// same as before.  Eight rows: with phi a thread takes 147 VGPRs (three waves
+// per SIMD), of which 16 rows leave one block per CU or, held to 128, 47
+// spills (512^3 2020 us); 12 rows 1582 us.
 // ---------------------------------------------------------------------------
-constexpr int PTX = 32, PTY = 8, PTHREADS = PTX * PTY;   // threads; 2 points each in x
-constexpr int PBX = 2 * PTX + 4, PUY = PTY + 2;           // u/v/w box row (68) and rows (10)
-constexpr int PPY = PTY + 3;                              // phi box rows (11), same row as u/v/w
-constexpr int PFX = 2 * PTX + 1, PFY = PTY + 1;           // force box (65 x 9)
+constexpr int PTX = 32, PTY = 8, PTHREADS = PTX * PTY;  // threads; 2 points each in x
+constexpr int PBX = 2 * PTX + 4, PUY = PTY + 2;           // u/v/w box row (68) and rows
+constexpr int PPY = PTY + 3;                              // phi box rows, same row as u/v/w
 static_assert((PBX / 2) * PUY <= 2 * PTHREADS && (PBX / 2) * PPY <= 2 * PTHREADS, "two pairs per thread");
-static_assert(PFX * PFY <= 3 * PTHREADS, "three force points per thread");
+static_assert(PTX == 32 && 2 * PTX + PTY <= PTHREADS, "two tile rows per wavefront; one edge cell per thread");
 
 template <typename T> struct Pair2;
 template <> struct Pair2<float> { typedef float2 type; };
@@ -900,7 +907,8 @@ __device__ __forceinline__ void k_momentum_x2_body(uint3 blk,
     if (halted(sc)) return;
     __shared__ T UL[3][3][PUY * PBX];
     __shared__ T PL[PHI ? 3 : 1][PHI ? PPY * PBX : 1];
-    __shared__ T FL[PHI ? 2 : 1][3][PHI ? PFY * PFX : 1];
+    __shared__ T FXL[PHI ? 2 : 1][PHI ? PTY : 1];
+    __shared__ T FYL[PHI ? 2 : 1][PHI ? (PTY + 1) * 2 * PTX : 1];
     const int n = c.n;
     const int tid = threadIdx.x;
     const int i0 = blk.x * (2 * PTX), j0 = blk.y * PTY, k0 = blk.z * kz;
@@ -931,16 +939,14 @@ __device__ __forceinline__ void k_momentum_x2_body(uint3 blk,
                 pu[r][0] = ld2(u + g); pu[r][1] = ld2(v + g); pu[r][2] = ld2(w + g);
             }
     };
-    auto store_u = [&](int m) {
-        const int slot = (m - k0 + 1) % 3;
+    auto store_u = [&](int slot) {
 #pragma unroll
         for (int r = 0; r < 2; r++) {
-            const int e = tid + r * PTHREADS;
+            const int e = tid + r * PTHREADS;              // pair e of the box is elements 2e, 2e + 1
             if (e < NP * PUY) {
-                const int b = (e / NP) * PBX + 2 * (e % NP);
-                UL[slot][0][b] = pu[r][0].x - um; UL[slot][0][b + 1] = pu[r][0].y - um;
-                UL[slot][1][b] = pu[r][1].x - vm; UL[slot][1][b + 1] = pu[r][1].y - vm;
-                UL[slot][2][b] = pu[r][2].x - wm; UL[slot][2][b + 1] = pu[r][2].y - wm;
+                UL[slot][0][2 * e] = pu[r][0].x - um; UL[slot][0][2 * e + 1] = pu[r][0].y - um;
+                UL[slot][1][2 * e] = pu[r][1].x - vm; UL[slot][1][2 * e + 1] = pu[r][1].y - vm;
+                UL[slot][2][2 * e] = pu[r][2].x - wm; UL[slot][2][2 * e + 1] = pu[r][2].y - wm;
             }
         }
     };
@@ -952,66 +958,86 @@ __device__ __forceinline__ void k_momentum_x2_body(uint3 blk,
                 if (tid + r * PTHREADS < NP * PPY) pp[r] = ld2(phi + foff[r] + zoff);
         }
     };
-    auto store_phi = [&](int m) {
+    auto store_phi = [&](int slot) {
         if constexpr (PHI) {
-            const int slot = (m - k0 + 2) % 3;
 #pragma unroll
             for (int r = 0; r < 2; r++) {
                 const int e = tid + r * PTHREADS;
                 if (e < NP * PPY) {
-                    const int b = (e / NP) * PBX + 2 * (e % NP);
-                    PL[slot][b] = pp[r].x;
-                    PL[slot][b + 1] = pp[r].y;
+                    PL[slot][2 * e] = pp[r].x;
+                    PL[slot][2 * e + 1] = pp[r].y;
                 }
             }
         }
     };
-    auto load_u = [&](int m) { fetch_u(m); store_u(m); };
-    auto load_phi = [&](int m) { fetch_phi(m); store_phi(m); };
-    auto force = [&](int m) {           // CSF force at cell centres (first half) on plane m (as in k_momentum)
-        if constexpr (PHI) {
-            const int ps = (m - k0 + 2) % 3, psm = (m - 1 - k0 + 2) % 3, psp = (m + 1 - k0 + 2) % 3;
-            const int fs = (m - k0 + 1) & 1;
-            const T sig6 = (T)((T)6.0 * c.sigma), eps = (T)c.eps, epsi = (T)c.epsi;
-            const T dxi = q.dxi, ddxi = q.ddxi;
-            for (int e = tid; e < PFX * PFY; e += PTHREADS) {
-                int fx_ = e % PFX, fy_ = e / PFX;
-                int pc = (fy_ + 1) * PBX + (fx_ + 1);
-                T f0 = PL[ps][pc];
-                T fxp = PL[ps][pc + 1], fxm = PL[ps][pc - 1];
-                T fyp = PL[ps][pc + PBX], fym = PL[ps][pc - PBX];
-                T fzp = PL[psp][pc], fzm = PL[psm][pc];
-                T t1 = f0 * ((T)1.0 - f0) * ((T)1.0 - (T)2.0 * f0) * epsi;
-                T s6 = (((((fxp + fxm) + fyp) + fym) + fzp) + fzm) - (T)6.0 * f0;
-                T chem = t1 - eps * s6 * ddxi;
-                FL[fs][0][e] = sig6 * chem * ((T)0.5 * (fxp - fxm) * dxi);
-                FL[fs][1][e] = sig6 * chem * ((T)0.5 * (fyp - fym) * dxi);
-                FL[fs][2][e] = sig6 * chem * ((T)0.5 * (fzp - fzm) * dxi);
-            }
-        }
-    };
-
-    load_u(k0 - 1);
-    load_u(k0);
-    load_phi(k0 - 2);
-    load_phi(k0 - 1);
-    load_phi(k0);
-    fetch_u(k0 + 1);
-    fetch_phi(k0 + 1);
-    __syncthreads();
-    force(k0 - 1);
-    __syncthreads();
-
     const int tx = tid % PTX, ty = tid / PTX;
     const int i = i0 + 2 * tx, j = j0 + ty;
     const bool active = (i < n) && (j < n);        // n even: i+1 < n with i
     const int kend = min(k0 + kz, n);
-    const int uc = (ty + 1) * PBX + (2 * tx + 2);
-    const int fc = (ty + 1) * PFX + (2 * tx + 1);
-    const size_t cxy = (size_t)(i < n ? i : 0) + (size_t)n * (j < n ? j : 0);
-    const T sj = (T)sinf[j < n ? j : 0], cj = (T)cosf[j < n ? j : 0];
-    const int ia = i < n ? i : 0, ib = i + 1 < n ? i + 1 : 0;
-    const T sia = (T)sinf[ia], cia = (T)cosf[ia], sib = (T)sinf[ib], cib = (T)cosf[ib];
+    const int uc = (ty + 1) * PBX + (2 * tx + 2), pc = (ty + 2) * PBX + (2 * tx + 2);
+    // The cell before the tile in x (row tid) or y (column tid - PTY) whose force this thread forms too.
+    const bool edge_x = tid < PTY, edge = tid < 2 * PTX + PTY;
+    const int ec = edge_x ? (tid + 2) * PBX + 1 : PBX + (tid - PTY + 2);
+    const T sig6 = (T)((T)6.0 * c.sigma), eps = (T)c.eps, epsi = (T)c.epsi;
+    auto chem = [&](const T *P0, const T *Pp, int e, T fm) {
+        const T f0 = P0[e];
+        T t1 = f0 * ((T)1.0 - f0) * ((T)1.0 - (T)2.0 * f0) * epsi;
+        T s6 = (((((P0[e + 1] + P0[e - 1]) + P0[e + PBX]) + P0[e - PBX]) + Pp[e]) + fm) - (T)6.0 * f0;
+        return t1 - eps * s6 * q.ddxi;
+    };
+    auto part = [&](T ch, T fp, T fm) { return sig6 * ch * ((T)0.5 * (fp - fm) * q.dxi); };
+    // as in k_momentum, for the thread's two points
+    T fown[2] = {}, fedge = (T)0.0, FX[2][9] = {}, FY[2][9] = {}, FZ[2][9] = {}, fzm[2] = {};
+    auto force = [&](int s0, int sp, int buf) {
+        if constexpr (PHI) {
+            const T *P0 = PL[s0], *Pp = PL[sp];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int e = pc + h;
+                const T ch = chem(P0, Pp, e, fown[h]);
+                FX[h][4] = part(ch, P0[e + 1], P0[e - 1]);
+                FY[h][4] = part(ch, P0[e + PBX], P0[e - PBX]);
+                FZ[h][4] = part(ch, Pp[e], fown[h]);
+                FYL[buf][(ty + 1) * 2 * PTX + 2 * tx + h] = FY[h][4];
+                fown[h] = P0[e];
+            }
+            if (edge) {
+                const T ch = chem(P0, Pp, ec, fedge);
+                if (edge_x) FXL[buf][tid] = part(ch, P0[ec + 1], P0[ec - 1]);
+                else FYL[buf][tid - PTY] = part(ch, P0[ec + PBX], P0[ec - PBX]);
+                fedge = P0[ec];
+            }
+        }
+    };
+    const int ic = i < n ? i : 0, jc = j < n ? j : 0;
+    const size_t cxy = (size_t)ic + (size_t)n * jc;
+
+    // prologue: slot of plane m in either ring: (m - k0) % 3
+    fetch_u(k0);
+    T u1[3], v1[2], v1p[2], w1[2];      // plane k-1: u at i .. i+2, v at j and j+1, w
+    {
+        const size_t zm = nn * (size_t)wrap(k0 - 1, n), row = zm + (size_t)n * jc;
+        const P2 a = ld2(u + row + ic), b = ld2(v + row + ic), d = ld2(w + row + ic),
+                 e = ld2(v + zm + (size_t)n * (jc + 1 == n ? 0 : jc + 1) + ic);
+        u1[0] = a.x - um; u1[1] = a.y - um;
+        u1[2] = u[row + (ic + 2 == n ? 0 : ic + 2)] - um;
+        v1[0] = b.x - vm; v1[1] = b.y - vm;
+        v1p[0] = e.x - vm; v1p[1] = e.y - vm;
+        w1[0] = d.x - wm; w1[1] = d.y - wm;
+    }
+    P2 fzz;
+    fzz.x = fzz.y = (T)0.0;
+    if constexpr (PHI) {
+        fzz = ld2(phi + cxy + nn * (size_t)wrap(k0 - 2, n));
+        fetch_phi(k0 - 1); store_phi(2);
+        fetch_phi(k0); store_phi(0);
+        fetch_phi(k0 + 1); store_phi(1);
+    }
+    store_u(0);
+    fetch_u(k0 + 1);
+    if (k0 + 1 < kend) fetch_phi(k0 + 2);
+    const T sj = (T)sinf[jc], cj = (T)cosf[jc];
+    const T sia = (T)sinf[ic], cia = (T)cosf[ic], sib = (T)sinf[ic + 1], cib = (T)cosf[ic + 1];
     P2 ro[3];
     ro[0].x = ro[0].y = ro[1].x = ro[1].y = ro[2].x = ro[2].y = (T)0.0;
     if (active) {
@@ -1019,34 +1045,57 @@ __device__ __forceinline__ void k_momentum_x2_body(uint3 blk,
         ro[1] = ld2(rvo + cxy + nn * (size_t)k0);
         ro[2] = ld2(rwo + cxy + nn * (size_t)k0);
     }
+    __syncthreads();
+    if constexpr (PHI) {
+        fzm[0] = part(chem(PL[2], PL[0], pc, fzz.x), PL[0][pc], fzz.x);
+        fzm[1] = part(chem(PL[2], PL[0], pc + 1, fzz.y), PL[0][pc + 1], fzz.y);
+        fown[0] = PL[2][pc];
+        fown[1] = PL[2][pc + 1];
+        if (edge) fedge = PL[2][ec];
+        __syncthreads();          // the first plane's store takes slot 2
+    }
+    force(0, 1, 0);
+    int sa = 0, sb = 1, sn = 2, buf = 0;       // slots of planes k, k+1 and the free one
     for (int k = k0; k < kend; k++) {
-        store_phi(k + 1);
-        if (k + 1 < kend) fetch_phi(k + 2);
-        __syncthreads();
-        force(k);
-        store_u(k + 1);
-        if (k + 1 < kend) fetch_u(k + 2);
+        const bool more = k + 1 < kend;
+        store_u(sb);
+        if (more) {
+            if constexpr (PHI) {
+                store_phi(sn);
+                if (k + 2 < kend) fetch_phi(k + 3);
+            }
+            fetch_u(k + 2);
+        }
         const P2 r0 = ro[0], r1 = ro[1], r2 = ro[2];
-        if (active && k + 1 < kend) {
+        if (active && more) {
             ro[0] = ld2(ruo + cxy + nn * (size_t)(k + 1));
             ro[1] = ld2(rvo + cxy + nn * (size_t)(k + 1));
             ro[2] = ld2(rwo + cxy + nn * (size_t)(k + 1));
         }
         __syncthreads();
+        if constexpr (PHI) {
+            FX[0][3] = prev_lane(FX[1][4]);
+            if (tx == 0) FX[0][3] = FXL[buf][ty];
+            FX[1][3] = FX[0][4];
+            FY[0][1] = FYL[buf][ty * 2 * PTX + 2 * tx];
+            FY[1][1] = FYL[buf][ty * 2 * PTX + 2 * tx + 1];
+        }
+        const T *U0 = UL[sa][0], *V0 = UL[sa][1], *W0 = UL[sa][2];
+        const T *Up = UL[sb][0], *Vp = UL[sb][1], *Wp = UL[sb][2];
+        const T sk = (T)sinf[k], ck = (T)cosf[k];
+        T oa[6], ob[6];
+        mom_point<PHI, PBX, 3>(U0, V0, W0, Up, Vp, Wp, uc, u1[0], v1[0], w1[0], u1[1], v1p[0], FX[0], FY[0], FZ[0],
+                               fzm[0], 4, sk, cj, sia, ck, sj, cia, r0.x, r1.x, r2.x, q, oa);
+        mom_point<PHI, PBX, 3>(U0, V0, W0, Up, Vp, Wp, uc + 1, u1[1], v1[1], w1[1], u1[2], v1p[1], FX[1], FY[1], FZ[1],
+                               fzm[1], 4, sk, cj, sib, ck, sj, cib, r0.y, r1.y, r2.y, q, ob);
+#pragma unroll
+        for (int h = 0; h < 3; h++) u1[h] = U0[uc + h];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            v1[h] = V0[uc + h]; v1p[h] = V0[uc + PBX + h]; w1[h] = W0[uc + h];
+            fzm[h] = FZ[h][4];
+        }
         if (active) {
-            const int s0 = (k - k0 + 1) % 3, sm = (k - k0) % 3, sp = (k - k0 + 2) % 3;
-            const int fs = (k - k0 + 1) & 1, fsm = (k - k0) & 1;
-            const T *Um = UL[sm][0], *Vm = UL[sm][1], *Wm = UL[sm][2];
-            const T sk = (T)sinf[k], ck = (T)cosf[k];
-            T oa[6], ob[6];
-            mom_point<PHI, PBX, PFX>(UL[s0][0], UL[s0][1], UL[s0][2], UL[sp][0], UL[sp][1], UL[sp][2], uc,
-                                     Um[uc], Vm[uc], Wm[uc], Um[uc + 1], Vm[uc + PBX], FL[fs][0], FL[fs][1],
-                                     FL[fs][2], PHI ? FL[fsm][2][fc] : (T)0.0, fc, sk, cj, sia, ck, sj, cia, r0.x,
-                                     r1.x, r2.x, q, oa);
-            mom_point<PHI, PBX, PFX>(UL[s0][0], UL[s0][1], UL[s0][2], UL[sp][0], UL[sp][1], UL[sp][2], uc + 1,
-                                     Um[uc + 1], Vm[uc + 1], Wm[uc + 1], Um[uc + 2], Vm[uc + 1 + PBX], FL[fs][0],
-                                     FL[fs][1], FL[fs][2], PHI ? FL[fsm][2][fc + 1] : (T)0.0, fc + 1, sk, cj, sib, ck,
-                                     sj, cib, r0.y, r1.y, r2.y, q, ob);
             const size_t t = cxy + nn * (size_t)k;
             st2nt(us + t, oa[0], ob[0]);
             st2nt(vs + t, oa[1], ob[1]);
@@ -1055,6 +1104,10 @@ __device__ __forceinline__ void k_momentum_x2_body(uint3 blk,
             st2nt(rvo + t, oa[4], ob[4]);
             st2nt(rwo + t, oa[5], ob[5]);
         }
+        buf ^= 1;
+        if (more) force(sb, sn, buf);
+        const int t = sa;
+        sa = sb; sb = sn; sn = t;
     }
 }
 
