@@ -793,9 +793,9 @@ __device__ __forceinline__ void k_momentum_body(uint3 blk,
         fzm = part(chem(PL[2], PL[0], pc, fzz), PL[0][pc], fzz);
         fown = PL[2][pc];
         if (edge) fedge = PL[2][ec];
-        __syncthreads();          // the first plane's store takes slot 2
     }
     force(0, 1, 0);
+    if constexpr (PHI) __syncthreads();        // the first plane's store takes slot 2, read above
     // One barrier a plane.  What is stored before the barrier of plane k (u of
     // k+1, phi of k+2) takes the slots of u(k-2) and phi(k-1), last read before
     // the barrier of plane k-1; force(k+1) writes the buffer that output(k-1)
@@ -1052,9 +1052,9 @@ __device__ __forceinline__ void k_momentum_x2_body(uint3 blk,
         fown[0] = PL[2][pc];
         fown[1] = PL[2][pc + 1];
         if (edge) fedge = PL[2][ec];
-        __syncthreads();          // the first plane's store takes slot 2
     }
     force(0, 1, 0);
+    if constexpr (PHI) __syncthreads();        // the first plane's store takes slot 2, read above
     int sa = 0, sb = 1, sn = 2, buf = 0;       // slots of planes k, k+1 and the free one
     for (int k = k0; k < kend; k++) {
         const bool more = k + 1 < kend;
