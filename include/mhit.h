@@ -257,6 +257,13 @@ int mhit_drop_count_noalloc(mhit_ctx *ctx, int max_drops, int *n_drops, double *
  * localise a difference. */
 int mhit_debug_math(int op, size_t count, const double *x, double *y);
 int mhit_debug_buffer(mhit_ctx *ctx, int which, double *host);
+/* How the pass that `knob` (MHIT_KNOB_*) shapes would be launched for a box of
+ * nx with the shapes value[MHIT_KNOBS] of mhit_set_tuning (the same ones are
+ * valid), in a box stepped alone (use 0), a gang (1) or the turbulent start
+ * (2): out[0] the kernel's form (0 march, 1 registers, 2 staged through LDS,
+ * 3 the form of small boxes, which has no such shape), out[1] the shape,
+ * out[2] threads and out[3] dynamic LDS bytes of a block.  No device needed. */
+int mhit_debug_launch_shape(int nx, int precision, int use, const int *value, int knob, int *out);
 
 /* ------------------------------------------------------------------------- */
 /* Ensemble serving (no counterpart in the reference, which runs one box per  */

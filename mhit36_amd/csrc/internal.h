@@ -144,6 +144,17 @@ int knob_candidates(int knob, const Consts &c, const FftPlan &pl, int *out, int 
 int knob_default(int knob, const Consts &c, const FftPlan &pl);
 // Whether the default form of this box's pass has no such shape (small boxes).
 bool knob_unused(int knob, const Consts &c, const FftPlan &pl);
+// What runs the passes: a box stepped alone, a gang, the turbulent start.
+enum FftUse { FFT_BOX, FFT_GANG, FFT_START };
+// How the pass that `knob` shapes would be launched: the form of its kernel
+// (FORM_SMALL: one that has no such shape), its shape, threads and dynamic LDS
+// bytes of a block.
+enum { FORM_MARCH, FORM_REGS, FORM_LDS, FORM_SMALL };
+struct LaunchShape {
+    int form, shape, threads;
+    size_t lds;
+};
+LaunchShape launch_shape(int knob, FftUse use, const Consts &c, const FftPlan &pl, const Tuning &tu);
 
 void launch_acdi(const Fields &f, const Consts &c, const Tuning &tu, hipStream_t s, LaunchInfo *li);
 void launch_momentum(const Fields &f, const Consts &c, const Tuning &tu, double alpha, double beta,

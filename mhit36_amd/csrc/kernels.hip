@@ -3546,20 +3546,21 @@ static int col_tile(const FftPlan &pl)
 // The lengths the register kernels are compiled for, with the stage plan as
 // constants: the column passes for their default tile (rtile_n) alone, the x
 // passes for any number of line pairs per block.  FFT_SIZES_GANG: also in gang
-// launches (boxes of up to 128^3).
+// launches (boxes of up to 128^3).  The turbulent start's z pass is compiled for none.
 #define FFT_SIZES_PLANE(X) X(32) X(36) X(48) X(54) X(64)
 #define FFT_SIZES_GANG(X) FFT_SIZES_PLANE(X) X(72) X(96) X(108) X(128)
 #define FFT_SIZES(X) FFT_SIZES_GANG(X) X(144) X(162) X(192) X(216) X(256) X(288) X(324) X(384) X(432) X(486) X(512) X(1024)
 
-static bool compiled_n(int n, bool gang)
+static bool compiled_n(int n, FftUse use)
 {
+    if (use == FFT_START) return false;
 #define FFT_CASE(N) case N:
     switch (n) {
     FFT_SIZES_GANG(FFT_CASE)
         return true;
     default: break;
     }
-    if (gang) return false;
+    if (use == FFT_GANG) return false;
     switch (n) {
     FFT_SIZES(FFT_CASE)
         return true;
@@ -3602,28 +3603,49 @@ static void with_plane_n(int n, Fn &&fn)
 // thread per 8 elements).
 static bool pow2_regs(const FftPlan &pl) { return pl.n >= 16 && is_pow2(pl.n); }
 
-// Which form an x pass takes, and a column pass of tile tkx: the register
-// kernels where n is compiled (a column pass also needs its default tile) or a
-// power of two, else the LDS-staged kernels.
-static bool x_regs(const FftPlan &pl, bool gang = false) { return compiled_n(pl.n, gang) || pow2_regs(pl); }
-static bool col_regs(const FftPlan &pl, int tkx, bool gang = false)
-{
-    return pow2_regs(pl) || (compiled_n(pl.n, gang) && tkx == rtile_n(pl.n));
-}
-// The length a column pass of tile tkx is compiled for, or 0.
-static int col_n(const FftPlan &pl, int tkx) { return tkx == rtile_n(pl.n) ? pl.n : 0; }
-// Default shapes.
-static int default_pairs(const FftPlan &pl, bool gang = false) { return x_regs(pl, gang) ? rpairs_n(pl.n) : pairs_per_block(pl); }
-static int default_tile(const FftPlan &pl, bool gang = false)
-{
-    return pow2_regs(pl) || compiled_n(pl.n, gang) ? rtile_n(pl.n) : col_tile(pl);
-}
 static int fft_threads(const FftPlan &pl, int nlines)
 {
     int t = nlines * (pl.n / plan_rmin(pl));
     t = ((t + 63) / 64) * 64;
     return t < 64 ? 64 : t;
 }
+
+// How an x pass and a column pass are launched for a shape set by hand (0: the
+// default): the register kernels where n is compiled (a column pass also needs
+// its default tile) or a power of two, else the LDS-staged kernels.  A shape is
+// chosen for the one-box passes, and another use of it may run the other form:
+// the default column tile of the register kernels (8 at 432 and 486) gives the
+// LDS-staged ones up to 1984 threads, so they take their own where it does not fit.
+struct FftPass {
+    int lines, threads;                  // pairs or columns, and threads, of a block
+    size_t lds;
+    bool regs;
+    int n;                               // the length it is compiled for, or 0 (in with_n's list or not)
+};
+static FftPass x_pass(const FftPlan &pl, int set, FftUse use)
+{
+    FftPass q;
+    q.regs = compiled_n(pl.n, use) || pow2_regs(pl);
+    q.lines = set ? set : q.regs ? rpairs_n(pl.n) : pairs_per_block(pl);
+    q.threads = q.regs ? q.lines * line_threads(pl.n) : fft_threads(pl, q.lines);
+    q.lds = sizeof(double2) * (size_t)q.lines * (q.regs ? rline_stride(pl.n) : pl.n + 1);
+    q.n = pl.n;
+    return q;
+}
+static FftPass col_pass(const FftPlan &pl, int set, FftUse use)
+{
+    const bool compiled = compiled_n(pl.n, use), pow2 = pow2_regs(pl);
+    FftPass q;
+    q.lines = set ? set : compiled || pow2 ? rtile_n(pl.n) : col_tile(pl);
+    q.regs = pow2 || (compiled && q.lines == rtile_n(pl.n));
+    if (!q.regs && fft_threads(pl, q.lines) > FFT_MAX_THREADS) q.lines = col_tile(pl);
+    q.threads = q.regs ? q.lines * line_threads(pl.n) : fft_threads(pl, q.lines);
+    q.lds = sizeof(double2) * (size_t)q.lines * pl.n;
+    q.n = q.lines == rtile_n(pl.n) ? pl.n : 0;
+    return q;
+}
+static int default_pairs(const FftPlan &pl) { return x_pass(pl, 0, FFT_BOX).lines; }
+static int default_tile(const FftPlan &pl) { return col_pass(pl, 0, FFT_BOX).lines; }
 
 // Whether a box's x and y passes run plane by plane in one block: a small
 // compiled length whose x and y shapes are the defaults (a shape set by hand
@@ -3638,7 +3660,7 @@ bool plane_fwd_alone(const Consts &c) { return c.n <= 32 || (c.mixed && c.n <= 4
 bool plane_passes(const Consts &c, const FftPlan &pl, const Tuning &tu)
 {
     auto def = [&](int knob, int d) { return tu.v[knob] == 0 || tu.v[knob] == d; };
-    return c.n <= PLANE_MAX && compiled_n(c.n, true) && def(KNOB_XPAIRS, default_pairs(pl)) &&
+    return c.n <= PLANE_MAX && compiled_n(c.n, FFT_GANG) && def(KNOB_XPAIRS, default_pairs(pl)) &&
            def(KNOB_XIPAIRS, default_pairs(pl)) && def(KNOB_YTILE, default_tile(pl));
 }
 
@@ -3688,32 +3710,49 @@ int knob_candidates(int knob, const Consts &c, const FftPlan &pl, int *out, int 
     return k;
 }
 
+LaunchShape launch_shape(int knob, FftUse use, const Consts &c, const FftPlan &pl, const Tuning &tu)
+{
+    if (knob == KNOB_KZ_ACDI) {
+        const int kz = tu.v[knob] ? tu.v[knob] : kz_acdi(c.n, c.mixed);
+        if (use == FFT_BOX && acdi_in_boxes(c, tu)) return {FORM_SMALL, 0, BTHREADS, 0};
+        return {FORM_MARCH, kz, ATHREADS, 0};
+    }
+    if (knob == KNOB_KZ_MOM) {
+        const int kz = tu.v[knob] ? tu.v[knob] : kz_momentum(c.n, c.mixed);
+        if (use == FFT_BOX && momentum_by_point(c, tu)) return {FORM_SMALL, 0, DTX * DTY, 0};
+        return {FORM_MARCH, kz, c.mixed ? PTHREADS : MTHREADS, 0};
+    }
+    const bool planes = use != FFT_START && knob != KNOB_ZTILE && plane_passes(c, pl, tu);
+    if (planes && (use == FFT_GANG || knob == KNOB_XIPAIRS || plane_fwd_alone(c)))
+        return {FORM_SMALL, 0, plane_threads(c.n), plane_lds(c.n)};
+    const bool x = knob == KNOB_XPAIRS || knob == KNOB_XIPAIRS;
+    // the turbulent start's y and x passes are the one-box ones
+    const FftPass q = x ? x_pass(pl, tu.v[knob], use == FFT_START ? FFT_BOX : use)
+                        : col_pass(pl, tu.v[knob], use == FFT_START && knob == KNOB_YTILE ? FFT_BOX : use);
+    return {q.regs ? FORM_REGS : FORM_LDS, q.lines, q.threads, q.lds};
+}
+
 void launch_xfwd(const Fields &f, const Consts &c, const FftPlan &pl, const Tuning &tu, hipStream_t s,
                  LaunchInfo *li)
 {
-    const int ppb = tu.v[KNOB_XPAIRS] ? tu.v[KNOB_XPAIRS] : default_pairs(pl), pairs = c.n * c.n / 2;
-    const dim3 grid(pairs / ppb);
+    const FftPass q = x_pass(pl, tu.v[KNOB_XPAIRS], FFT_BOX);
+    const int ppb = q.lines, pairs = c.n * c.n / 2;
+    const dim3 grid(pairs / ppb), blk(q.threads);
     const float *us = (const float *)f.us, *vs = (const float *)f.vs, *ws = (const float *)f.ws;
-    if (x_regs(pl)) {
-        const size_t shm = sizeof(double2) * (size_t)ppb * rline_stride(c.n);
-        const dim3 blk(ppb * line_threads(c.n));
-        with_n<false>(c.n, [&](auto NC) {
+    if (q.regs) {
+        with_n<false>(q.n, [&](auto NC) {
             constexpr int N = decltype(NC)::value;
             if (c.mixed)
-                hipLaunchKernelGGL((k_xfwd_r<float, N>), grid, blk, shm, s, us, vs, ws, f.spec, f.tw, f.sc, c, pl, ppb,
+                hipLaunchKernelGGL((k_xfwd_r<float, N>), grid, blk, q.lds, s, us, vs, ws, f.spec, f.tw, f.sc, c, pl, ppb,
                                    f.ld);
             else
-                hipLaunchKernelGGL((k_xfwd_r<double, N>), grid, blk, shm, s, f.us, f.vs, f.ws, f.spec, f.tw, f.sc, c,
+                hipLaunchKernelGGL((k_xfwd_r<double, N>), grid, blk, q.lds, s, f.us, f.vs, f.ws, f.spec, f.tw, f.sc, c,
                                    pl, ppb, f.ld);
         });
+    } else if (c.mixed) {
+        hipLaunchKernelGGL(k_xfwd<float>, grid, blk, q.lds, s, us, vs, ws, f.spec, f.tw, f.sc, c, pl, ppb, f.ld);
     } else {
-        const size_t shm = sizeof(double2) * (size_t)ppb * (c.n + 1);
-        const dim3 blk(fft_threads(pl, ppb));
-        if (c.mixed)
-            hipLaunchKernelGGL(k_xfwd<float>, grid, blk, shm, s, us, vs, ws, f.spec, f.tw, f.sc, c, pl, ppb, f.ld);
-        else
-            hipLaunchKernelGGL(k_xfwd<double>, grid, blk, shm, s, f.us, f.vs, f.ws, f.spec, f.tw, f.sc, c, pl, ppb,
-                               f.ld);
+        hipLaunchKernelGGL(k_xfwd<double>, grid, blk, q.lds, s, f.us, f.vs, f.ws, f.spec, f.tw, f.sc, c, pl, ppb, f.ld);
     }
     li->name = "xfwd_div"; li->bytes = (c.mixed ? 2.5 : 4.0) * F(c);
 }
@@ -3745,22 +3784,21 @@ void launch_plane_inv(const Fields &f, const Consts &c, hipStream_t s, LaunchInf
 void launch_ypass(const Fields &f, const Consts &c, const FftPlan &pl, const Tuning &tu, int inverse,
                   hipStream_t s, LaunchInfo *li)
 {
-    const int tkx = tu.v[KNOB_YTILE] ? tu.v[KNOB_YTILE] : default_tile(pl), nh = c.n / 2 + 1;
-    const dim3 grid((nh + tkx - 1) / tkx, c.n);
-    const size_t shm = sizeof(double2) * (size_t)tkx * c.n;
-    if (col_regs(pl, tkx)) {
-        const dim3 blk(tkx * line_threads(c.n));
-        with_n<false>(col_n(pl, tkx), [&](auto NC) {
+    const FftPass q = col_pass(pl, tu.v[KNOB_YTILE], FFT_BOX);
+    const int tkx = q.lines, nh = c.n / 2 + 1;
+    const dim3 grid((nh + tkx - 1) / tkx, c.n), blk(q.threads);
+    if (q.regs) {
+        with_n<false>(q.n, [&](auto NC) {
             constexpr int N = decltype(NC)::value, TK = N ? rtile_n(N) : 0;
             if (inverse)
-                hipLaunchKernelGGL((k_ypass_r<1, N, TK>), grid, blk, shm, s, f.spec, f.tw, f.sc, pl, f.ld, tkx);
+                hipLaunchKernelGGL((k_ypass_r<1, N, TK>), grid, blk, q.lds, s, f.spec, f.tw, f.sc, pl, f.ld, tkx);
             else
-                hipLaunchKernelGGL((k_ypass_r<-1, N, TK>), grid, blk, shm, s, f.spec, f.tw, f.sc, pl, f.ld, tkx);
+                hipLaunchKernelGGL((k_ypass_r<-1, N, TK>), grid, blk, q.lds, s, f.spec, f.tw, f.sc, pl, f.ld, tkx);
         });
     } else if (inverse) {
-        hipLaunchKernelGGL(k_ypass<1>, grid, dim3(fft_threads(pl, tkx)), shm, s, f.spec, f.tw, f.sc, pl, f.ld, tkx);
+        hipLaunchKernelGGL(k_ypass<1>, grid, blk, q.lds, s, f.spec, f.tw, f.sc, pl, f.ld, tkx);
     } else {
-        hipLaunchKernelGGL(k_ypass<-1>, grid, dim3(fft_threads(pl, tkx)), shm, s, f.spec, f.tw, f.sc, pl, f.ld, tkx);
+        hipLaunchKernelGGL(k_ypass<-1>, grid, blk, q.lds, s, f.spec, f.tw, f.sc, pl, f.ld, tkx);
     }
     li->name = inverse ? "y_inv" : "y_fwd";
     li->bytes = 2.0 * 16.0 * (double)nh * c.n * c.n;
@@ -3769,18 +3807,16 @@ void launch_ypass(const Fields &f, const Consts &c, const FftPlan &pl, const Tun
 void launch_zpoisson(const Fields &f, const Consts &c, const FftPlan &pl, const Tuning &tu, hipStream_t s,
                      LaunchInfo *li)
 {
-    const int tkx = tu.v[KNOB_ZTILE] ? tu.v[KNOB_ZTILE] : default_tile(pl), nh = c.n / 2 + 1;
-    const dim3 grid((nh + tkx - 1) / tkx, c.n);
-    const size_t shm = sizeof(double2) * (size_t)tkx * c.n;
-    if (col_regs(pl, tkx)) {
-        with_n<false>(col_n(pl, tkx), [&](auto NC) {
+    const FftPass q = col_pass(pl, tu.v[KNOB_ZTILE], FFT_BOX);
+    const int tkx = q.lines, nh = c.n / 2 + 1;
+    const dim3 grid((nh + tkx - 1) / tkx, c.n), blk(q.threads);
+    if (q.regs) {
+        with_n<false>(q.n, [&](auto NC) {
             constexpr int N = decltype(NC)::value, TK = N ? rtile_n(N) : 0;
-            hipLaunchKernelGGL((k_zpoisson_r<N, TK>), grid, dim3(tkx * line_threads(c.n)), shm, s, f.spec, f.tw, f.ktab,
-                               f.sc, pl, f.ld, tkx);
+            hipLaunchKernelGGL((k_zpoisson_r<N, TK>), grid, blk, q.lds, s, f.spec, f.tw, f.ktab, f.sc, pl, f.ld, tkx);
         });
     } else {
-        hipLaunchKernelGGL(k_zpoisson, grid, dim3(fft_threads(pl, tkx)), shm, s, f.spec, f.tw, f.ktab, f.sc, pl, f.ld,
-                           tkx);
+        hipLaunchKernelGGL(k_zpoisson, grid, blk, q.lds, s, f.spec, f.tw, f.ktab, f.sc, pl, f.ld, tkx);
     }
     li->name = "z_poisson";
     li->bytes = 2.0 * 16.0 * (double)nh * c.n * c.n;
@@ -3789,17 +3825,15 @@ void launch_zpoisson(const Fields &f, const Consts &c, const FftPlan &pl, const 
 void launch_xinv(const Fields &f, const Consts &c, const FftPlan &pl, const Tuning &tu, hipStream_t s,
                  LaunchInfo *li)
 {
-    const int ppb = tu.v[KNOB_XIPAIRS] ? tu.v[KNOB_XIPAIRS] : default_pairs(pl), pairs = c.n * c.n / 2;
-    if (x_regs(pl)) {
-        const size_t shm = sizeof(double2) * (size_t)ppb * rline_stride(c.n);
-        with_n<false>(c.n, [&](auto NC) {
-            hipLaunchKernelGGL((k_xinv_r<decltype(NC)::value>), dim3(pairs / ppb), dim3(ppb * line_threads(c.n)), shm,
-                               s, f.spec, f.p, f.tw, f.sc, pl, ppb, f.ld);
+    const FftPass q = x_pass(pl, tu.v[KNOB_XIPAIRS], FFT_BOX);
+    const int ppb = q.lines, pairs = c.n * c.n / 2;
+    const dim3 grid(pairs / ppb), blk(q.threads);
+    if (q.regs) {
+        with_n<false>(q.n, [&](auto NC) {
+            hipLaunchKernelGGL((k_xinv_r<decltype(NC)::value>), grid, blk, q.lds, s, f.spec, f.p, f.tw, f.sc, pl, ppb, f.ld);
         });
     } else {
-        const size_t shm = sizeof(double2) * (size_t)ppb * (c.n + 1);
-        hipLaunchKernelGGL(k_xinv, dim3(pairs / ppb), dim3(fft_threads(pl, ppb)), shm, s, f.spec, f.p, f.tw, f.sc, pl,
-                           ppb, f.ld);
+        hipLaunchKernelGGL(k_xinv, grid, blk, q.lds, s, f.spec, f.p, f.tw, f.sc, pl, ppb, f.ld);
     }
     li->name = "x_inv"; li->bytes = 16.0 * (double)(c.n / 2 + 1) * c.n * c.n + F(c);
 }
@@ -3909,15 +3943,10 @@ void launch_gang_step(const GangBox *g, int nbox, unsigned euler, bool publish, 
         const int nb = z.cnt, n = z.n, nh = n / 2 + 1, pairs = n * n / 2, ld = z.ld;
         const FftPlan &pl = z.plan;
         const Tuning &tu = z.tune;
-        const int xp = tu.v[KNOB_XPAIRS] ? tu.v[KNOB_XPAIRS] : default_pairs(pl, true);
-        const int xip = tu.v[KNOB_XIPAIRS] ? tu.v[KNOB_XIPAIRS] : default_pairs(pl, true);
-        const int ty = tu.v[KNOB_YTILE] ? tu.v[KNOB_YTILE] : default_tile(pl, true);
-        const int tz = tu.v[KNOB_ZTILE] ? tu.v[KNOB_ZTILE] : default_tile(pl, true);
-        const bool xr = x_regs(pl, true), yr = col_regs(pl, ty, true), zr = col_regs(pl, tz, true);
-        const size_t line = sizeof(double2) * (size_t)(xr ? rline_stride(n) : n + 1);
+        const FftPass xf = x_pass(pl, tu.v[KNOB_XPAIRS], FFT_GANG), xi = x_pass(pl, tu.v[KNOB_XIPAIRS], FFT_GANG);
+        const FftPass yp = col_pass(pl, tu.v[KNOB_YTILE], FFT_GANG), zp = col_pass(pl, tu.v[KNOB_ZTILE], FFT_GANG);
+        const int xp = xf.lines, xip = xi.lines, ty = yp.lines, tz = zp.lines;
         const dim3 gx(pairs / xp, nb), gxi(pairs / xip, nb), gy((nh + ty - 1) / ty, n, nb), gz((nh + tz - 1) / tz, n, nb);
-        const size_t shy = sizeof(double2) * (size_t)ty * n, shz = sizeof(double2) * (size_t)tz * n;
-        const int lt = line_threads(n);
         const bool planes = z.planes;
         if (planes) {
             with_plane_n(n, [&](auto NC) {
@@ -3927,49 +3956,49 @@ void launch_gang_step(const GangBox *g, int nbox, unsigned euler, bool publish, 
                 else
                     hipLaunchKernelGGL((kg_plane_fwd<double, N>), dim3(N, nb), dim3(plane_threads(N)), plane_lds(N), s, gs, ld);
             });
-        } else if (xr) {
-            with_n<true>(n, [&](auto NC) {
+        } else if (xf.regs) {
+            with_n<true>(xf.n, [&](auto NC) {
                 constexpr int N = decltype(NC)::value;
                 if (gl.mixed)
-                    hipLaunchKernelGGL((kg_xfwd<float, true, N>), gx, dim3(xp * lt), xp * line, s, gs, pl, xp, ld);
+                    hipLaunchKernelGGL((kg_xfwd<float, true, N>), gx, dim3(xf.threads), xf.lds, s, gs, pl, xp, ld);
                 else
-                    hipLaunchKernelGGL((kg_xfwd<double, true, N>), gx, dim3(xp * lt), xp * line, s, gs, pl, xp, ld);
+                    hipLaunchKernelGGL((kg_xfwd<double, true, N>), gx, dim3(xf.threads), xf.lds, s, gs, pl, xp, ld);
             });
         } else if (gl.mixed) {
-            hipLaunchKernelGGL((kg_xfwd<float, false, 0>), gx, dim3(fft_threads(pl, xp)), xp * line, s, gs, pl, xp, ld);
+            hipLaunchKernelGGL((kg_xfwd<float, false, 0>), gx, dim3(xf.threads), xf.lds, s, gs, pl, xp, ld);
         } else {
-            hipLaunchKernelGGL((kg_xfwd<double, false, 0>), gx, dim3(fft_threads(pl, xp)), xp * line, s, gs, pl, xp, ld);
+            hipLaunchKernelGGL((kg_xfwd<double, false, 0>), gx, dim3(xf.threads), xf.lds, s, gs, pl, xp, ld);
         }
         auto ypass = [&](auto SGC) {
             constexpr int SG = decltype(SGC)::value;
-            if (yr)
-                with_n<true>(col_n(pl, ty), [&](auto NC) {
-                    hipLaunchKernelGGL((kg_ypass<SG, true, decltype(NC)::value>), gy, dim3(ty * lt), shy, s, gs, pl, ld,
-                                       ty);
+            if (yp.regs)
+                with_n<true>(yp.n, [&](auto NC) {
+                    hipLaunchKernelGGL((kg_ypass<SG, true, decltype(NC)::value>), gy, dim3(yp.threads), yp.lds, s, gs, pl,
+                                       ld, ty);
                 });
             else
-                hipLaunchKernelGGL((kg_ypass<SG, false, 0>), gy, dim3(fft_threads(pl, ty)), shy, s, gs, pl, ld, ty);
+                hipLaunchKernelGGL((kg_ypass<SG, false, 0>), gy, dim3(yp.threads), yp.lds, s, gs, pl, ld, ty);
         };
         if (!planes) ypass(std::integral_constant<int, -1>());
-        if (zr)
-            with_n<true>(col_n(pl, tz), [&](auto NC) {
-                hipLaunchKernelGGL((kg_zpoisson<true, decltype(NC)::value>), gz, dim3(tz * lt), shz, s, gs, pl, ld, tz);
+        if (zp.regs)
+            with_n<true>(zp.n, [&](auto NC) {
+                hipLaunchKernelGGL((kg_zpoisson<true, decltype(NC)::value>), gz, dim3(zp.threads), zp.lds, s, gs, pl, ld,
+                                   tz);
             });
         else
-            hipLaunchKernelGGL((kg_zpoisson<false, 0>), gz, dim3(fft_threads(pl, tz)), shz, s, gs, pl, ld, tz);
+            hipLaunchKernelGGL((kg_zpoisson<false, 0>), gz, dim3(zp.threads), zp.lds, s, gs, pl, ld, tz);
         if (!planes) ypass(std::integral_constant<int, 1>());
         if (planes)
             with_plane_n(n, [&](auto NC) {
                 constexpr int N = decltype(NC)::value;
                 hipLaunchKernelGGL(kg_plane_inv<N>, dim3(N, nb), dim3(plane_threads(N)), plane_lds(N), s, gs, ld);
             });
-        else if (xr)
-            with_n<true>(n, [&](auto NC) {
-                hipLaunchKernelGGL((kg_xinv<true, decltype(NC)::value>), gxi, dim3(xip * lt), xip * line, s, gs, pl, xip,
-                                   ld);
+        else if (xi.regs)
+            with_n<true>(xi.n, [&](auto NC) {
+                hipLaunchKernelGGL((kg_xinv<true, decltype(NC)::value>), gxi, dim3(xi.threads), xi.lds, s, gs, pl, xip, ld);
             });
         else
-            hipLaunchKernelGGL((kg_xinv<false, 0>), gxi, dim3(fft_threads(pl, xip)), xip * line, s, gs, pl, xip, ld);
+            hipLaunchKernelGGL((kg_xinv<false, 0>), gxi, dim3(xi.threads), xi.lds, s, gs, pl, xip, ld);
         if (fork && q > 0) (void)hipEventRecord(fs->join[q - 1], s);
     }
     s = s0;
@@ -3993,12 +4022,9 @@ void launch_ic_potential(const Fields &f, const Consts &c, const FftPlan &pl, co
     const unsigned g = nblocks(total, BLK) < 65536 ? nblocks(total, BLK) : 65536;
     hipLaunchKernelGGL(k_ic_spectrum, dim3(g), dim3(BLK), 0, s, f.spec, c.n, f.ld, comp, seedmix, kp, kmax);
     const int nh = c.n / 2 + 1;
-    const bool regs = pow2_regs(pl);
-    const int tkx = tu.v[KNOB_ZTILE] ? tu.v[KNOB_ZTILE] : regs ? rtile_n(c.n) : col_tile(pl);
-    const size_t shm = sizeof(double2) * (size_t)tkx * c.n;
-    hipLaunchKernelGGL(regs ? k_zinv_r : k_zinv, dim3((nh + tkx - 1) / tkx, c.n),
-                       dim3(regs ? tkx * line_threads(c.n) : fft_threads(pl, tkx)), shm, s, f.spec, f.tw, f.ktab, f.sc, pl,
-                       f.ld, tkx);
+    const FftPass q = col_pass(pl, tu.v[KNOB_ZTILE], FFT_START);
+    hipLaunchKernelGGL(q.regs ? k_zinv_r : k_zinv, dim3((nh + q.lines - 1) / q.lines, c.n), dim3(q.threads), q.lds, s,
+                       f.spec, f.tw, f.ktab, f.sc, pl, f.ld, q.lines);
     LaunchInfo li;
     launch_ypass(f, c, pl, tu, 1, s, &li);
     Fields g2 = f;

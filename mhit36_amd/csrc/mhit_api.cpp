@@ -439,14 +439,19 @@ extern "C" int mhit_create(const mhit_params *p, mhit_ctx **out)
     return create_impl(p, out, nullptr, nullptr);
 }
 
+static bool grid_ok(int n)
+{
+    int rad[MAXSTAGES + 4];
+    return n >= 4 && n % 2 == 0 && plan_radices(n, rad) != 0 && n <= 2048;
+}
+
 // A context on `stream` (own stream when null) with memory from `arena` (hipMalloc when null).
 static int create_impl(const mhit_params *p, mhit_ctx **out, Arena *arena, hipStream_t stream)
 {
     if (!p || !out) return MHIT_ERR_ARG;
     *out = nullptr;
     const int n = p->nx;
-    int rad[MAXSTAGES + 4];
-    if (n < 4 || n % 2 != 0 || plan_radices(n, rad) == 0 || n > 2048) return MHIT_ERR_BAD_N;
+    if (!grid_ok(n)) return MHIT_ERR_BAD_N;
     if (p->precision != MHIT_FP64 && p->precision != MHIT_MIXED) return MHIT_ERR_UNSUPPORTED;
     if (p->dt == 0.0 || p->rho == 0.0 || p->epsr == 0.0) return MHIT_ERR_ARG;
     int ndev = 0;
@@ -1518,21 +1523,49 @@ extern "C" int mhit_autotune(mhit_ctx *c, int flags, mhit_tuning *out)
     return MHIT_OK;
 }
 
+// Shapes set by hand, each 0 or one of its knob's candidates.
+static bool tuning_from(const int *value, const Consts &k, const FftPlan &pl, Tuning *t)
+{
+    for (int q = 0; q < KNOB_COUNT; q++) {
+        const int v = value[q];
+        if (v == 0) continue;
+        int cand[12];
+        const int nc = knob_candidates(q, k, pl, cand, 12);
+        bool ok = false;
+        for (int i = 0; i < nc; i++) ok = ok || cand[i] == v;
+        if (!ok) return false;
+        t->v[q] = v;
+    }
+    return true;
+}
+
 extern "C" int mhit_set_tuning(mhit_ctx *c, const mhit_tuning *in)
 {
     if (!c || !in) return MHIT_ERR_ARG;
     Tuning t;
-    for (int q = 0; q < KNOB_COUNT; q++) {
-        const int v = in->value[q];
-        if (v == 0) continue;
-        int cand[12];
-        const int nc = knob_candidates(q, c->kc, c->plan, cand, 12);
-        bool ok = false;
-        for (int i = 0; i < nc; i++) ok = ok || cand[i] == v;
-        if (!ok) return MHIT_ERR_ARG;
-        t.v[q] = v;
-    }
+    if (!tuning_from(in->value, c->kc, c->plan, &t)) return MHIT_ERR_ARG;
     c->tune = t;
+    return MHIT_OK;
+}
+
+extern "C" int mhit_debug_launch_shape(int nx, int precision, int use, const int *value, int knob, int *out)
+{
+    if (!value || !out || use < FFT_BOX || use > FFT_START || knob < 0 || knob >= KNOB_COUNT) return MHIT_ERR_ARG;
+    if (precision != MHIT_FP64 && precision != MHIT_MIXED) return MHIT_ERR_UNSUPPORTED;
+    Consts k;
+    memset(&k, 0, sizeof(k));
+    k.n = nx;
+    k.mixed = precision == MHIT_MIXED ? 1 : 0;
+    FftPlan pl;
+    std::vector<double2> tw;
+    if (!grid_ok(nx) || plan_build(nx, &pl, &tw) != 0) return MHIT_ERR_BAD_N;
+    Tuning t;
+    if (!tuning_from(value, k, pl, &t)) return MHIT_ERR_ARG;
+    const LaunchShape s = launch_shape(knob, (FftUse)use, k, pl, t);
+    out[0] = s.form;
+    out[1] = s.shape;
+    out[2] = s.threads;
+    out[3] = (int)s.lds;
     return MHIT_OK;
 }
 
