@@ -1028,9 +1028,11 @@ extern "C" int mhit_step(mhit_ctx *c, int nsteps, mhit_diag *d)
     double *phi0 = c->f.phi, *phin0 = c->f.phin;
     const int since0 = c->nsteps_since_init, steps0 = c->dev_steps;
     for (int st = 0; st < nsteps; st++) enqueue_step(c, st == nsteps - 1);
-    HIPCHK(hipGetLastError());
+    // On an error steps may have run all the same, the last without its mirror:
+    // the state below is brought to where the device is before it is reported.
+    const hipError_t launched = hipGetLastError();
     Scalars s1;
-    int rc = wait_steps(c, nsteps, &s1);
+    int rc = launched == hipSuccess ? wait_steps(c, nsteps, &s1) : read_scalars(c, &s1);
     if (rc) return rc;
     const int done = s1.steps - steps0;
     // phi/phin were swapped once per enqueued step; keep the parity of the
@@ -1045,6 +1047,7 @@ extern "C" int mhit_step(mhit_ctx *c, int nsteps, mhit_diag *d)
         c->halted = 1;
         c->halt_status = s1.status;
     }
+    HIPCHK(launched);
     if (d) {
         d->steps_done = done;
         d->t = c->t;
@@ -1126,6 +1129,7 @@ extern "C" int mhit_step_batch(mhit_ctx *const *ctx, int nbox, int nsteps, mhit_
         std::swap(desc[GANG_MAX + j].f.phi, desc[GANG_MAX + j].f.phin);
     }
     std::vector<int> since0(m);
+    hipError_t launched = hipSuccess;
     if (m > 0) {
         hipStream_t s = lead->stream;
         HIPCHK(hipMemcpyAsync(lead->gang, desc.data(), sizeof(GangBox) * GANG_MAX, hipMemcpyHostToDevice, s));
@@ -1140,17 +1144,22 @@ extern "C" int mhit_step_batch(mhit_ctx *const *ctx, int nbox, int nsteps, mhit_
             const GangBox *g = lead->gang + (run[0]->kc.phiflag && (st & 1) ? GANG_MAX : 0);
             launch_gang_step(g, m, st == 0 ? euler : 0u, st == nsteps - 1, gl, s, &lead->gang_fs);
         }
-        HIPCHK(hipGetLastError());
+        launched = hipGetLastError();
         HIPCHK(hipStreamSynchronize(s));
     }
     const double ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-    int first = MHIT_OK;
+    int first = MHIT_OK, failed = MHIT_OK;
     for (int b = 0, q = 0; b < nbox; b++) {
         mhit_ctx *c = ctx[b];
         const int steps0 = c->dev_steps;
         Scalars s1;
-        int rc = c->halted ? read_scalars(c, &s1) : wait_steps(c, nsteps, &s1);
-        if (rc) return rc;
+        // on an error every box's own scalars, as in mhit_step
+        int rc = c->halted || launched != hipSuccess ? read_scalars(c, &s1) : wait_steps(c, nsteps, &s1);
+        if (rc) {
+            failed = rc;
+            if (!c->halted) q++;
+            continue;
+        }
         int done = 0;
         if (!c->halted) {
             done = s1.steps - steps0;
@@ -1177,7 +1186,8 @@ extern "C" int mhit_step_batch(mhit_ctx *const *ctx, int nbox, int nsteps, mhit_
             d[b].ms = ms;
         }
     }
-    return first;
+    HIPCHK(launched);
+    return failed ? failed : first;
 }
 
 // ---------------------------------------------------------------------------
