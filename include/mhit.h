@@ -224,7 +224,10 @@ typedef struct mhit_tuning {
 int mhit_autotune(mhit_ctx *ctx, int flags, mhit_tuning *out);
 int mhit_get_tuning(mhit_ctx *ctx, mhit_tuning *out);
 /* Set this context's shapes by hand: value[k] = 0 selects the heuristic, any
- * other value must be one of the knob's valid shapes (MHIT_ERR_ARG if not). */
+ * other value must be one of the knob's valid shapes (MHIT_ERR_ARG if not).  By
+ * default small boxes run forms of the passes that have no such shape, and
+ * mhit_autotune leaves them; a value other than 0, also the one in heuristic[],
+ * selects the form that has it. */
 int mhit_set_tuning(mhit_ctx *ctx, const mhit_tuning *in);
 
 /* Drop count and sizes of the context's phi, as post/DropCountSize computes

@@ -143,7 +143,7 @@ struct Tuning {
 int knob_candidates(int knob, const Consts &c, const FftPlan &pl, int *out, int cap);
 int knob_default(int knob, const Consts &c, const FftPlan &pl);
 // Whether the default form of this box's pass has no such shape (small boxes).
-bool knob_unused(int knob, const Consts &c, const FftPlan &pl);
+bool knob_unused(int knob, const Consts &c);
 // What runs the passes: a box stepped alone, a gang, the turbulent start.
 enum FftUse { FFT_BOX, FFT_GANG, FFT_START };
 // How the pass that `knob` shapes would be launched: the form of its kernel
@@ -175,7 +175,7 @@ void launch_reduce(const Fields &f, const Consts &c, hipStream_t s, LaunchInfo *
 void launch_finalize(const Fields &f, const Consts &c, bool publish, hipStream_t s, LaunchInfo *li);
 // The x and y passes of small boxes, plane by plane, in place of launch_xfwd and
 // the forward launch_ypass, and of the inverse pair.
-bool plane_passes(const Consts &c, const FftPlan &pl, const Tuning &tu);
+bool plane_passes(const Consts &c, const Tuning &tu);
 bool plane_fwd_alone(const Consts &c);   // the forward pair too, in a box stepped alone
 void launch_plane_fwd(const Fields &f, const Consts &c, hipStream_t s, LaunchInfo *li);
 void launch_plane_inv(const Fields &f, const Consts &c, hipStream_t s, LaunchInfo *li);

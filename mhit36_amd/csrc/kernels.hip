@@ -3449,16 +3449,11 @@ static int kz_momentum(int n, int mixed, int boxes = 1)
     return march_kz(n, ((n + tx - 1) / tx) * ((n + ty - 1) / ty), mixed ? 768 : 512, mixed ? 3 : 1, 32, boxes);
 }
 
-// The forms of small boxes take no slab height: they run unless one was set by
-// hand that differs from the default.
-static bool kz_default(const Tuning &tu, int knob, int kz) { return tu.v[knob] == 0 || tu.v[knob] == kz; }
-static bool acdi_in_boxes(const Consts &c, const Tuning &tu)
-{
-    return c.n <= 72 && kz_default(tu, KNOB_KZ_ACDI, kz_acdi(c.n, c.mixed));
-}
+// The forms of small boxes take no slab height: they run unless one was set by hand.
+static bool acdi_in_boxes(const Consts &c, const Tuning &tu) { return c.n <= 72 && tu.v[KNOB_KZ_ACDI] == 0; }
 static bool momentum_by_point(const Consts &c, const Tuning &tu)
 {
-    return c.n <= (c.mixed ? 96 : 64) && kz_default(tu, KNOB_KZ_MOM, kz_momentum(c.n, c.mixed));
+    return c.n <= (c.mixed ? 96 : 64) && tu.v[KNOB_KZ_MOM] == 0;
 }
 
 template <typename T>
@@ -3648,8 +3643,8 @@ static int default_pairs(const FftPlan &pl) { return x_pass(pl, 0, FFT_BOX).line
 static int default_tile(const FftPlan &pl) { return col_pass(pl, 0, FFT_BOX).lines; }
 
 // Whether a box's x and y passes run plane by plane in one block: a small
-// compiled length whose x and y shapes are the defaults (a shape set by hand
-// asks for the separate passes).
+// compiled length with no x or y shape set by hand (one asks for the separate
+// passes).
 // One box: n blocks leave most CUs idle, and the forward passes, whose threads
 // load eleven values per point pair, gain only at 32^3 and in FP32 up to 48^3
 // (forward pair / in one, us: 32^3 11.1 / 9.2, 48^3 FP32 9.7 / 8.7, FP64 9.7 /
@@ -3657,11 +3652,10 @@ static int default_tile(const FftPlan &pl) { return col_pass(pl, 0, FFT_BOX).lin
 // size (64^3 10.0 / 8.1).  A gang fills the CUs: 8 boxes of 64^3 20.4 / 15.6 and
 // 18.1 / 10.1.
 bool plane_fwd_alone(const Consts &c) { return c.n <= 32 || (c.mixed && c.n <= 48); }
-bool plane_passes(const Consts &c, const FftPlan &pl, const Tuning &tu)
+bool plane_passes(const Consts &c, const Tuning &tu)
 {
-    auto def = [&](int knob, int d) { return tu.v[knob] == 0 || tu.v[knob] == d; };
-    return c.n <= PLANE_MAX && compiled_n(c.n, FFT_GANG) && def(KNOB_XPAIRS, default_pairs(pl)) &&
-           def(KNOB_XIPAIRS, default_pairs(pl)) && def(KNOB_YTILE, default_tile(pl));
+    return c.n <= PLANE_MAX && compiled_n(c.n, FFT_GANG) && tu.v[KNOB_XPAIRS] == 0 && tu.v[KNOB_XIPAIRS] == 0 &&
+           tu.v[KNOB_YTILE] == 0;
 }
 
 // Tunable launch shapes.  Every candidate satisfies what the kernels assume:
@@ -3678,13 +3672,13 @@ int knob_default(int knob, const Consts &c, const FftPlan &pl)
     }
 }
 
-bool knob_unused(int knob, const Consts &c, const FftPlan &pl)
+bool knob_unused(int knob, const Consts &c)
 {
     switch (knob) {
     case KNOB_KZ_ACDI: return acdi_in_boxes(c, Tuning());
     case KNOB_KZ_MOM: return momentum_by_point(c, Tuning());
     case KNOB_ZTILE: return false;
-    default: return plane_passes(c, pl, Tuning());
+    default: return plane_passes(c, Tuning());
     }
 }
 
@@ -3722,7 +3716,7 @@ LaunchShape launch_shape(int knob, FftUse use, const Consts &c, const FftPlan &p
         if (use == FFT_BOX && momentum_by_point(c, tu)) return {FORM_SMALL, 0, DTX * DTY, 0};
         return {FORM_MARCH, kz, c.mixed ? PTHREADS : MTHREADS, 0};
     }
-    const bool planes = use != FFT_START && knob != KNOB_ZTILE && plane_passes(c, pl, tu);
+    const bool planes = use != FFT_START && knob != KNOB_ZTILE && plane_passes(c, tu);
     if (planes && (use == FFT_GANG || knob == KNOB_XIPAIRS || plane_fwd_alone(c)))
         return {FORM_SMALL, 0, plane_threads(c.n), plane_lds(c.n)};
     const bool x = knob == KNOB_XPAIRS || knob == KNOB_XIPAIRS;
@@ -3897,7 +3891,7 @@ void gang_layout(const GangBox *d, int nbox, const GangSize *sizes, GangLaunch *
             z.off = b;
             z.cnt = 0;
             z.n = n;
-            z.planes = plane_passes(d[b].c, z.plan, z.tune);
+            z.planes = plane_passes(d[b].c, z.tune);
         }
         gl->size[gl->nsize - 1].cnt++;
     }

@@ -978,7 +978,7 @@ static void enqueue_step(mhit_ctx *c, bool publish)
         std::swap(f.phi, f.phin);
     }
     timed(c, [&](LaunchInfo *li) { launch_momentum(f, k, c->tune, alpha, beta, s, li); });
-    const bool planes = plane_passes(k, c->plan, c->tune);
+    const bool planes = plane_passes(k, c->tune);
     if (planes && plane_fwd_alone(k)) {
         timed(c, [&](LaunchInfo *li) { launch_plane_fwd(f, k, s, li); });
     } else {
@@ -1460,7 +1460,7 @@ static int tune_impl(mhit_ctx *c, double *ms_h, double *ms_t)
     }
     for (int knob = 0; knob < KNOB_COUNT && rc == MHIT_OK; knob++) {
         if (knob == KNOB_KZ_ACDI && !c->kc.phiflag) continue;
-        if (knob_unused(knob, c->kc, c->plan)) continue;
+        if (knob_unused(knob, c->kc)) continue;
         int cand[12];
         const int nc = knob_candidates(knob, c->kc, c->plan, cand, 12);
         const int def = knob_default(knob, c->kc, c->plan);

@@ -51,6 +51,26 @@ def test_every_shape_fits_every_use(precision):
     assert not bad, bad
 
 
+@pytest.mark.parametrize("precision", [0, 1])
+def test_a_shape_set_by_hand_is_the_one_that_runs(precision):
+    """Small boxes run forms without a shape, unless one is set by hand: then
+    the pass that has it runs, with that shape, also where it is the default."""
+    small = set()
+    for n in LENGTHS:
+        for knob in KNOBS:
+            if launch(n, precision, 0, knob)[0] == SMALL:
+                small.add((knob, n))
+            for v in [2 ** q for q in range(11)]:
+                got = launch(n, precision, 0, knob, **{knob: v})
+                if got:
+                    assert got[0] == MARCH if knob.startswith("kz") else got[0] in (REGS, LDS), (n, knob, v, got)
+                    assert got[1] == v, (n, knob, v, got)
+    sizes = {knob: [n for k, n in sorted(small) if k == knob] for knob in KNOBS}
+    assert sizes["kz_phase"] == [n for n in LENGTHS if n <= 72]
+    assert sizes["kz_momentum"] == [n for n in LENGTHS if n <= (96 if precision else 64)]
+    assert sizes["xinv_pairs"] == [32, 36, 48, 54, 64] and not sizes["z_tile"]
+
+
 def test_unknown_lengths_and_shapes_are_refused():
     value, out = (ctypes.c_int * len(KNOBS))(), (ctypes.c_int * 4)()
     lib = _lib.load()
