@@ -2711,6 +2711,16 @@ __device__ __forceinline__ unsigned gang_block(const GangGrid &gg, int nbox, uns
     return box;
 }
 
+// A pointer field of a descriptor, read as one to device memory: a kernel's own
+// pointer arguments are known to be that, one that is read from memory is not,
+// and its accesses are flat ones, each with a 64-bit address in VGPRs, and never
+// scalar loads.
+template <typename T, typename F>
+__device__ __forceinline__ T *global_ptr(F *const &field)
+{
+    return (T *)*reinterpret_cast<__attribute__((address_space(1))) T *const *>((uintptr_t)&field);
+}
+
 // Tile coordinates of a box's block `l` in a grid of gx x gy tiles per slab.
 __device__ __forceinline__ uint3 tile_of(unsigned l, unsigned gx, unsigned gy)
 {
@@ -2732,7 +2742,11 @@ __global__ void __launch_bounds__(ATHREADS, sizeof(T) == 4 ? 8 : 4) kg_acdi(cons
 // euler: bit b set when box b takes its first (Euler) step, main.f90:323-324.
 // The CSF force uses phi^{n+1} (main.f90:604-658): the buffer the phase pass
 // of this step has just written, phin in the step's descriptor.
-// At most 128 VGPRs (4 waves per SIMD), as in the one-box kernel.
+// At most 128 VGPRs (4 waves per SIMD), as in the one-box kernel, and 2 values
+// spilled as there.  With the descriptor's pointers taken as they are (flat
+// accesses, the means in VGPRs) it spilled 13, and a step of 8 boxes FP64 with
+// phi took 55.0 / 125 / 170 / 589 / 1152 us at 32 / 48 / 64 / 96 / 128^3 instead
+// of 52.5 / 115 / 159 / 555 / 1095 (8 rows, two barriers: 55.8 / 125 / 163 / 577 / 1128).
 template <int PHI, typename T>
 __global__ void __launch_bounds__(MTHREADS, 4) kg_momentum(const GangBox *__restrict__ g, int nbox, unsigned euler,
                                                         GangGrid gg)
@@ -2743,10 +2757,11 @@ __global__ void __launch_bounds__(MTHREADS, 4) kg_momentum(const GangBox *__rest
     const bool eu = (euler >> box) & 1u;
     const unsigned n = (unsigned)B.c.n;
     const int kz = gg.kz[box];
-    k_momentum_body<PHI, T>(tile_of(l, (n + MTX - 1) / MTX, (n + MTY - 1) / MTY), (const T *)B.f.u,
-                            (const T *)B.f.v, (const T *)B.f.w, (const T *)B.f.phin, (T *)B.f.us, (T *)B.f.vs,
-                            (T *)B.f.ws, (T *)B.f.ruo, (T *)B.f.rvo, (T *)B.f.rwo, B.f.sinf, B.f.cosf, B.f.sc,
-                            B.c, eu ? 1.0 : 1.5, eu ? 0.0 : 0.5, kz);
+    k_momentum_body<PHI, T>(tile_of(l, (n + MTX - 1) / MTX, (n + MTY - 1) / MTY), global_ptr<const T>(B.f.u),
+                            global_ptr<const T>(B.f.v), global_ptr<const T>(B.f.w), global_ptr<const T>(B.f.phin),
+                            global_ptr<T>(B.f.us), global_ptr<T>(B.f.vs), global_ptr<T>(B.f.ws), global_ptr<T>(B.f.ruo),
+                            global_ptr<T>(B.f.rvo), global_ptr<T>(B.f.rwo), global_ptr<const double>(B.f.sinf),
+                            global_ptr<const double>(B.f.cosf), global_ptr<const Scalars>(B.f.sc), B.c, eu ? 1.0 : 1.5, eu ? 0.0 : 0.5, kz);
 }
 
 template <int PHI, typename T>
