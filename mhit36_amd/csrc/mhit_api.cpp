@@ -583,6 +583,13 @@ static int read_scalars(mhit_ctx *c, Scalars *s)
     return MHIT_OK;
 }
 
+// Enqueues *d = 0.0; the caller waits for the stream before the slot is used again.
+static hipError_t clear_value(mhit_ctx *c, double *d)
+{
+    c->hs->copy.umean = 0.0;
+    return hipMemcpyAsync(d, &c->hs->copy.umean, sizeof(double), hipMemcpyHostToDevice, c->stream);
+}
+
 // A field between device memory (`values` FP32 or FP64, `width` bytes each) and
 // the caller's FP64 array, in pieces staged through pinned blocks.  The copy
 // engine moves a piece while other threads narrow, widen or subtract the mean
@@ -591,8 +598,9 @@ static int read_scalars(mhit_ctx *c, Scalars *s)
 // against 114-142 ms through pageable memory with one thread, FP32 state
 // 15-17 against 222 ms.
 constexpr int COPY_THREADS = 8;               // 16 hardware threads serve one GPU
+// `clear`: a device value set to 0 along with the copy, in the same wait.
 template <typename Fn>                        // convert(first value, count, staged piece)
-static int staged_copy(mhit_ctx *c, void *dev, size_t values, size_t width, bool out, Fn &&convert)
+static int staged_copy(mhit_ctx *c, void *dev, size_t values, size_t width, bool out, Fn &&convert, double *clear = nullptr)
 {
     const size_t bytes = values * width;
     const int most = (int)std::min<size_t>(COPY_THREADS, std::max<size_t>(1, bytes / HOST_BLOCK));
@@ -630,6 +638,10 @@ static int staged_copy(mhit_ctx *c, void *dev, size_t values, size_t width, bool
     HIPCHK(hipGetDevice(&cur));
     void *own = g_host.block(true);
     if (!own) return MHIT_ERR_OOM;
+    if (clear && clear_value(c, clear) != hipSuccess) {
+        g_host.give_block(own);
+        return MHIT_ERR_HIP;
+    }
     void *stage[COPY_THREADS];
     std::thread th[COPY_THREADS];
     int started = 0;
@@ -706,6 +718,14 @@ struct HostField {
     }
 };
 
+// An FP64 field of these sizes goes in by the runtime's own copy from pageable
+// memory: it reads the caller's pages in place, while one to four threads (one
+// per 4 MB) copy them to a block first.  Direct / staged, us: 64^3 95 / 98,
+// 96^3 213 / 276, 108^3 292 / 335, 128^3 476 / 515, 144^3 656 / 655, 192^3
+// 1900 / 1400; below 64^3 staged is level or, with the caller's pages not yet
+// known to the runtime, much faster (36^3 175 / 36).
+constexpr size_t DIRECT_IN_ABOVE = (size_t)2 << 20, DIRECT_IN_MOST = (size_t)16 << 20;
+
 extern "C" int mhit_set_field(mhit_ctx *c, int fieldn, const double *host)
 {
     if (!c || !host) return MHIT_ERR_ARG;
@@ -713,25 +733,26 @@ extern "C" int mhit_set_field(mhit_ctx *c, int fieldn, const double *host)
     if (!d) return MHIT_ERR_ARG;
     c->loaded = true;
     const size_t n = c->p.nx, n3 = n * n * n;
-    int rc;
-    if (c->kc.mixed && fieldn != 4) {
-        rc = staged_copy(c, d, n3, sizeof(float), false, [&](size_t v, size_t k, void *stage) {
-            float *f = (float *)stage;
-            for (size_t q = 0; q < k; q++) f[q] = (float)host[v + q];
-        });
-    } else {
-        rc = staged_copy(c, d, n3, sizeof(double), false,
-                         [&](size_t v, size_t k, void *stage) { memcpy(stage, host + v, k * sizeof(double)); });
-    }
-    if (rc) return rc;
-    if (fieldn <= 3) {
-        // the stored field is now the field itself: its pending mean is zero
-        double *m = &c->f.sc->umean + (fieldn - 1);
-        c->hs->copy.umean = 0.0;
-        HIPCHK(hipMemcpyAsync(m, &c->hs->copy.umean, sizeof(double), hipMemcpyHostToDevice, c->stream));
+    // the stored field is now the field itself: its pending mean is zero
+    double *mean = fieldn <= 3 ? &c->f.sc->umean + (fieldn - 1) : nullptr;
+    if (c->kc.mixed && fieldn != 4)
+        return staged_copy(
+            c, d, n3, sizeof(float), false,
+            [&](size_t v, size_t k, void *stage) {
+                float *f = (float *)stage;
+                for (size_t q = 0; q < k; q++) f[q] = (float)host[v + q];
+            },
+            mean);
+    const size_t bytes = n3 * sizeof(double);
+    if (bytes > DIRECT_IN_ABOVE && bytes <= DIRECT_IN_MOST) {
+        HIPCHK(hipMemcpyAsync(d, host, bytes, hipMemcpyHostToDevice, c->stream));
+        if (mean) HIPCHK(clear_value(c, mean));
         HIPCHK(hipStreamSynchronize(c->stream));
+        return MHIT_OK;
     }
-    return MHIT_OK;
+    return staged_copy(
+        c, d, n3, sizeof(double), false,
+        [&](size_t v, size_t k, void *stage) { memcpy(stage, host + v, k * sizeof(double)); }, mean);
 }
 
 extern "C" int mhit_get_field(mhit_ctx *c, int fieldn, double *host)
