@@ -419,8 +419,8 @@ __device__ __forceinline__ void k_acdi_body(uint3 blk,
 }
 
 // FP32: 8 waves per SIMD (63 VGPRs).  FP64: held to the 128 VGPRs of 4 waves
-// per SIMD (two blocks per CU); its one spilled value belongs to the log's
-// branch for zero, negative or non-finite arguments.  Held to the 80 VGPRs of
+// per SIMD (two blocks per CU), with 14 spills by the compiler's count, in 12
+// bytes of scratch per lane.  Held to the 80 VGPRs of
 // 6 waves (three blocks, which the 44 KB of LDS would allow) the pass spills
 // in the march and runs 2.3x slower.
 template <typename T>
@@ -439,9 +439,9 @@ __global__ void __launch_bounds__(ATHREADS, sizeof(T) == 4 ? 8 : 4) k_acdi(
 // a block owns BTX x BTY x BTZ cells, forms psi on them and two cells around,
 // then the flux on them and the face neighbours, then the output: three steps
 // with a barrier between, in exchange for psi at 3 cells per cell instead of
-// 1.4 plus the prologue.  March / box, us (event times): FP64 32^3 12.2 / 8.5,
-// 64^3 13.1 / 12.2, 72^3 22.2 / 18.0, 96^3 22.7 / 25.2; FP32 32^3 8.4 / 6.8,
-// 72^3 12.5 / 11.7, 96^3 12.9 / 15.3: used up to 72^3.
+// 1.4 plus the prologue.  March / box, us (event times): FP64 32^3 12.0 / 8.5,
+// 64^3 12.8 / 11.6, 72^3 22.3 / 17.8, 96^3 22.7 / 25.2; FP32 32^3 8.5 / 6.7,
+// 72^3 12.2 / 11.4, 96^3 12.9 / 15.3: used up to 72^3.
 // ---------------------------------------------------------------------------
 constexpr int BTX = 16, BTY = 8, BTZ = 4, BTHREADS = BTX * BTY * BTZ;
 constexpr int BPX = BTX + 4, BPY = BTY + 4, BPZ = BTZ + 4, BPSI = BPX * BPY * BPZ;
@@ -558,7 +558,8 @@ __global__ void __launch_bounds__(BTHREADS) k_acdi_box(
 // less halo (rows of u: 18/16 instead of 10/8) and with one barrier the two
 // blocks of a CU still cover each other's waits.  256^3 and 512^3 with phi:
 // 394 and 3056 us (8 rows, two barriers a plane) -> 360 and 2907 (8 rows, one
-// barrier) -> 348 and 2730 (16 rows); 351 and 2742 with 32 rows.  Without phi:
+// barrier) -> 348 and 2730 (16 rows; 2490-2820 at 512^3 on other boxes); 351 and
+// 2742 with 32 rows.  128 VGPRs with phi, 2 values spilled.  Without phi:
 // 345 and 2588 -> 325 and 2638 -> 308 and 2435.  13 (12) values at the 5.4 TB/s
 // of a large copy are 2585 (2390) us at 512^3.
 // ---------------------------------------------------------------------------
@@ -868,7 +869,7 @@ __global__ void __launch_bounds__(MTHREADS, 4) k_momentum(
 // arithmetic is mom_point, as in k_momentum, so the results are those of
 // k_momentum<PHI, T> bit for bit.  One barrier a plane as there: with phi
 // 192^3 102 -> 88 us, 256^3 211 -> 185, 512^3 1450 -> 1414; without it the
-// same as before.  Eight rows: with phi a thread takes 147 VGPRs (three waves
+// same as before (512^3 1.41-1.47 ms on other boxes).  Eight rows: with phi a thread takes 147 VGPRs (three waves
 // per SIMD), of which 16 rows leave one block per CU or, held to 128, 47
 // spills (512^3 2020 us); 12 rows 1582 us.
 // ---------------------------------------------------------------------------
@@ -1129,11 +1130,16 @@ __global__ void __launch_bounds__(PTHREADS) k_momentum_x2(
 // every neighbour loaded from the caches, the CSF force formed at the point and
 // at its three lower neighbours.  49 loads per point, all in flight at once,
 // and no barrier.  mom_point on 3 x 3 neighbourhoods (row stride 3, the point
-// at 4): the results are those of k_momentum bit for bit.  March / point with
-// the phase field, us (event times): FP64 32^3 10.9 / 6.7, 64^3 14.3 / 13.0,
-// 72^3 21.7 / 20.0 but without the phase field 18.0 at either, 96^3 29.7 / 32.9;
-// FP32 32^3 11.5 / 6.6, 64^3 13.2 / 8.9, 96^3 22.1 / 18.2, 108^3 28.3 / 29.5:
-// used up to 64^3 and 96^3.  Bound by the L1: 49 loads of 512 bytes per wavefront.
+// at 4): the results are those of k_momentum bit for bit.  March at its best
+// slab / point, with the phase field, us (event times): FP64 32^3 10.2 / 6.6,
+// 48^3 10.8 / 10.2, 54^3 11.2 / 11.3, 64^3 12.0 / 12.8, 72^3 22.0 / 20.0, 96^3
+// 26.4 / 32.9; FP32 32^3 9.9 / 6.5, 64^3 10.5 / 8.3, 72^3 13.5 / 12.3, 96^3 17.7 /
+// 17.7, 108^3 22.7 / 29.5.  Used up to 64^3 and 96^3: the lines were drawn
+// against a march with two barriers a plane (64^3 FP64 14.3, 96^3 FP32 22.1 us);
+// with one the two are level there.  72^3 FP64 stays with the march, which
+// without the phase field is level too (19.2 / 18.0) at two planes a slab,
+// though kz_momentum gives it four (24.3 us).
+// Bound by the L1: 49 loads of 512 bytes per wavefront.
 // At most 4 waves per SIMD, or the compiler saves registers and waits for
 // the loads in groups (FP64 32^3 7.9 us).
 // ---------------------------------------------------------------------------
@@ -3445,12 +3451,14 @@ static int march_kz(int n, int tiles, int slots, int extra, int most, int boxes 
     return best;
 }
 // The constants are fitted to sweeps of kz at 16^3 to 512^3 (16, 32, 48, 64,
-// 96, 108, 128, 192, 256, 384, 512; times in us, this rule / the best kz / a
-// target of 2048 blocks, the rule before):
-//   phase field FP64   64^3: 13.1 / 13.1 / 22.3  128^3: 32.5 / 32.5 / 54.9  256^3: 184 / 184 / 195
-//   phase field FP32   64^3: 9.2 / 9.2 / 14.0    128^3: 17.8 / 17.8 / 22.8  256^3: 86.4 / 86.4 / 86.4
-//   momentum FP64      72^3: 24.3 / 22.0         128^3: 45.6 / 45.6         256^3: 342 / 342
-//   momentum FP32      64^3: 13.1 / 13.1 / 25.9  128^3: 31.9 / 31.9 / 35.4  256^3: 192 / 192 / 201
+// 96, 108, 128, 192, 256, 384, 512).  This rule / the best power of two, us, with
+// the phase field and the momentum march of one barrier a plane (16 rows FP64):
+//   phase field FP64   96^3 22.5 / 22.4   128^3 33.0 / 33.0   192^3 95.2 / 94.9   256^3 182 / 182
+//   phase field FP32   96^3 12.7 / 12.7   128^3 17.7 / 17.7   192^3 42.6 / 42.6   256^3 85.7 / 85.7
+//   momentum FP64      72^3 24.3 / 22.0   128^3 46.2 / 46.1   192^3 152 / 152     256^3 340 / 340
+//   momentum FP32     108^3 26.0 / 22.7   128^3 29.0 / 29.0   192^3 82.9 / 82.8   256^3 175 / 175
+// (with a target of 2048 blocks instead: phase field FP64 128^3 54.9, 256^3 195).
+// Only powers of two that divide n are tried: 54, 162 and 486 get two planes.
 // A phase-field block recomputes 4 planes of psi in its prologue; two FP64
 // blocks are resident per CU (as of the momentum pass), of FP32's four the last adds little.  A momentum
 // block's prologue reads planes that its neighbour has just read.
@@ -3664,7 +3672,8 @@ static int default_tile(const FftPlan &pl) { return col_pass(pl, 0, FFT_BOX).lin
 // load eleven values per point pair, gain only at 32^3 and in FP32 up to 48^3
 // (forward pair / in one, us: 32^3 11.1 / 9.2, 48^3 FP32 9.7 / 8.7, FP64 9.7 /
 // 14.9, 64^3 FP32 10.6 / 12.0, FP64 12.3 / 16.1); the inverse passes gain at every
-// size (64^3 10.0 / 8.1).  A gang fills the CUs: 8 boxes of 64^3 20.4 / 15.6 and
+// size (64^3 10.0 / 8.1).  36^3 and 54^3, by the time of the step with either:
+// FP64 level or separate faster, FP32 within 6% either way.  A gang fills the CUs: 8 boxes of 64^3 20.4 / 15.6 and
 // 18.1 / 10.1.
 bool plane_fwd_alone(const Consts &c) { return c.n <= 32 || (c.mixed && c.n <= 48); }
 bool plane_passes(const Consts &c, const Tuning &tu)
